@@ -52,7 +52,8 @@ PEAK_HBM_GBS = 8000.0
 # shrink pass is 64, one kinetic pass 46, V*psi 2.
 STAGE_FLOPS = {"uncompress": 0, "zero": 0, "xy_fwd": 220, "z_kin": 46, "z_pot": 130,
                "xy_bwd_compress": 128, "x_grow_kin": 110, "y_grow": 64, "y_kin": 46,
-               "y_shrink": 64, "x_shrink": 64, "compress": 0}
+               "y_shrink": 64, "x_shrink": 64, "compress": 0,
+               "z_grow": 64, "xy_kin": 92, "xy_pot": 258, "z_back": 110}
 # per-pass matrix-core sequence: the x kinetic alone, then one plane grow
 STAGE_FLOPS_MFMA_PASSES = dict(STAGE_FLOPS, x_grow_kin=46, xy_fwd=128)
 
@@ -61,11 +62,12 @@ def stage_bytes(batch, esz):
     """compulsory HBM bytes per apply of each stage, from the batch's box
     geometry: working grids of esz bytes -- W (wavelet volume, 8 N1 N2 N3
     per box), K (same), T2 (L1 L2 2 N3), T1 (L1 2 N2 2 N3, line passes
-    only) -- FP64 psi read once (8 B per coefficient), hpsi read and written
+    only), TZ (2 N1 2 N2 L3, FP64 sequence) -- FP64 psi read once (8 B per coefficient), hpsi read and written
     once (16 B), each potential value read once (8 B)"""
     regs = batch["regions"]
     W = sum(8 * (r.n[0] + 1) * (r.n[1] + 1) * (r.n[2] + 1) for r in regs)
     T2 = sum(r.nfine[0] * r.nfine[1] * 2 * (r.n[2] + 1) for r in regs)
+    TZ = sum(4 * (r.n[0] + 1) * (r.n[1] + 1) * r.nfine[2] for r in regs)
     T1 = sum(r.nfine[0] * 4 * (r.n[1] + 1) * (r.n[2] + 1) for r in regs)
     nc = int(batch["ncoef"].sum())
     V = 8 * min(int(batch["pot"].numel()), int(sum(r.n_isf for r in regs)))
@@ -74,7 +76,9 @@ def stage_bytes(batch, esz):
             "xy_bwd_compress": esz * (T2 + W) + 16 * nc,
             "x_grow_kin": esz * (2 * W + T1), "y_grow": esz * (T1 + T2),
             "y_kin": esz * 3 * W, "y_shrink": esz * (T2 + T1),
-            "x_shrink": esz * (T1 + 2 * W), "compress": esz * W + 16 * nc}
+            "x_shrink": esz * (T1 + 2 * W), "compress": esz * W + 16 * nc,
+            "z_grow": 8 * nc + esz * TZ, "xy_kin": 8 * nc + esz * W,
+            "xy_pot": esz * 2 * TZ + V, "z_back": esz * (TZ + W) + 24 * nc}
 
 
 def path_of(prec, plane_enabled, stages):

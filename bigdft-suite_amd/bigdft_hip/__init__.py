@@ -326,7 +326,7 @@ class Context:
 
     def profile_read(self, reset=True):
         """{stage name: accumulated ms}, number of profiled launches"""
-        n = 16
+        n = 32
         ms = np.zeros(n)
         cnt = ctypes.c_int64()
         self._check(lib().bdft_profile_read(self.handle, n, _ptr(ms),

@@ -109,9 +109,9 @@ struct bdft_plan {
   bool owns_ws = false;
   DevBuf ws;           // own workspace (persistent plans)
   // workspace not bound yet (a part of a chunked plan): bytes it needs and
-  // the offsets of W, K, T1, T2, T3 in it
+  // the offsets of W, K, T1, T2, T3, TZ in it
   size_t ws_need = 0;
-  size_t ws_at[5] = {0, 0, 0, 0, 0};
+  size_t ws_at[6] = {0, 0, 0, 0, 0, 0};
   // chunked plan: parts over consecutive orbital ranges, run one after the
   // other on one workspace (ws of this plan) sized for the largest part
   std::vector<bdft_plan*> parts;
@@ -227,6 +227,7 @@ extern "C" int bdft_ctx_create(int device, bdft_ctx** out) {
   if (ctx->plane_lds) {
     mfma_attributes(ctx->plane_lds);
     line_attributes(ctx->plane_lds);
+    fp64_attributes(ctx->plane_lds);
   }
   const char* env = getenv("BDFT_LINE_PASSES");
   ctx->force_lines = env && env[0] == '1';
@@ -703,6 +704,8 @@ static int box_tiles(const BoxDesc& b, int pass, int zg) {
     case P_KZG: return cdiv((long long)cdiv(4LL * N1 * N2, TW), zg);
     case P_ZPG: return cdiv((long long)cdiv(L1, TW) * L2, zg);
     case P_ZPF: return cdiv((long long)L1 * L2, TW);
+    case P_CZ: return cdiv((long long)N1 * N2, CCOL);
+    case P_RP: return b.L[2];
   }
   return 0;
 }
@@ -719,6 +722,8 @@ struct PlanChoice {
   int fused, zvalu, bvalu;  // matrix-core sequence
   int plane;                // vector-unit sequence: plane-fused or line passes
   int xbig, zbig;
+  int nthr_rp[4];           // FP64 potential pass: threads by launch shape
+                            // (they set the order of the epot sums)
 };
 
 // point the plan's grids at their places in a workspace of ws_need bytes
@@ -728,6 +733,7 @@ static void bind_ws(bdft_plan* plan, char* w) {
   plan->B.T1 = w + plan->ws_at[2];
   plan->B.T2 = w + plan->ws_at[3];
   plan->B.T3 = w + plan->ws_at[4];
+  plan->B.TZ = w + plan->ws_at[5];
 }
 
 static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
@@ -759,8 +765,8 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   const bool f16 = precision == BDFT_PREC_F16X3;
   TabSet tabs;
   std::vector<BoxDesc> box((size_t)norb);
-  long long wtot = 0, t1tot = 0, t2tot = 0, t3tot = 0, psi_run = 0;
-  int maxN = 0;
+  long long wtot = 0, t1tot = 0, t2tot = 0, t3tot = 0, tztot = 0, psi_run = 0;
+  int maxN = 0, maxN3 = 0;
   bool xbig = false, zbig = false;
   int maxL3 = 0;
   bool need_zero = false;
@@ -811,6 +817,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     b.t1_off = t1tot;
     b.t2_off = t2tot;
     b.t3_off = t3tot;
+    b.tz_off = tztot;
     b.pot_off = pot_off ? pot_off[i] : 0;
     const long long ncoef = (long long)lr->nvctr_c + 7LL * lr->nvctr_f;
     // no psi_off: orbitals stored one after the other
@@ -832,9 +839,11 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     t1tot += (long long)b.L[0] * 4 * b.N[1] * b.N[2];
     t2tot += (long long)b.L[0] * b.L[1] * 2 * b.N[2];
     t3tot += (long long)b.L[0] * b.L[1] * b.L[2];
+    tztot += 4LL * b.N[0] * b.N[1] * b.L[2];
     xbig = xbig || b.N[0] > REG_N || b.L[0] > REG_L;
     zbig = zbig || b.L[2] > REG_L;
     maxL3 = std::max(maxL3, b.L[2]);
+    maxN3 = std::max(maxN3, b.N[2]);
     if (!lr->dense) need_zero = true;
   }
   // bundles per z-line tile of the matrix-core sequence: three, unless a
@@ -882,9 +891,8 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
       starts.push_back(acc);
     }
   }
-  // plane-fused sequence when every box qualifies: periodic axes need at
-  // least 18 coarse points (single wrap of the in-plane stencils) and both
-  // plane kernels must fit in LDS
+  // plane-fused sequence when the planes (and the FP64 sequence's z lines) of
+  // every box fit in LDS
   MfmaLds ml{};
   ml.zg = zg;
   bool mfma_bwd_ok = true, valu_bwd_ok = false;  // units that fit the backward pass
@@ -1053,36 +1061,55 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     // density plans (grow_plane) use the forward plane kernel without its
     // kinetic part; the preconditioner's plans keep the line passes
     bool plane = !ctx->force_lines && !mfma && (!density || grow_plane);
-    size_t lpf = 0, lpb = 0;
+    const bool d64 = esz == 8 && !density;   // the FP64 sequence (bdft_fp64.hip)
+    size_t lpf = 0, lpb = 0, lcz = 0;
+    bool fits = true;
     for (int i = 0; i < norb && plane; ++i) {
       const BoxDesc& b = box[i];
-      lpf = std::max(lpf, plane_lds_fwd(b.N[0], b.N[1], b.L[0], (int)esz));
-      lpb = std::max(lpb, plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1], (int)esz));
+      if (d64) {
+        fits = fits && fp64_fit_kin(b, ctx->plane_lds).shape &&
+               fp64_fit_pot(b, ctx->plane_lds).shape;
+        const size_t z = fp64_fit_z(b, ctx->plane_lds);
+        fits = fits && z;
+        lcz = std::max(lcz, z);
+      } else {
+        lpf = std::max(lpf, plane_lds_fwd(b.N[0], b.N[1], b.L[0], (int)esz));
+        lpb = std::max(lpb, plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1], (int)esz));
+      }
     }
-    if (std::max(lpf, lpb) > ctx->plane_lds) plane = false;
+    if (!fits || std::max(lpf, lpb) > ctx->plane_lds) plane = false;
     T.plane = plane ? 1 : 0;
     if (force) T.plane = force->plane;
     T.lds_pf = lpf;
     T.lds_pb = lpb;
-    // forward plane pass: the boxes grouped by how many of their
-    // work-groups fit a CU, by LDS and by threads (FP64: 768 per work-group,
-    // at most two; FP32: 512, at most four), one launch per group with the
-    // group's largest LDS, so that the largest box does not set every
-    // work-group's LDS; one group: the single launch over t[P_PF]
-    auto group = [&](int pass, int cap, auto lds_of, TileTable* tg, int* nt, size_t* lg,
-                     int* fitv, int& n, int off[4][2]) {
+    T.lds_cz = lcz;
+    T.maxN3 = maxN3;
+    T.maxL3 = maxL3;
+    // plane passes: the boxes grouped by how many of their work-groups fit a
+    // CU (FP32, at most four) or by launch shape (FP64), one launch per group
+    // with the group's largest LDS, so that the largest box does not set
+    // every work-group's LDS.  One group (n = 0) runs as a single launch
+    // over t[pass], with entry 0's shape, threads and LDS.
+    auto group = [&](int pass, auto fit_of, TileTable* tg, int* nt, size_t* lg, int* shape,
+                     int* nthr, int& n, int off[4][2]) {
       n = 0;
       std::vector<int> grp[4];
-      size_t gl[4] = {0, 0, 0, 0};
+      PlaneFit most[4] = {};
       for (int i = 0; i < norb; ++i) {
-        const size_t v = lds_of(box[i]);
-        const size_t fit = ctx->plane_lds / std::max(v, (size_t)1);
-        const int c = (int)std::min((size_t)cap, std::max((size_t)1, fit));
-        grp[c - 1].push_back(i);
-        gl[c - 1] = std::max(gl[c - 1], v);
+        const PlaneFit f = fit_of(box[i]);
+        const int c = f.shape - 1;
+        grp[c].push_back(i);
+        most[c].nt = std::max(most[c].nt, f.nt);
+        most[c].lds = std::max(most[c].lds, f.lds);
       }
       int ng = 0;
-      for (int c = 0; c < 4; ++c) ng += grp[c].empty() ? 0 : 1;
+      for (int c = 0; c < 4; ++c)
+        if (!grp[c].empty()) {
+          ++ng;
+          shape[0] = c + 1;
+          nthr[0] = most[c].nt;
+          lg[0] = most[c].lds;
+        }
       if (ng < 2) return;
       for (int c = 4; c >= 1; --c)
         if (!grp[c - 1].empty()) {
@@ -1097,22 +1124,36 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
           off[k][1] = (int)starts.size();
           for (int i : grp[c - 1]) starts.push_back(i);
           nt[k] = acc;
-          if (fitv) fitv[k] = c;
+          shape[k] = c;
+          nthr[k] = most[c - 1].nt;
           tg[k].nbox = (int)grp[c - 1].size();
           tg[k].uniform = 0;
-          lg[k] = gl[c - 1];
+          lg[k] = most[c - 1].lds;
         }
     };
     T.n_pfg = T.n_pbg = 0;
-    if (T.plane && !mfma && !density && ctx->plane_lds > 0) {
-      group(P_PF, esz == 8 ? 2 : 4,
-            [&](const BoxDesc& b) { return plane_lds_fwd(b.N[0], b.N[1], b.L[0], (int)esz); },
-            T.pfg, T.nt_pfg, T.lds_pfg, nullptr, T.n_pfg, pf_off);
-      group(P_PB, esz == 8 ? 2 : 4,
+    if (T.plane && d64) {
+      group(P_PF, [&](const BoxDesc& b) { return fp64_fit_kin(b, ctx->plane_lds); }, T.pfg,
+            T.nt_pfg, T.lds_pfg, T.shape_pfg, T.nthr_pfg, T.n_pfg, pf_off);
+      group(P_RP, [&](const BoxDesc& b) { return fp64_fit_pot(b, ctx->plane_lds); }, T.pbg,
+            T.nt_pbg, T.lds_pbg, T.shape_pbg, T.nthr_pbg, T.n_pbg, pb_off);
+      for (int k = 0; k < std::max(1, T.n_pbg) && force; ++k)
+        T.nthr_pbg[k] = force->nthr_rp[T.shape_pbg[k] - 1];
+    } else if (T.plane && !density && ctx->plane_lds > 0) {
+      auto fit = [&](size_t v) {
+        const size_t c = ctx->plane_lds / std::max(v, (size_t)1);
+        return PlaneFit{(int)std::min((size_t)4, std::max((size_t)1, c)), 0, v};
+      };
+      group(P_PF,
             [&](const BoxDesc& b) {
-              return plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1], (int)esz);
+              return fit(plane_lds_fwd(b.N[0], b.N[1], b.L[0], (int)esz));
             },
-            T.pbg, T.nt_pbg, T.lds_pbg, T.fit_pbg, T.n_pbg, pb_off);
+            T.pfg, T.nt_pfg, T.lds_pfg, T.shape_pfg, T.nthr_pfg, T.n_pfg, pf_off);
+      group(P_PB,
+            [&](const BoxDesc& b) {
+              return fit(plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1], (int)esz));
+            },
+            T.pbg, T.nt_pbg, T.lds_pbg, T.shape_pbg, T.nthr_pbg, T.n_pbg, pb_off);
     }
     // preconditioner plans (FP64): the x and y operator as one plane pass
     // where the W and K planes of the largest box fit in LDS
@@ -1132,6 +1173,11 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     T.t[P_PF].xcd = T.t[P_PB].xcd = T.t[P_UNC].xcd = po;
     T.pf2.xcd = T.pb2.xcd = po;
     for (int k = 0; k < 4; ++k) T.vbg[k].xcd = T.pfg[k].xcd = T.pbg[k].xcd = po;
+    // the two x-y kinetic planes of a coarse z read the same fine records
+    if (esz == 8 && !density) {
+      T.t[P_PF].xcd = 1;
+      for (int k = 0; k < 4; ++k) T.pfg[k].xcd = 1;
+    }
   }
   if (force) {
     xbig = force->xbig;
@@ -1146,6 +1192,8 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     got->plane = T.plane;
     got->xbig = xbig;
     got->zbig = zbig;
+    for (int k = 0; k < std::max(1, T.n_pbg); ++k)
+      if (esz == 8 && T.plane) got->nthr_rp[T.shape_pbg[k] - 1] = T.nthr_pbg[k];
     return BDFT_OK;  // choices only: nothing allocated
   }
   bdft_plan* plan = new bdft_plan();
@@ -1205,7 +1253,13 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   }
   const size_t nb_st = sizeof(int) * starts.size();
   int epass[4] = {P_XF, P_KY, P_KZ, P_ZP};
-  if (T.plane) epass[0] = P_PF;
+  const bool fp64_seq = T.plane && esz == 8 && !density;
+  if (fp64_seq) {
+    epass[0] = P_CZ;
+    epass[3] = P_RP;
+  } else if (T.plane) {
+    epass[0] = P_PF;
+  }
   plan->mlds = ml;
   if (mfma) {
     const size_t nt = sizeof(OpTab) * tabs.tabs.size();
@@ -1254,9 +1308,11 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   plan->B.tmax = f16 ? (float*)(m + al(nb_box) + al(nb_st) + al(nb_part) +
                                 al(sizeof(unsigned) * norb))
                      : nullptr;
-  hipError_t e1 = plan_h2d(arena, dbox, box.data(), nb_box);
-  hipError_t e2 = plan_h2d(arena, dst, starts.data(), nb_st);
-  if (e1 != hipSuccess || e2 != hipSuccess) {
+  // boxes and starts in one copy
+  std::vector<unsigned char> up(nb_st ? al(nb_box) + nb_st : nb_box);
+  memcpy(up.data(), box.data(), nb_box);
+  if (nb_st) memcpy(up.data() + al(nb_box), starts.data(), nb_st);
+  if (plan_h2d(arena, dbox, up.data(), up.size()) != hipSuccess) {
     dev_free(plan->meta);
     dev_free(plan->tabbuf);
     delete plan;
@@ -1305,16 +1361,23 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   // workspace: W | K | T1 | T2 | T3
   if (T.plane || mfma) t1tot = 0;
   if (!zbig) t3tot = 0;
+  // (FP64 sequence: K | TZ)
+  long long wv = wtot;
+  if (fp64_seq) wv = t2tot = t3tot = 0;
+  else tztot = 0;
   T.xbig = xbig;
   T.zbig = zbig;
   T.zshort = maxL3 <= ZSHORT_L;
-  const size_t ws_bytes = esz * (2 * al(wtot) + al(t1tot) + al(t2tot) + al(t3tot));
-  plan->ws_need = ws_bytes;
-  plan->ws_at[0] = 0;
-  plan->ws_at[1] = esz * al(wtot);
-  plan->ws_at[2] = esz * 2 * al(wtot);
-  plan->ws_at[3] = esz * (2 * al(wtot) + al(t1tot));
-  plan->ws_at[4] = esz * (2 * al(wtot) + al(t1tot) + al(t2tot));
+  {
+    const long long part[6] = {wv, wtot, t1tot, t2tot, t3tot, tztot};
+    size_t at = 0;
+    for (int k = 0; k < 6; ++k) {
+      plan->ws_at[k] = at;
+      at += esz * al(part[k]);
+    }
+    plan->ws_need = at;
+  }
+  const size_t ws_bytes = plan->ws_need;
   Batch& B = plan->B;
   B.box = dbox;
   B.nbox = norb;
@@ -2287,7 +2350,7 @@ extern "C" int bdft_compress_acc_d(bdft_ctx* ctx, const bdft_lr* lr, int norb,
 static const char* kStageNames[S_COUNT] = {
     "zero",   "uncompress", "x_grow_kin", "y_grow", "y_kin",    "z_kin",
     "z_pot",  "y_shrink",   "x_shrink",   "compress", "energy", "xy_fwd",
-    "xy_bwd_compress"};
+    "xy_bwd_compress", "z_grow", "xy_kin", "xy_pot", "z_back"};
 
 extern "C" int bdft_profile_enable(bdft_ctx* ctx, int on) {
   if (!ctx) return BDFT_ERR_ARG;

@@ -1,0 +1,878 @@
+// FP64 sequence of the local-Hamiltonian apply.
+//
+//   k_zgrow    psi -> TZ = G_z W            64 z lines of 16 coarse columns
+//   k_xykin    psi -> K  = K_x W + K_y W    one x-y plane of W
+//   k_xypot    TZ <- G_x^T G_y^T V G_y G_x TZ   one x-y plane at a fine z point
+//   k_zback    hpsi += compress(G_z^T TZ + K + K_z W)   64 z lines
+//
+// The wavelet volume W never reaches memory: the kernels that need it gather
+// it from the compressed coefficients (every 56-byte fine record read whole
+// by the z kernels, by two neighbouring planes in k_xykin), and V is applied
+// between the two halves of one plane's work, so the only grids are TZ
+// (2 N1 x 2 N2 x L3) and K.  88 bytes move per point of a periodic box where
+// the x-y-z order with W, K and (L1, L2, 2 N3) grids moved 112; a free box's
+// TZ is also (2 N1 2 N2 L3) / (L1 L2 2 N3) of that grid (0.66 at 28 coarse
+// points an axis).  Operators and filters are those of the line kernels
+// (growshrink.f90 comb_grow / comb_shrink, convolut_ib_optim.f90
+// ConvolkineticT); sums run in another order of the axes.
+//
+// Measured on 128 orbitals of a periodic 40^3 box (6.6e7 fine points), the
+// x-y-z order's kernels before: uncompress 183 us, forward planes 1085, z
+// kinetic 553, z potential 413, backward planes 689, an apply 2.65 ms; now
+// k_zgrow 0.24 ms (16 B per point: 4.4 TB/s, a large copy runs at 4.9),
+// k_xykin 0.52 and k_xypot 0.52 (3.5 and 3.7 times the time of their FMAs at
+// the FP64 peak; waits at barriers and LDS loads), k_zback 0.68 (40 B per
+// point: 3.9 TB/s), an apply 1.80 ms.  48 orbitals of a 64^3 box, whose pairs
+// of planes did not fit in LDS (line passes): 4.64 -> 2.99 ms; 256 free boxes
+// of 16 to 40 points an axis 2.70 -> 2.19 ms.
+//
+// Grid TZ of a box (tz_off): plane p3 = 0 .. L3 - 1, in it the wavelet plane
+// [j1 + 2 N1 j2]; K (w_off): the wavelet volume.
+#include <algorithm>
+
+#include "bdft_internal.h"
+#include "bdft_stencil.h"
+
+namespace bdft {
+
+// ---------------------------------------------------------------------------
+// z-line tiles: CC coarse columns q = i1 + N1 i2 of a box, each with its four
+// z lines (s1, s2): line l = col + CC (s1 + 2 s2), one lane per line.  A wave
+// works on one chunk of outputs of all 64 lines, so the chunk's rows are
+// uniform over the wave: LDS rows are read without bank conflicts at
+// immediate offsets, and a line end costs scalar instructions only.
+// ---------------------------------------------------------------------------
+constexpr int CC = CCOL;
+constexpr int NL = 4 * CC;      // lines of a tile
+static_assert(NL == 64, "one lane per line");
+
+// W of the tile's columns into LDS: row s3 N3 + i3 (wavelet z index),
+// lane l.  Thread e = tid mod 128 moves element e of every (tid / 128)-th coarse
+// z: columns' scaling coefficients for e < 16, else component (e - 16) mod 7
+// of column (e - 16) / 7, the order the records have in memory.
+struct RecElem {
+  int col, t;                   // column and component 0..7
+  __device__ __forceinline__ explicit RecElem(int e) {
+    if (e < CC) {
+      col = e;
+      t = 0;
+    } else {
+      col = (e - CC) / 7;
+      t = e - CC - 7 * col + 1;
+    }
+  }
+};
+
+template <int NT>
+__device__ __forceinline__ void load_columns(double* lds, const BoxDesc& bd, const double* psi,
+                                             int q0, int nq) {
+  constexpr int ZS = NT / 128, UR = 8;
+  const int N3 = bd.N[2], npl = bd.N[0] * bd.N[1];
+  const RecElem re(threadIdx.x & 127);
+  const int z0 = threadIdx.x >> 7;
+  const bool on = re.col < nq;
+  const int lin0 = q0 + (on ? re.col : 0);
+  const char* src = (const char*)(psi + bd.psi_off);
+  const unsigned off = re.t == 0 ? 0u : 8u * (unsigned)(bd.nvctr_c + re.t - 1);
+  const unsigned mul = re.t == 0 ? 8u : 56u;
+  double* dst = lds + (re.t >> 2) * N3 * NL + re.col + CC * (re.t & 3);
+  if (!bd.cinv && !bd.finv) {
+    for (int zb = z0; zb < N3; zb += ZS * UR) {
+      double v[UR];
+#pragma unroll
+      for (int u = 0; u < UR; ++u) {
+        const int z = min(zb + u * ZS, N3 - 1);
+        v[u] = *(const double*)(src + (off + mul * (unsigned)(lin0 + npl * z)));
+      }
+#pragma unroll
+      for (int u = 0; u < UR; ++u)
+        if (zb + u * ZS < N3) dst[(zb + u * ZS) * NL] = on ? v[u] : 0.0;
+    }
+  } else {
+    const int* inv = re.t == 0 ? bd.cinv : bd.finv;
+    for (int zb = z0; zb < N3; zb += ZS * UR) {
+      int r[UR];
+      double v[UR];
+#pragma unroll
+      for (int u = 0; u < UR; ++u) {
+        const int z = zb + u * ZS, lin = lin0 + npl * z;
+        r[u] = -1;
+        if (on && z < N3) r[u] = inv ? inv[lin] : lin;
+      }
+#pragma unroll
+      for (int u = 0; u < UR; ++u) {
+        v[u] = 0.0;
+        if (r[u] >= 0) v[u] = *(const double*)(src + (off + mul * (unsigned)r[u]));
+      }
+#pragma unroll
+      for (int u = 0; u < UR; ++u)
+        if (zb + u * ZS < N3) dst[(zb + u * ZS) * NL] = v[u];
+    }
+  }
+}
+
+// The taps of rows k0 .. k0 + NK - 1 of a line, k0 uniform over the wave:
+// tap(kk, k) with k a valid row.  Rows past a line end wrap (periodic) or
+// are left out (free: they hold zeros).
+template <int NK, typename F>
+__device__ __forceinline__ void line_taps(int k0, int n, int per, F tap) {
+  if (k0 >= 0 && k0 + NK <= n) {
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) tap(kk, k0 + kk);
+  } else if (per) {
+    int k = k0;
+    while (k < 0) k += n;
+    while (k >= n) k -= n;
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) {
+      tap(kk, k);
+      k = k + 1 == n ? 0 : k + 1;
+    }
+  } else {
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk)
+      if (k0 + kk >= 0 && k0 + kk < n) tap(kk, k0 + kk);
+  }
+}
+
+// a tile's lines: first column, columns, and this lane's line
+struct ColTile {
+  int q0, nq;
+  bool on;       // this lane's column is one of the box
+  unsigned at;   // its line in a wavelet plane, j1 + 2 N1 j2
+  __device__ __forceinline__ ColTile(const BoxDesc& bd, int lt) {
+    const int N1 = bd.N[0], N2 = bd.N[1];
+    q0 = lt * CC;
+    nq = min(CC, N1 * N2 - q0);
+    const int lane = threadIdx.x & 63, col = lane & (CC - 1), s = lane / CC;
+    on = col < nq;
+    const int q = q0 + (on ? col : 0);
+    const int i2 = qdiv(q, N1, 1.0f / (float)N1), i1 = q - i2 * N1;
+    at = (unsigned)(i1 + N1 * (s & 1) + 2 * N1 * (i2 + N2 * (s >> 1)));
+  }
+};
+
+// ---------------------------------------------------------------------------
+// TZ = G_z W
+// ---------------------------------------------------------------------------
+constexpr int ZG_NT = 256;
+__global__ __launch_bounds__(ZG_NT) void k_zgrow(Batch B, TileTable tt) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  double* lds = (double*)smem;
+  const int tile = tile_of(tt);
+  const int lb = find_box(tt, tile);
+  const BoxDesc bd = B.box[table_box(tt, lb)];
+  const int N3 = bd.N[2], L3 = bd.L[2], per = bd.per;
+  const ColTile ct(bd, tile - box_first_tile(tt, lb));
+  load_columns<ZG_NT>(lds, bd, B.psi, ct.q0, ct.nq);
+  __syncthreads();
+  const double* c = lds + (threadIdx.x & 63);
+  const double* d = c + N3 * NL;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const size_t ps = 4 * (size_t)(bd.N[0] * bd.N[1]);
+  double* out = (double*)B.TZ + bd.tz_off + ct.at;
+  for (int p0 = 8 * w; p0 < L3; p0 += 8 * (ZG_NT / 64)) {
+    double o[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) o[r] = 0.0;
+    line_taps<19>(grow_k0(p0, per), N3, per,
+                  [&](int kk, int k) { grow_tap(kk, c[k * NL], d[k * NL], o); });
+    if (ct.on) {
+      double* q = out + ps * p0;
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        if (p0 + r < L3) q[ps * r] = o[r];
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// hpsi += compress(G_z^T TZ + K + K_z W), ekin partial.  MI: chunks of four
+// coarse z per wave, their sums held in registers while the LDS rows change
+// from W to TZ to the records of hpsi.
+// ---------------------------------------------------------------------------
+template <int ZB_NT, int MI, int WPE>
+__global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, TileTable ft,
+                                                 double* part) {
+  constexpr int NW = ZB_NT / 64;
+  extern __shared__ __align__(16) unsigned char smem[];
+  double* lds = (double*)smem;
+  __shared__ double red[NW];
+  const int tile = tile_of(tt);
+  const int lb = find_box(tt, tile);
+  const int b = table_box(tt, lb);
+  const BoxDesc bd = B.box[b];
+  const int lt = tile - box_first_tile(tt, lb);
+  const int N3 = bd.N[2], L3 = bd.L[2], per = bd.per;
+  const ColTile ct(bd, lt);
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const size_t ps = 4 * (size_t)(bd.N[0] * bd.N[1]);
+  load_columns<ZB_NT>(lds, bd, B.psi, ct.q0, ct.nq);
+  __syncthreads();
+  double o[MI][8];   // c, then d
+  double ek = 0.0;
+  {
+    const double* c = lds + lane;
+    const double* d = c + N3 * NL;
+    const double ks = bd.kscale[2];
+    const double* K = (const double*)B.K + bd.w_off + ct.at;
+#pragma unroll
+    for (int m = 0; m < MI; ++m) {
+      const int i0 = 4 * (w + m * NW);
+      if (i0 < N3) {
+        double k[8];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int z = min(i0 + r, N3 - 1);
+          k[r] = K[ps * z];
+          k[4 + r] = K[ps * (N3 + z)];
+          o[m][r] = o[m][4 + r] = 0.0;
+        }
+        line_taps<32>(i0 - 14, N3, per, [&](int kk, int z) {
+          kin_tap(kk, c[z * NL], d[z * NL], o[m], o[m] + 4);
+        });
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          o[m][r] = fma(o[m][r], ks, k[r]);
+          o[m][4 + r] = fma(o[m][4 + r], ks, k[4 + r]);
+          if (i0 + r < N3) {   // lanes off the box hold W = 0
+            ek = fma(o[m][r], c[(i0 + r) * NL], ek);
+            ek = fma(o[m][4 + r], d[(i0 + r) * NL], ek);
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();
+  {
+    // the lines of TZ: one row of 64 values per wave and step
+    const double* src = (const double*)B.TZ + bd.tz_off + ct.at;
+    constexpr int UR = 8;
+    for (int pb = w; pb < L3; pb += NW * UR) {
+      double v[UR];
+#pragma unroll
+      for (int u = 0; u < UR; ++u) v[u] = src[ps * min(pb + u * NW, L3 - 1)];
+#pragma unroll
+      for (int u = 0; u < UR; ++u)
+        if (pb + u * NW < L3) lds[(pb + u * NW) * NL + lane] = v[u];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    const int i0 = 4 * (w + m * NW);
+    if (i0 < N3) {
+      // summed by itself: on top of the larger kinetic term every tap would
+      // round at its size
+      double g[8] = {};
+      line_taps<37>(per ? 2 * i0 - 14 : 2 * i0, L3, per, [&](int qq, int p) {
+        shrink_tap<double, 4>(qq, lds[p * NL + lane], g, g + 4);
+      });
+#pragma unroll
+      for (int r = 0; r < 8; ++r) o[m][r] += g[r];
+    }
+  }
+  const double eks = block_sum_rt(ek, red);   // starts with a barrier
+  if (threadIdx.x == 0) part[box_first_tile(ft, b) + lt] = eks;
+  // the sums as records: row i3, element e of RecElem (lane's component
+  // s + 4 s3, s = lane / CC; component 0 is the scaling coefficient)
+  {
+    const int col = lane & (CC - 1), s = lane / CC;
+    const int ec = s == 0 ? col : CC + 7 * col + s - 1, ed = CC + 7 * col + s + 3;
+#pragma unroll
+    for (int m = 0; m < MI; ++m) {
+      const int i0 = 4 * (w + m * NW);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (i0 + r < N3) {
+          lds[(i0 + r) * 2 * NL + ec] = o[m][r];
+          lds[(i0 + r) * 2 * NL + ed] = o[m][4 + r];
+        }
+    }
+  }
+  __syncthreads();
+  {
+    constexpr int ZS = ZB_NT / 128, UR = 4;
+    const int e = threadIdx.x & 127, npl = bd.N[0] * bd.N[1];
+    const RecElem re(e);
+    if (re.col < ct.nq) {
+      char* dst = (char*)(B.hpsi + bd.psi_off);
+      const unsigned off = re.t == 0 ? 0u : 8u * (unsigned)(bd.nvctr_c + re.t - 1);
+      const unsigned mul = re.t == 0 ? 8u : 56u;
+      const int lin0 = ct.q0 + re.col;
+      const int* inv = re.t == 0 ? bd.cinv : bd.finv;
+      for (int zb = threadIdx.x >> 7; zb < N3; zb += ZS * UR) {
+        int rec[UR];
+        double v[UR];
+#pragma unroll
+        for (int u = 0; u < UR; ++u) {
+          const int z = zb + u * ZS, lin = lin0 + npl * z;
+          rec[u] = -1;
+          if (z < N3) rec[u] = inv ? inv[lin] : lin;
+        }
+#pragma unroll
+        for (int u = 0; u < UR; ++u)
+          v[u] = rec[u] >= 0 ? *(const double*)(dst + (off + mul * (unsigned)rec[u])) : 0.0;
+#pragma unroll
+        for (int u = 0; u < UR; ++u)
+          if (rec[u] >= 0)
+            *(double*)(dst + (off + mul * (unsigned)rec[u])) =
+                v[u] + lds[(zb + u * ZS) * 2 * NL + e];
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// in-plane passes.  One of a thread's work items is one chunk of a line, lanes along the
+// lines.  A pass keeps its items' outputs in registers (at most MI items of 8
+// values a thread) and writes them over the plane after a barrier, transposed
+// where the next pass runs along the other axis: the lines are LDS rows of
+// odd stride (taps at immediate offsets, 64 lanes on 64 rows meet no bank
+// twice) and one plane of LDS serves all passes, two work-groups per CU up to
+// 49 periodic or 36 free coarse points (two planes, 150 KB at 48, allow one,
+// whose load, passes and store run one after the other).  Two chunks of a
+// line per item (half the LDS reads, half the coefficients) and coefficients
+// from scalar loads (half the scalar instructions) were both slower: 0.60 and
+// 0.65 ms against 0.59 for k_xypot on the batch above.
+//
+// Line ends: a wave whose chunks all lie inside their lines reads them
+// directly.  Otherwise, periodic: through a line map in LDS (any N); free:
+// the taps past the line are masked out per lane (they read whatever lies
+// next to the row, PAD values around the plane keep that inside the
+// allocation) and cost nothing where the whole wave is past the line.
+// ---------------------------------------------------------------------------
+constexpr int PAD = 24;   // rows are read at most 15 values before and 20 past their end
+
+// NK taps from value k0 of a line of n values: load(kk) reads tap kk's
+// input(s) from the row, mapped(kk) through the line map, apply(kk, x) adds
+// it to the outputs
+template <int NK, typename FL, typename FM, typename FA>
+__device__ __forceinline__ void row_taps(int k0, int n, int per, FL load, FM mapped, FA apply) {
+  if (__all(k0 >= 0 && k0 + NK <= n)) {
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) apply(kk, load(kk));
+  } else if (per) {
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) apply(kk, mapped(kk));
+  } else {
+    // loads run two taps ahead of the masked sums
+    auto x0 = load(0), x1 = load(1);
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) {
+      const auto x = x0;
+      x0 = x1;
+      if (kk + 2 < NK) x1 = load(kk + 2);
+      if ((unsigned)(k0 + kk) < (unsigned)n) apply(kk, x);
+    }
+  }
+}
+
+__device__ __forceinline__ double2 at2(const double* ln, int2 e) {
+  return make_double2(*(const double*)((const char*)ln + e.x),
+                      *(const double*)((const char*)ln + e.y));
+}
+
+// G of a wavelet row [c; d] of N + N values: 8 fine outputs from k = k0 ..
+// k0 + 18; m: the axis's coarse line map
+__device__ __forceinline__ void grow_row(const double* ln, const int2* m, int N, int k0, int per,
+                                         double o[8]) {
+#pragma unroll
+  for (int r = 0; r < 8; ++r) o[r] = 0.0;
+  const double *c = ln + k0, *d = ln + N + k0;
+  const int2* mm = m + (k0 + MOFF);
+  row_taps<19>(
+      k0, N, per, [&](int kk) { return make_double2(c[kk], d[kk]); },
+      [&](int kk) { return at2(ln, mm[kk]); },
+      [&](int kk, double2 x) { grow_tap(kk, x.x, x.y, o); });
+}
+
+// wavelet-basis kinetic (unscaled) of a wavelet row: coarse outputs i0 .. i0
+// + 3 (c in o[0..3], d in o[4..7])
+__device__ __forceinline__ void kin_row(const double* ln, const int2* m, int N, int i0, int per,
+                                        double o[8]) {
+#pragma unroll
+  for (int r = 0; r < 8; ++r) o[r] = 0.0;
+  const double *c = ln + i0 - 14, *d = ln + N + i0 - 14;
+  const int2* mm = m + (i0 - 14 + MOFF);
+  row_taps<32>(
+      i0 - 14, N, per, [&](int kk) { return make_double2(c[kk], d[kk]); },
+      [&](int kk) { return at2(ln, mm[kk]); },
+      [&](int kk, double2 x) { kin_tap(kk, x.x, x.y, o, o + 4); });
+}
+
+// G^T of a fine row of L values: coarse outputs i0 .. i0 + 3; m: fine line
+// map (periodic)
+__device__ __forceinline__ void shrink_row(const double* ln, const int* m, int L, int i0,
+                                           int per, double o[8]) {
+#pragma unroll
+  for (int r = 0; r < 8; ++r) o[r] = 0.0;
+  const int p0 = per ? 2 * i0 - 14 : 2 * i0;
+  const double* x = ln + p0;
+  const int* mm = m + 2 * i0;
+  row_taps<37>(
+      p0, L, per, [&](int qq) { return x[qq]; },
+      [&](int qq) { return *(const double*)((const char*)ln + mm[qq]); },
+      [&](int qq, double v) { shrink_tap<double, 4>(qq, v, o, o + 4); });
+}
+
+// line maps of a periodic axis: coarse entry e (k = e - MOFF, up to N + 20):
+// byte offsets of c and d at k modulo N; fine entry e (up to 2 N + 42): that
+// of fine index e - 14 modulo 2 N
+__host__ __device__ constexpr int cmap_len(int N) { return N + MOFF + 21; }
+__host__ __device__ constexpr int smap_len(int N) { return 2 * N + 44; }
+__device__ __forceinline__ void build_maps(int2* mc, int* mf, int N, int tid, int nt) {
+  for (int e = tid; e < cmap_len(N); e += nt) {
+    int k = e - MOFF;
+    while (k < 0) k += N;
+    while (k >= N) k -= N;
+    mc[e] = make_int2(8 * k, 8 * (N + k));
+  }
+  if (mf)
+    for (int e = tid; e < smap_len(N); e += nt) {
+      int p = e - 14;
+      while (p < 0) p += 2 * N;
+      while (p >= 2 * N) p -= 2 * N;
+      mf[e] = 8 * p;
+    }
+}
+
+// items (chunk ch, line j) of a pass over nch chunks of n lines; d: the
+// thread's first item
+template <int MI, typename F>
+__device__ __forceinline__ void each_item(ItDiv d, int n, int nch, F f) {
+#pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    if (d.ch < nch) f(m, d.ch, d.j);
+    d.next(n);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// K = K_x W + K_y W of one x-y plane (wavelet z index i3 + N3 s3; the two
+// planes of a coarse z are neighbouring tiles: they read the same fine
+// records).  K_y, along the columns, goes to memory first; K_x goes over the
+// plane in LDS and from there is added to it.
+// ---------------------------------------------------------------------------
+template <int NTM, int MI, int WPE>
+__global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int tile = tile_of(tt);
+  const int lb = find_box(tt, tile);
+  const BoxDesc bd = B.box[table_box(tt, lb)];
+  const int lt = tile - box_first_tile(tt, lb);
+  const int N1 = bd.N[0], N2 = bd.N[1], N3 = bd.N[2], per = bd.per;
+  const int s3 = lt & 1, i3 = lt >> 1;
+  const int W1 = 2 * N1, W2 = 2 * N2, RA = W1 + 1, npl = N1 * N2;
+  double* A = (double*)smem;
+  int2* mx = (int2*)(A + (W2 + 1) * RA);
+  int2* my = mx + map_len(N1);
+  const int tid = threadIdx.x, nt = blockDim.x;
+  // gather: thread's component c = s1 + 2 s2 of every (nt / 4)-th point
+  {
+    constexpr int UR = 8;
+    const int c = tid & 3, st = nt >> 2;
+    const bool cs = c == 0 && s3 == 0;
+    const char* src = (const char*)(B.psi + bd.psi_off);
+    const unsigned off = cs ? 0u : 8u * (unsigned)(bd.nvctr_c + c + 4 * s3 - 1);
+    const unsigned mul = cs ? 8u : 56u;
+    const int* inv = cs ? bd.cinv : bd.finv;
+    const bool dense = !bd.cinv && !bd.finv;
+    const int lin0 = npl * i3;
+    double* base = A + (c >> 1) * N2 * RA + (c & 1) * N1;
+    ItDiv d(tid >> 2, N1, st);
+    for (int pb = tid >> 2; pb < npl; pb += st * UR) {
+      double v[UR];
+      if (dense) {
+#pragma unroll
+        for (int u = 0; u < UR; ++u)
+          v[u] = *(const double*)(src + (off + mul * (unsigned)(lin0 + min(pb + u * st, npl - 1))));
+      } else {
+        int r[UR];
+#pragma unroll
+        for (int u = 0; u < UR; ++u) {
+          const int p = pb + u * st;
+          r[u] = -1;
+          if (p < npl) r[u] = inv ? inv[lin0 + p] : lin0 + p;
+        }
+#pragma unroll
+        for (int u = 0; u < UR; ++u)
+          v[u] = r[u] >= 0 ? *(const double*)(src + (off + mul * (unsigned)r[u])) : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < UR; ++u) {
+        if (pb + u * st < npl) base[d.ch * RA + d.j] = v[u];
+        d.next(N1);
+      }
+    }
+  }
+  build_map(mx, N1, per, sizeof(double), W1, tid, nt);
+  build_map(my, N2, per, RA * sizeof(double), W2, tid, nt);
+  for (int i = tid; i < W2; i += nt) A[i * RA + W1] = 0.0;
+  for (int i = tid; i < RA; i += nt) A[W2 * RA + i] = 0.0;
+  __syncthreads();
+  double* K = (double*)B.K + bd.w_off + (long long)W1 * W2 * (i3 + N3 * s3);
+  const double kx = bd.kscale[0], ky = bd.kscale[1];
+  const int cy = (N2 + 3) >> 2, cx = (N1 + 3) >> 2;
+  each_item<MI>(ItDiv(tid, W1, nt), W1, cy, [&](int, int ch, int j1) {
+    const int i0 = 4 * ch;
+    double oc[4], od[4];
+    kin4_any(PLine<double>{A + j1, RA}, my, N2, i0, oc, od);
+    const unsigned at = 8u * (unsigned)(j1 + W1 * i0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (i0 + r < N2) {
+        *(double*)((char*)(K + W1 * r) + at) = oc[r] * ky;
+        *(double*)((char*)(K + W1 * (N2 + r)) + at) = od[r] * ky;
+      }
+  });
+  double o[MI][8];
+  const ItDiv d2(tid, W2, nt);
+  each_item<MI>(d2, W2, cx, [&](int m, int ch, int j2) {
+    kin4_any(PLine<double>{A + j2 * RA, 1}, mx, N1, 4 * ch, o[m], o[m] + 4);
+  });
+  __syncthreads();
+  each_item<MI>(d2, W2, cx, [&](int m, int ch, int j2) {
+    double* a = A + j2 * RA + 4 * ch;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (4 * ch + r < N1) {
+        a[r] = o[m][r] * kx;
+        a[N1 + r] = o[m][4 + r] * kx;
+      }
+  });
+  __syncthreads();
+  // two values at a time (rows of 2 N1 values: 16-byte aligned)
+  const int tot = N1 * W2;
+  double2* K2 = (double2*)K;
+  ItDiv d(tid, N1, nt);
+  constexpr int UR = 4;
+  for (int i = tid; i < tot; i += nt * UR) {
+    double2 v[UR];
+#pragma unroll
+    for (int u = 0; u < UR; ++u) v[u] = K2[min(i + u * nt, tot - 1)];
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      if (i + u * nt < tot) {
+        const double* a = A + d.ch * RA + 2 * d.j;
+        K2[i + u * nt] = make_double2(v[u].x + a[0], v[u].y + a[1]);
+      }
+      d.next(N1);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// TZ <- G_x^T G_y^T V G_y G_x TZ of the plane at fine z point p3, epot
+// partial.  LDS: x lines as rows (stride RX) for G_x and G_x^T, y lines as
+// rows (RY) in between.
+// ---------------------------------------------------------------------------
+template <int NTM, int MI, int WPE>
+__global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileTable ft,
+                                                    double* part) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ double red[NTM / 64];
+  const int tile = tile_of(tt);
+  const int lb = find_box(tt, tile);
+  const int b = table_box(tt, lb);
+  const BoxDesc bd = B.box[b];
+  const int p3 = tile - box_first_tile(tt, lb);
+  const int N1 = bd.N[0], N2 = bd.N[1], L1 = bd.L[0], L2 = bd.L[1], per = bd.per;
+  const int W1 = 2 * N1, W2 = 2 * N2, RX = L1 | 1, RY = L2 | 1;
+  double* A = (double*)smem + PAD;
+  // line maps, one pair for both axes of a square plane
+  const bool sq = N1 == N2;
+  int2* mx = (int2*)(A + max(W2 * RX, L1 * RY) + PAD);
+  int2* my = mx + (sq ? 0 : cmap_len(N1));
+  int* sx = (int*)(my + cmap_len(N2));
+  int* sy = sx + (sq ? 0 : smap_len(N1));
+  const int tid = threadIdx.x, nt = blockDim.x;
+  double* T = (double*)B.TZ + bd.tz_off + (long long)W1 * W2 * p3;
+  // the plane, two values at a time (rows of 2 N1, planes of 4 N1 N2 values:
+  // 16-byte aligned)
+  const ItDiv dn(tid, N1, nt);
+  {
+    constexpr int UR = 4;
+    const int tot = N1 * W2;
+    const double2* src = (const double2*)T;
+    ItDiv d = dn;
+    for (int i = tid; i < tot; i += nt * UR) {
+      double2 v[UR];
+#pragma unroll
+      for (int u = 0; u < UR; ++u) v[u] = src[min(i + u * nt, tot - 1)];
+#pragma unroll
+      for (int u = 0; u < UR; ++u) {
+        if (i + u * nt < tot) {
+          double* a = A + d.ch * RX + 2 * d.j;
+          a[0] = v[u].x;
+          a[1] = v[u].y;
+        }
+        d.next(N1);
+      }
+    }
+  }
+  if (per) {
+    build_maps(mx, sx, N1, tid, nt);
+    if (!sq) build_maps(my, sy, N2, tid, nt);
+  }
+  __syncthreads();
+  double o[MI][8];
+  const ItDiv dw(tid, W2, nt), dl(tid, L1, nt);
+  // G_x on the rows j2, written as columns of the y rows
+  const int gx = (L1 + 7) >> 3, gy = (L2 + 7) >> 3;
+  each_item<MI>(dw, W2, gx, [&](int m, int ch, int j2) {
+    grow_row(A + j2 * RX, mx, N1, grow_k0(8 * ch, per), per, o[m]);
+  });
+  __syncthreads();
+  each_item<MI>(dw, W2, gx, [&](int m, int ch, int j2) {
+    double* a = A + 8 * ch * RY + j2;
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      if (8 * ch + r < L1) a[r * RY] = o[m][r];
+  });
+  __syncthreads();
+  // G_y and V on the rows p1.  V outside the potential box is zero, the
+  // zeroing of psir there (potential.f90:874-947); those points read a value
+  // of the box and discard it, so all loads of a chunk are in flight together
+  // while its stencil runs.
+  const int q3 = p3 - bd.ishift[2];
+  const bool in3 = q3 >= 0 && q3 < bd.potdim[2];
+  const unsigned pd1 = (unsigned)bd.potdim[0];
+  const double* pot = B.pot + bd.pot_off +
+                      (size_t)pd1 * (unsigned)bd.potdim[1] *
+                          (unsigned)min(max(q3, 0), bd.potdim[2] - 1);
+  const double cz = bd.conf_on ? conf_axis2(bd, 2, p3) : 0.0;
+  double ep = 0.0;
+  each_item<MI>(dl, L1, gy, [&](int m, int ch, int p1) {
+    const int q1 = p1 - bd.ishift[0], q20 = 8 * ch - bd.ishift[1];
+    // rows of the chunk inside the box and the potential box
+    const bool in13 = in3 && q1 >= 0 && q1 < bd.potdim[0];
+    const int rlo = -q20, rhi = in13 ? min(L2 - 8 * ch, bd.potdim[1] - q20) : 0;
+    double v[8];
+    const bool whole = __all(rlo <= 0 && rhi >= 8);
+    if (whole) {
+      const unsigned v0 = 8u * ((unsigned)q1 + pd1 * (unsigned)q20);
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        v[r] = *(const double*)((const char*)(pot + r * (size_t)pd1) + v0);
+    } else {
+      const unsigned v0 = (unsigned)min(max(q1, 0), bd.potdim[0] - 1);
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        v[r] = pot[v0 + pd1 * (unsigned)min(max(q20 + r, 0), bd.potdim[1] - 1)];
+    }
+    grow_row(A + p1 * RY, my, N2, grow_k0(8 * ch, per), per, o[m]);
+    if (bd.conf_on || !whole) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const bool ok = r >= rlo && r < rhi;
+        v[r] = ok ? v[r] : 0.0;
+        if (bd.conf_on && ok)
+          v[r] += conf_term(bd, cz + conf_axis2(bd, 0, p1) + conf_axis2(bd, 1, 8 * ch + r));
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const double vp = v[r] * o[m][r];
+      ep = fma(vp, o[m][r], ep);
+      o[m][r] = vp;
+    }
+  });
+  __syncthreads();
+  each_item<MI>(dl, L1, gy, [&](int m, int ch, int p1) {
+    double* a = A + p1 * RY + 8 * ch;
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      if (8 * ch + r < L2) a[r] = o[m][r];
+  });
+  __syncthreads();
+  // G_y^T on the rows p1, written as columns of the x rows
+  const int cy = (N2 + 3) >> 2, cx = (N1 + 3) >> 2;
+  each_item<MI>(dl, L1, cy, [&](int m, int ch, int p1) {
+    shrink_row(A + p1 * RY, sy, L2, 4 * ch, per, o[m]);
+  });
+  __syncthreads();
+  each_item<MI>(dl, L1, cy, [&](int m, int ch, int p1) {
+    double* a = A + 4 * ch * RX + p1;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (4 * ch + r < N2) {
+        a[r * RX] = o[m][r];
+        a[(N2 + r) * RX] = o[m][4 + r];
+      }
+  });
+  __syncthreads();
+  // G_x^T on the rows j2
+  each_item<MI>(dw, W2, cx, [&](int m, int ch, int j2) {
+    shrink_row(A + j2 * RX, sx, L1, 4 * ch, per, o[m]);
+  });
+  __syncthreads();
+  each_item<MI>(dw, W2, cx, [&](int m, int ch, int j2) {
+    double* a = A + j2 * RX + 4 * ch;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (4 * ch + r < N1) {
+        a[r] = o[m][r];
+        a[N1 + r] = o[m][4 + r];
+      }
+  });
+  const double eps = block_sum_rt(ep, red);   // has the barriers
+  if (tid == 0) part[box_first_tile(ft, b) + p3] = eps;
+  {
+    const int tot = N1 * W2;
+    double2* dst = (double2*)T;
+    ItDiv d = dn;
+    for (int i = tid; i < tot; i += nt) {
+      const double* a = A + d.ch * RX + 2 * d.j;
+      dst[i] = make_double2(a[0], a[1]);
+      d.next(N1);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+// LDS bytes of the kernels for a box
+constexpr size_t LDS_STATIC = 128;   // the kernels' static LDS (reductions)
+static size_t lds_z(int N3, int L3) { return (size_t)NL * (L3 > 2 * N3 ? L3 : 2 * N3) * 8; }
+size_t fp64_fit_z(const BoxDesc& b, size_t plane_lds) {
+  const size_t v = lds_z(b.N[2], b.L[2]);
+  return v + LDS_STATIC <= plane_lds ? v : 0;
+}
+static size_t fp64_lds_kin(int N1, int N2) {
+  return 8 * ((size_t)(2 * N2 + 1) * (2 * N1 + 1) + map_len(N1) + map_len(N2));
+}
+static size_t fp64_lds_pot(int N1, int N2, int L1, int L2) {
+  const size_t x = (size_t)2 * N2 * (L1 | 1), y = (size_t)L1 * (L2 | 1);
+  size_t maps = 0;
+  if (L1 == 2 * N1) {
+    maps = 8 * (size_t)cmap_len(N2) + 4 * (size_t)smap_len(N2);
+    if (N1 != N2) maps += 8 * (size_t)cmap_len(N1) + 4 * (size_t)smap_len(N1);
+  }
+  return 8 * ((x > y ? x : y) + 2 * PAD) + maps;
+}
+// Launch shapes of the in-plane kernels by items (8 values) of a plane's
+// largest pass and by the work-groups whose LDS fits a CU; work-groups of 4,
+// 8, 12 or 16 waves, as many on each SIMD (work-groups of 7 and 13 waves ran
+// 20 to 40 % slower, and two of 13 do not share a CU).  2 to 4: at least that
+// many work-groups per CU, two items per thread (80 VGPRs: 24 waves per CU);
+// 1: one, three items.
+constexpr int S2_NT = 768, S1_NT = 1024;
+static PlaneFit plane_fit(size_t lds, int items, size_t plane_lds) {
+  plane_lds -= std::min(plane_lds, LDS_STATIC);
+  if (items <= 512 && lds <= plane_lds / 4) return {4, items <= 256 ? 128 : 256, lds};
+  if (items <= 1024 && lds <= plane_lds / 3) return {3, 512, lds};
+  if (items <= 2 * S2_NT && lds <= plane_lds / 2) return {2, items <= 1024 ? 512 : 768, lds};
+  if (items <= 3 * S1_NT && lds <= plane_lds) return {1, items <= 1536 ? 768 : 1024, lds};
+  return {0, 0, lds};
+}
+static int chunks(int n, int len) { return (n + len - 1) / len; }
+PlaneFit fp64_fit_kin(const BoxDesc& b, size_t plane_lds) {
+  const int N1 = b.N[0], N2 = b.N[1];
+  return plane_fit(fp64_lds_kin(N1, N2),
+                   std::max(2 * N1 * chunks(N2, 4), 2 * N2 * chunks(N1, 4)), plane_lds);
+}
+PlaneFit fp64_fit_pot(const BoxDesc& b, size_t plane_lds) {
+  const int N1 = b.N[0], N2 = b.N[1], L1 = b.L[0], L2 = b.L[1];
+  return plane_fit(fp64_lds_pot(N1, N2, L1, L2),
+                   std::max(std::max(2 * N2 * chunks(L1, 8), L1 * chunks(L2, 8)),
+                            std::max(L1 * chunks(N2, 4), 2 * N2 * chunks(N1, 4))),
+                   plane_lds);
+}
+
+static hipError_t launch_zgrow(const Batch& B, const TileTable& t, int ntiles, size_t lds,
+                               hipStream_t s) {
+  if (ntiles > 0) k_zgrow<<<ntiles, ZG_NT, lds, s>>>(B, t);
+  return hipGetLastError();
+}
+static hipError_t launch_zback(const Batch& B, const TileTable& t, const TileTable& ft,
+                               int ntiles, size_t lds, int maxN3, double* part, hipStream_t s) {
+  if (ntiles <= 0) return hipSuccess;
+  if (maxN3 <= 32) k_zback<512, 1, 4><<<ntiles, 512, lds, s>>>(B, t, ft, part);
+  else if (maxN3 <= 48) k_zback<768, 1, 6><<<ntiles, 768, lds, s>>>(B, t, ft, part);
+  else if (maxN3 <= 64) k_zback<512, 2, 4><<<ntiles, 512, lds, s>>>(B, t, ft, part);
+  else k_zback<1024, 3, 4><<<ntiles, 1024, lds, s>>>(B, t, ft, part);
+  return hipGetLastError();
+}
+static hipError_t launch_xykin(const Batch& B, const TileTable& t, int ntiles, size_t lds,
+                               int nt, int shape, hipStream_t s) {
+  if (ntiles <= 0) return hipSuccess;
+  if (shape >= 2) k_xykin<S2_NT, 2, 6><<<ntiles, nt, lds, s>>>(B, t);
+  else k_xykin<S1_NT, 3, 4><<<ntiles, nt, lds, s>>>(B, t);
+  return hipGetLastError();
+}
+static hipError_t launch_xypot(const Batch& B, const TileTable& t, const TileTable& ft,
+                               int ntiles, size_t lds, int nt, int shape, double* part,
+                               hipStream_t s) {
+  if (ntiles <= 0) return hipSuccess;
+  if (shape >= 2) k_xypot<S2_NT, 2, 6><<<ntiles, nt, lds, s>>>(B, t, ft, part);
+  else k_xypot<S1_NT, 3, 4><<<ntiles, nt, lds, s>>>(B, t, ft, part);
+  return hipGetLastError();
+}
+
+// ev: null, or 2 S_COUNT events recorded before / after each stage
+hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
+                           hipEvent_t* ev) {
+  auto mark = [&](int stage, int end) {
+    if (ev) (void)hipEventRecord(ev[2 * stage + end], s);
+  };
+  mark(S_ZG, 0);
+  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], PT.lds_cz, s);
+  mark(S_ZG, 1);
+  // one launch per group of boxes, or one over all of them
+  mark(S_KXY, 0);
+  if (e == hipSuccess && PT.n_pfg == 0)
+    e = launch_xykin(B, PT.t[P_PF], PT.ntiles[P_PF], PT.lds_pfg[0], PT.nthr_pfg[0],
+                     PT.shape_pfg[0], s);
+  for (int k = 0; k < PT.n_pfg && e == hipSuccess; ++k)
+    e = launch_xykin(B, PT.pfg[k], PT.nt_pfg[k], PT.lds_pfg[k], PT.nthr_pfg[k],
+                     PT.shape_pfg[k], s);
+  mark(S_KXY, 1);
+  mark(S_XYP, 0);
+  if (e == hipSuccess && PT.n_pbg == 0)
+    e = launch_xypot(B, PT.t[P_RP], PT.t[P_RP], PT.ntiles[P_RP], PT.lds_pbg[0],
+                     PT.nthr_pbg[0], PT.shape_pbg[0], PT.part[3], s);
+  for (int k = 0; k < PT.n_pbg && e == hipSuccess; ++k)
+    e = launch_xypot(B, PT.pbg[k], PT.t[P_RP], PT.nt_pbg[k], PT.lds_pbg[k], PT.nthr_pbg[k],
+                     PT.shape_pbg[k], PT.part[3], s);
+  mark(S_XYP, 1);
+  mark(S_ZB, 0);
+  if (e == hipSuccess)
+    e = launch_zback(B, PT.t[P_CZ], PT.t[P_CZ], PT.ntiles[P_CZ], PT.lds_cz, PT.maxN3,
+                     PT.part[0], s);
+  mark(S_ZB, 1);
+  if (e != hipSuccess) return e;
+  EnergyTables et;
+  et.t[0] = PT.t[P_CZ];
+  et.p[0] = PT.part[0];
+  et.t[1] = PT.t[P_RP];
+  et.p[1] = PT.part[3];
+  et.nk = 1;
+  et.n = 2;
+  mark(S_ENERGY, 0);
+  launch_energy(et, B, s);
+  mark(S_ENERGY, 1);
+  if (ev)
+    for (int st : {S_ZERO, S_UNC, S_XF, S_YF, S_KY, S_KZ, S_ZP, S_YB, S_XB, S_COMP, S_PF, S_PB}) {
+      mark(st, 0);
+      mark(st, 1);
+    }
+  return hipGetLastError();
+}
+
+// raise the dynamic-LDS limit of the kernels to lds bytes
+void fp64_attributes(size_t lds) {
+  const void* k[] = {(const void*)k_zgrow,         (const void*)k_zback<512, 1, 4>,
+                     (const void*)k_zback<768, 1, 6>,   (const void*)k_zback<512, 2, 4>,
+                     (const void*)k_zback<1024, 3, 4>,
+                     (const void*)k_xykin<S2_NT, 2, 6>, (const void*)k_xypot<S2_NT, 2, 6>,
+                     (const void*)k_xykin<S1_NT, 3, 4>, (const void*)k_xypot<S1_NT, 3, 4>};
+  for (const void* f : k)
+    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
+        hipSuccess)
+      (void)hipGetLastError();
+}
+
+}  // namespace bdft

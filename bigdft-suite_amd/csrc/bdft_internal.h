@@ -47,6 +47,7 @@ struct BoxDesc {
   long long w_off;      // offset of the wavelet volume (8 N1 N2 N3)
   long long t1_off;     // offset of (L1, 2N2, 2N3)
   long long t2_off;     // offset of (L1, L2, 2N3)
+  long long tz_off;     // offset of (2N1, 2N2, L3) (FP64 sequence)
   long long t3_off;     // offset of the real volume (L1, L2, L3): z lines
                         // longer than 192 points only (k_zgrowpot)
   long long pot_off;    // offset into the potential array
@@ -366,6 +367,7 @@ struct Batch {
   void* T1;             // (L1,2N2,2N3) volumes
   void* T2;             // (L1,L2,2N3) volumes
   void* T3;             // (L1,L2,L3) volumes (long z lines only)
+  void* TZ;             // (2N1,2N2,L3) volumes (FP64 sequence)
                         // (element type: double, or float for mixed precision)
   double* part;         // energy partial sums, one slot per (pass, tile)
   double* ekin;         // per-box kinetic energy (device)
@@ -398,15 +400,19 @@ __device__ __forceinline__ float t2_line_unscale(const Batch& B, const BoxDesc& 
 // P_ZP: z lines by rows of x (32 lines of one y per tile); P_ZPF: the same
 // lines as one run x + L1 y, 32 consecutive lines per tile (a tile may span
 // two rows), so that only a box's last tile is partly empty (k_zpot).
+// P_CZ: runs of CCOL coarse columns (z lines of the FP64 sequence); P_RP:
+// real-z planes of its potential pass.
 enum Pass { P_UNC = 0, P_XF, P_YF, P_KY, P_KZ, P_ZP, P_YB, P_XB, P_PF, P_PB, P_KZG, P_ZPG,
-            P_ZPF, P_COUNT };
+            P_ZPF, P_CZ, P_RP, P_COUNT };
+constexpr int CCOL = 16;    // coarse columns (64 z lines) per P_CZ tile
 constexpr int ZGROUP = 3;   // bundles per z-line tile unless LDS asks for 2
 
 struct PassTables {
   TileTable t[P_COUNT];
   int ntiles[P_COUNT];   // total tiles (grid size) of each pass
   double* part[4];       // energy partials: xfwd|plane_fwd, kin_y, kin_z, zpot
-  int plane;             // 1: plane-fused sequence, 0: line passes
+  int plane;             // 1: plane-fused sequence (FP64: bdft_fp64.hip),
+                         // 0: line passes
   size_t lds_pf, lds_pb; // LDS bytes of the plane kernels
   // matrix-core plane kernels: boxes needing more than half a CU's LDS get
   // launches of their own (t[P_PF], t[P_PB] then cover the other boxes)
@@ -418,21 +424,25 @@ struct PassTables {
   TileTable vbg[4];
   int nt_vbg[4];
   int n_vbg;
-  // forward plane pass of the FP64 / FP32 plane-fused sequence: the boxes
-  // in groups by how many of their work-groups fit a CU (LDS and threads),
-  // one launch per group; the kinetic partials keep t[P_PF]'s tile numbers
+  // forward plane pass of the FP32 plane-fused sequence and x-y kinetic pass
+  // of the FP64 one: the boxes in groups by how many of their work-groups
+  // fit a CU (FP32) or by launch shape (FP64), one launch per group; the
+  // partials keep the whole batch's tile numbers
   TileTable pfg[4];
   int nt_pfg[4];
   size_t lds_pfg[4];
+  int shape_pfg[4], nthr_pfg[4];   // FP64: launch shape and threads
   int n_pfg;
-  // backward plane pass of the FP64 / FP32 plane-fused sequence, grouped
-  // the same way; fit_pbg: work-groups per CU of each group (an FP64 group
-  // of two runs the kernel bounded to six waves per SIMD)
+  // backward plane pass of the FP32 plane-fused sequence and potential pass
+  // of the FP64 one, grouped the same way
   TileTable pbg[4];
   int nt_pbg[4];
   size_t lds_pbg[4];
-  int fit_pbg[4];
+  int shape_pbg[4], nthr_pbg[4];
   int n_pbg;
+  // z-line kernels of the FP64 sequence: LDS and longest line of the batch
+  size_t lds_cz;
+  int maxN3, maxL3;
   // preconditioner: x and y operator in one plane pass (FP64 planes that fit)
   int pc_plane;
   size_t lds_pc;
@@ -452,7 +462,7 @@ struct PassTables {
 
 // Launch stages in order; profiling records one event pair per stage.
 enum Stage { S_ZERO = 0, S_UNC, S_XF, S_YF, S_KY, S_KZ, S_ZP, S_YB, S_XB,
-             S_COMP, S_ENERGY, S_PF, S_PB, S_COUNT };
+             S_COMP, S_ENERGY, S_PF, S_PB, S_ZG, S_KXY, S_XYP, S_ZB, S_COUNT };
 
 struct EnergyTables {
   TileTable t[4];       // partial sums of ekin (first nk entries) then epot
@@ -579,6 +589,20 @@ struct Fork {
 hipError_t launch_mfma(const Batch& B, const PassTables& PT, const MfmaLds& L,
                        long long wtotal, bool need_zero, int precision, hipStream_t s,
                        hipEvent_t* ev, const Fork* fk = nullptr);
+// FP64 sequence (bdft_fp64.hip)
+// LDS bytes of the z-line kernels for a box, 0: they do not fit
+size_t fp64_fit_z(const BoxDesc& b, size_t plane_lds);
+// launch shape of an in-plane kernel for a box: shape (1-4, of the boxes that
+// share a launch; 0: the plane does not fit), threads and LDS bytes
+struct PlaneFit {
+  int shape, nt;
+  size_t lds;
+};
+PlaneFit fp64_fit_kin(const BoxDesc& b, size_t plane_lds);
+PlaneFit fp64_fit_pot(const BoxDesc& b, size_t plane_lds);
+void fp64_attributes(size_t lds);
+hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
+                           hipEvent_t* ev);
 size_t plane_lds_fwd(int N1, int N2, int L1, int elem);
 size_t plane_lds_bwd(int N1, int N2, int L1, int L2, int elem);
 // preconditioner: K = c W + K_x W + K_y W per x-y plane (P_PF tiles)
@@ -594,7 +618,7 @@ hipError_t launch_plane_grow(const Batch& B, const TileTable& t, int ntiles, siz
                              hipStream_t s);
 template <typename T>
 hipError_t launch_plane_bwd(const Batch& B, const TileTable& t, int ntiles, size_t lds,
-                            hipStream_t s, bool occ2 = false);
+                            hipStream_t s);
 hipError_t launch_transfer(const Batch& B, const TileTable& t, int ntiles,
                            long long wtotal, bool compress, hipStream_t s);
 // ev: null, or 2*S_COUNT events recorded before/after each stage;

@@ -1537,7 +1537,7 @@ static hipError_t launch_mfma_t(const Batch& B, const PassTables& PT, const Mfma
   launch_energy(et, B, s);
   mark(S_ENERGY, 1);
   if (ev) {
-    const int unused[] = {S_YF, S_YB, S_XB, S_COMP};
+    const int unused[] = {S_YF, S_YB, S_XB, S_COMP, S_ZG, S_KXY, S_XYP, S_ZB};
     for (int st : unused) {
       mark(st, 0);
       mark(st, 1);

@@ -1247,7 +1247,7 @@ hipError_t launch_density(const Batch& B, const PassTables& T, const DenArgs& D,
 }
 
 // ---------------------------------------------------------------------------
-// host-side launcher of the whole FP64 sequence
+// host-side launcher: the FP32 plane-fused sequence and the line passes
 // ---------------------------------------------------------------------------
 size_t lds_bytes(int maxN, int elem) {
   return (size_t)2 * (maxN + HL + HR) * LDW * elem;
@@ -1282,6 +1282,13 @@ static hipError_t launch_seq(const Batch& B, const PassTables& PT, int maxN,
   auto mark = [&](int stage, int end) {
     if (ev) (void)hipEventRecord(ev[2 * stage + end], s);
   };
+  // stages of the other sequences: empty event pairs
+  auto unused = [&](std::initializer_list<int> st) {
+    for (int x : st) {
+      mark(x, 0);
+      mark(x, 1);
+    }
+  };
   mark(S_ZERO, 0);
   if (need_zero) {
     const long long nb = (wtotal + NT - 1) / NT;
@@ -1294,7 +1301,10 @@ static hipError_t launch_seq(const Batch& B, const PassTables& PT, int maxN,
   mark(S, 1);
   BDFT_STAGE(S_UNC, P_UNC, 0, (k_uncompress<T, false>), B, PT.t[P_UNC])
   EnergyTables et;
-  if (PT.plane) {
+  bool fused = false;
+  if constexpr (sizeof(T) == 4) fused = PT.plane != 0;
+  if (fused) {
+    if constexpr (sizeof(T) == 4) {
     mark(S_PF, 0);
     if (PT.n_pfg > 0) {
       for (int k = 0; k < PT.n_pfg; ++k)
@@ -1314,8 +1324,7 @@ static hipError_t launch_seq(const Batch& B, const PassTables& PT, int maxN,
     if (PT.n_pbg > 0) {
       for (int k = 0; k < PT.n_pbg; ++k)
         if (PT.nt_pbg[k] > 0)
-          launch_plane_bwd<T>(B, PT.pbg[k], PT.nt_pbg[k], PT.lds_pbg[k], s,
-                              sizeof(T) == 8 && PT.fit_pbg[k] == 2);
+          launch_plane_bwd<T>(B, PT.pbg[k], PT.nt_pbg[k], PT.lds_pbg[k], s);
     } else if (PT.ntiles[P_PB] > 0) {
       launch_plane_bwd<T>(B, PT.t[P_PB], PT.ntiles[P_PB], PT.lds_pb, s);
     }
@@ -1328,6 +1337,7 @@ static hipError_t launch_seq(const Batch& B, const PassTables& PT, int maxN,
     et.p[2] = PT.part[3];
     et.nk = 2;
     et.n = 3;
+    }
   } else {
     if (PT.xbig) {
       BDFT_STAGE(S_XF, P_XF, lds, (k_xfwd<T, true>), B, PT.t[P_XF], PT.part[0])
@@ -1359,21 +1369,19 @@ static hipError_t launch_seq(const Batch& B, const PassTables& PT, int maxN,
   mark(S_ENERGY, 0);
   k_energy<<<B.nbox, 128, 0, s>>>(et, B.nbox, B.ekin, B.epot);
   mark(S_ENERGY, 1);
-  if (ev) {  // stages of the other sequence: empty event pairs
-    const int unused_plane[] = {S_XF, S_YF, S_KY, S_YB, S_XB, S_COMP};
-    const int unused_lines[] = {S_PF, S_PB};
-    if (PT.plane)
-      for (int st : unused_plane) { mark(st, 0); mark(st, 1); }
-    else
-      for (int st : unused_lines) { mark(st, 0); mark(st, 1); }
+  if (ev) {
+    if (fused) unused({S_XF, S_YF, S_KY, S_YB, S_XB, S_COMP});
+    else unused({S_PF, S_PB});
+    unused({S_ZG, S_KXY, S_XYP, S_ZB});
   }
   return hipGetLastError();
 }
 
 hipError_t launch_passes(const Batch& B, const PassTables& T, int maxN, long long wtotal,
                          bool need_zero, int fp32, hipStream_t s, hipEvent_t* ev) {
-  return fp32 ? launch_seq<float>(B, T, maxN, wtotal, need_zero, s, ev)
-              : launch_seq<double>(B, T, maxN, wtotal, need_zero, s, ev);
+  if (fp32) return launch_seq<float>(B, T, maxN, wtotal, need_zero, s, ev);
+  if (T.plane) return launch_fp64_seq(B, T, s, ev);
+  return launch_seq<double>(B, T, maxN, wtotal, need_zero, s, ev);
 }
 
 hipError_t launch_transfer(const Batch& B, const TileTable& t, int ntiles,

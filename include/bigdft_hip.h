@@ -350,14 +350,16 @@ int bdft_ctx_info(const bdft_ctx *ctx, int64_t *lds_per_block,
  *                         allocation-free calls are not chunked)
  *   BDFT_OPT_TILE_ORDER   0: the plane and (un)compress passes take their
  *                         tiles in dispatch order (default); 1: in one
- *                         contiguous range per XCD, as the z-line and line
- *                         passes always do (work-groups are dealt to the 8
- *                         XCDs in turn, each with its own L2)
+ *                         contiguous range per XCD, as the z-line, line and
+ *                         FP64 x-y kinetic passes always do (work-groups are
+ *                         dealt to the 8 XCDs in turn, each with its own L2)
  *   BDFT_OPT_PERSIST      0: the z potential pass launches one work-group
  *                         per tile (default); 1: a persistent launch of
  *                         resident work-groups over a work queue of the
  *                         tiles, boxes in order of decreasing size (each
- *                         work-group ends at the end of its stretch)
+ *                         work-group ends at the end of its stretch); the
+ *                         FP64 plane-fused sequence applies the potential
+ *                         in its x-y planes and has no such pass
  * A change drops the context's cached plans; plans already created by
  * bdft_plan_create keep the options they were made with. */
 #define BDFT_OPT_LINE_PASSES 1

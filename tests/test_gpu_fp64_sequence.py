@@ -1,0 +1,80 @@
+"""The FP64 plane-fused sequence (bdft_fp64.hip) against the oracle at the
+edges of its launch rules: extents where an in-plane work-group changes its
+shape (8, 12 or 16 waves, one or more per CU) or the planes stop fitting and
+the batch takes the line passes, z lines where the z kernels change their
+chunks per wave or stop fitting, and coarse planes that leave a partly empty
+last run of 16 columns.
+
+FP64 sums of at most 2 x 31 (G, G^T) and 58 (kinetic) products per axis, in
+another order than the oracle's: 1e-12 per element (guarded relative) and in
+the energies, the bar of every FP64 parity test.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import dense_region, okeys, random_pot, random_psi, region_from_grids, rel_err
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import bigdft_hip
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    c = bigdft_hip.Context(0)
+    yield c
+    c.close()
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+# n (coarse points - 1) per axis
+SIZES = [("P", n) for n in [
+    (0, 0, 0), (15, 0, 4), (4, 3, 1), (7, 15, 2), (16, 16, 1),   # column runs, 4 waves
+    (22, 22, 1), (31, 31, 0), (38, 41, 1),                       # 8 waves
+    (48, 48, 1), (49, 49, 1), (54, 55, 0),                       # half a CU's LDS, 12 waves
+    (63, 63, 0), (69, 69, 0), (70, 70, 0), (84, 40, 0),          # 16 waves, beyond
+    (1, 2, 31), (2, 1, 32), (1, 2, 47), (2, 1, 48), (1, 2, 63), (2, 1, 64),
+    (1, 0, 158), (0, 1, 159)]] + [("F", n) for n in [
+    (0, 0, 0), (4, 3, 1), (15, 16, 1), (20, 21, 0), (25, 26, 1),
+    (35, 35, 0), (36, 36, 0), (40, 30, 1), (55, 55, 0), (56, 57, 0),
+    (1, 2, 31), (2, 1, 32), (1, 2, 48), (2, 1, 64), (1, 0, 144), (0, 1, 146)]]
+
+
+@pytest.mark.parametrize("geo,n", SIZES, ids=[f"{g}{n[0]}x{n[1]}x{n[2]}" for g, n in SIZES])
+@pytest.mark.parametrize("keys", ["dense", "sparse"])
+def test_launch_edges_match_the_oracle(ctx, geo, n, keys):
+    reg = dense_region(geo, n, (0.45, 0.4, 0.5))
+    if keys == "sparse":   # half the coarse points, a quarter of them fine
+        rng = np.random.default_rng(sum(n) + 5)
+        lg = rng.random(tuple(x + 1 for x in n)) < 0.5
+        lg[0, 0, 0] = True
+        fine = lg & (rng.random(lg.shape) < 0.5)
+        fine[0, 0, 0] = True
+        reg = region_from_grids(geo, n, (0.45, 0.4, 0.5), lg, fine)
+    print(f"case {geo} n={n} {keys} nvctr=({reg.nvctr_c},{reg.nvctr_f})", flush=True)
+    norb = 2
+    psi, h0 = random_psi(reg, norb, 31), random_psi(reg, norb, 32)
+    pot = random_pot(reg, 33)
+    lr = ctx.region(reg)
+    d_h = dev(h0)
+    ek = torch.zeros(norb, dtype=torch.float64, device="cuda")
+    ep = torch.zeros_like(ek)
+    ctx.locham(lr, dev(pot), dev(psi), d_h, ek, ep)
+    ctx.sync()
+    lr.close()
+    ho, eo, po = oracle.locham(geo, reg.n, reg.nfl, reg.nfu, reg.hgrid, okeys(reg), pot, psi, h0)
+    # element by element against the sums' own scale: an isolated point's
+    # value may cancel to far below the terms it is made of
+    h = d_h.cpu().numpy()
+    assert np.abs(h - ho).max() < TOL * np.abs(ho - h0).max()
+    if keys == "dense":
+        assert rel_err(h - h0, ho - h0) < TOL
+    assert rel_err(ek.cpu().numpy(), eo) < TOL
+    assert rel_err(ep.cpu().numpy(), po) < TOL
