@@ -1058,16 +1058,17 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     }
   }
   {
-    // density plans (grow_plane) use the forward plane kernel without its
-    // kinetic part; the preconditioner's plans keep the line passes
+    // density plans (grow_plane) use the first half of the sequence (FP32:
+    // the forward plane kernel without its kinetic part); the
+    // preconditioner's plans keep the line passes
     bool plane = !ctx->force_lines && !mfma && (!density || grow_plane);
-    const bool d64 = esz == 8 && !density;   // the FP64 sequence (bdft_fp64.hip)
+    const bool d64 = esz == 8;   // the FP64 sequence (bdft_fp64.hip)
     size_t lpf = 0, lpb = 0, lcz = 0;
     bool fits = true;
     for (int i = 0; i < norb && plane; ++i) {
       const BoxDesc& b = box[i];
       if (d64) {
-        fits = fits && fp64_fit_kin(b, ctx->plane_lds).shape &&
+        fits = fits && (density || fp64_fit_kin(b, ctx->plane_lds).shape) &&
                fp64_fit_pot(b, ctx->plane_lds).shape;
         const size_t z = fp64_fit_z(b, ctx->plane_lds);
         fits = fits && z;
@@ -1133,8 +1134,9 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     };
     T.n_pfg = T.n_pbg = 0;
     if (T.plane && d64) {
-      group(P_PF, [&](const BoxDesc& b) { return fp64_fit_kin(b, ctx->plane_lds); }, T.pfg,
-            T.nt_pfg, T.lds_pfg, T.shape_pfg, T.nthr_pfg, T.n_pfg, pf_off);
+      if (!density)
+        group(P_PF, [&](const BoxDesc& b) { return fp64_fit_kin(b, ctx->plane_lds); }, T.pfg,
+              T.nt_pfg, T.lds_pfg, T.shape_pfg, T.nthr_pfg, T.n_pfg, pf_off);
       group(P_RP, [&](const BoxDesc& b) { return fp64_fit_pot(b, ctx->plane_lds); }, T.pbg,
             T.nt_pbg, T.lds_pbg, T.shape_pbg, T.nthr_pbg, T.n_pbg, pb_off);
       for (int k = 0; k < std::max(1, T.n_pbg) && force; ++k)
@@ -1253,7 +1255,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   }
   const size_t nb_st = sizeof(int) * starts.size();
   int epass[4] = {P_XF, P_KY, P_KZ, P_ZP};
-  const bool fp64_seq = T.plane && esz == 8 && !density;
+  const bool fp64_seq = T.plane && esz == 8;
   if (fp64_seq) {
     epass[0] = P_CZ;
     epass[3] = P_RP;
@@ -1361,15 +1363,16 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   // workspace: W | K | T1 | T2 | T3
   if (T.plane || mfma) t1tot = 0;
   if (!zbig) t3tot = 0;
-  // (FP64 sequence: K | TZ)
-  long long wv = wtot;
+  // (FP64 sequence: K | TZ, density: TZ)
+  long long wv = wtot, kv = wtot;
   if (fp64_seq) wv = t2tot = t3tot = 0;
   else tztot = 0;
+  if (fp64_seq && density) kv = 0;
   T.xbig = xbig;
   T.zbig = zbig;
   T.zshort = maxL3 <= ZSHORT_L;
   {
-    const long long part[6] = {wv, wtot, t1tot, t2tot, t3tot, tztot};
+    const long long part[6] = {wv, kv, t1tot, t2tot, t3tot, tztot};
     size_t at = 0;
     for (int k = 0; k < 6; ++k) {
       plan->ws_at[k] = at;
@@ -1827,28 +1830,66 @@ extern "C" int bdft_density_d(bdft_ctx* ctx, const bdft_lr* lr, int norb, const 
   D.nisf = (long long)lr->L[0] * lr->L[1] * lr->L[2];
   D.norb = norb;
   D.nspin = nspin;
-  D.nxt = cdiv(lr->L[0], TW);
-  D.nbund = D.nxt * lr->L[1];
-  const int want = std::max(1, std::min(std::min(norb, 64), cdiv(4096, D.nbund)));
-  D.gsize = cdiv(norb, want);
-  D.ngroups = cdiv(norb, D.gsize);
+  // per orbital: hfac and its spin (or its number, FP64 planes); groups of
+  // orbitals whose partial densities are written and summed
+  std::vector<double> hf(hfac, hfac + norb);
+  std::vector<int32_t> meta(sp);
+  size_t nparts;
+  const bool planes = plan->T.plane && precision == BDFT_PREC_FP64;
+  if (planes) {
+    // the orbitals by spin, in groups of one spin: 1536 planes or so of
+    // work-groups (six per CU; more groups would only write more partials)
+    meta.clear();
+    for (int s = 0; s < nspin; ++s)
+      for (int i = 0; i < norb; ++i)
+        if (sp[i] == s) meta.push_back(i);
+    for (int k = 0; k < norb; ++k) hf[k] = hfac[meta[k]];
+    const int n0 = (int)std::count(sp.begin(), sp.end(), 0);
+    const int want = std::max(1, std::min(norb, cdiv(1536, lr->L[2])));
+    D.gsize = cdiv(norb, want);
+    std::vector<int32_t> start;
+    for (int k = 0; k < n0; k += D.gsize) start.push_back(k);
+    D.gspin = (int)start.size();
+    for (int k = n0; k < norb; k += D.gsize) start.push_back(k);
+    D.ngroups = (int)start.size();
+    start.push_back(norb);
+    meta.insert(meta.end(), start.begin(), start.end());
+    nparts = (size_t)D.ngroups;
+  } else {
+    D.nxt = cdiv(lr->L[0], TW);
+    D.nbund = D.nxt * lr->L[1];
+    const int want = std::max(1, std::min(std::min(norb, 64), cdiv(4096, D.nbund)));
+    D.gsize = cdiv(norb, want);
+    D.ngroups = cdiv(norb, D.gsize);
+    nparts = (size_t)D.ngroups * nspin;
+  }
   auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-  const size_t nb_h = sizeof(double) * norb, nb_s = sizeof(int32_t) * norb;
-  const size_t nb_p = sizeof(double) * (size_t)D.ngroups * nspin * (size_t)D.nisf;
+  const size_t nb_h = sizeof(double) * norb, nb_s = sizeof(int32_t) * meta.size();
+  const size_t nb_p = sizeof(double) * nparts * (size_t)D.nisf;
   DevBuf& buf = ctx->den_buf;
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));  // the buffer may be reallocated
   int rc = dev_alloc(ctx, buf, al(nb_h) + al(nb_s) + al(nb_p));
   if (rc) return rc;
   char* q = (char*)buf.p;
-  hipError_t e = hipMemcpy(q, hfac, nb_h, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(q + al(nb_h), sp.data(), nb_s, hipMemcpyHostToDevice);
+  // one copy
+  std::vector<unsigned char> up(al(nb_h) + nb_s);
+  memcpy(up.data(), hf.data(), nb_h);
+  memcpy(up.data() + al(nb_h), meta.data(), nb_s);
+  hipError_t e = hipMemcpy(q, up.data(), up.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) {
     D.hfac = (const double*)q;
-    D.spin = (const int*)(q + al(nb_h));
     D.part = (double*)(q + al(nb_h) + al(nb_s));
     D.rho = rho;
-    e = launch_density(plan->B, plan->T, D, plan->maxN, plan->wtotal, plan->need_zero,
-                       precision == BDFT_PREC_FP32, ctx->stream);
+    const int* m = (const int*)(q + al(nb_h));
+    if (planes) {
+      D.order = m;
+      D.gstart = m + norb;
+      e = launch_fp64_density(plan->B, plan->T, D, lr->L[2], ctx->stream);
+    } else {
+      D.spin = m;
+      e = launch_density(plan->B, plan->T, D, plan->maxN, plan->wtotal, plan->need_zero,
+                         precision == BDFT_PREC_FP32, ctx->stream);
+    }
   }
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess)

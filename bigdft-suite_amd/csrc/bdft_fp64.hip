@@ -343,7 +343,7 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
 // next to the row, PAD values around the plane keep that inside the
 // allocation) and cost nothing where the whole wave is past the line.
 // ---------------------------------------------------------------------------
-constexpr int PAD = 24;   // rows are read at most 15 values before and 20 past their end
+constexpr int PAD = 16, PADE = 8;   // rows are read at most 15 values before, 5 past their end
 
 // NK taps from value k0 of a line of n values: load(kk) reads tap kk's
 // input(s) from the row, mapped(kk) through the line map, apply(kk, x) adds
@@ -564,40 +564,43 @@ __global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt) {
 }
 
 // ---------------------------------------------------------------------------
-// TZ <- G_x^T G_y^T V G_y G_x TZ of the plane at fine z point p3, epot
-// partial.  LDS: x lines as rows (stride RX) for G_x and G_x^T, y lines as
-// rows (RY) in between.
+// A plane of TZ (2 N1 x 2 N2) in LDS: x lines as rows (stride RX) for G_x and
+// G_x^T, y lines as rows (RY) in between.
 // ---------------------------------------------------------------------------
-template <int NTM, int MI, int WPE>
-__global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileTable ft,
-                                                    double* part) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ double red[NTM / 64];
-  const int tile = tile_of(tt);
-  const int lb = find_box(tt, tile);
-  const int b = table_box(tt, lb);
-  const BoxDesc bd = B.box[b];
-  const int p3 = tile - box_first_tile(tt, lb);
-  const int N1 = bd.N[0], N2 = bd.N[1], L1 = bd.L[0], L2 = bd.L[1], per = bd.per;
-  const int W1 = 2 * N1, W2 = 2 * N2, RX = L1 | 1, RY = L2 | 1;
-  double* A = (double*)smem + PAD;
-  // line maps, one pair for both axes of a square plane
-  const bool sq = N1 == N2;
-  int2* mx = (int2*)(A + max(W2 * RX, L1 * RY) + PAD);
-  int2* my = mx + (sq ? 0 : cmap_len(N1));
-  int* sx = (int*)(my + cmap_len(N2));
-  int* sy = sx + (sq ? 0 : smap_len(N1));
-  const int tid = threadIdx.x, nt = blockDim.x;
-  double* T = (double*)B.TZ + bd.tz_off + (long long)W1 * W2 * p3;
-  // the plane, two values at a time (rows of 2 N1, planes of 4 N1 N2 values:
-  // 16-byte aligned)
-  const ItDiv dn(tid, N1, nt);
-  {
+struct Plane {
+  int N1, N2, L1, L2, per, W1, W2, RX, RY;
+  double* A;
+  int2 *mx, *my;   // line maps, one pair for both axes of a square plane
+  int *sx, *sy;
+  ItDiv dn, dw, dl;   // first pair of values, first x and y items
+  __device__ __forceinline__ Plane(const BoxDesc& bd, unsigned char* smem)
+      : N1(bd.N[0]), N2(bd.N[1]), L1(bd.L[0]), L2(bd.L[1]), per(bd.per), W1(2 * N1),
+        W2(2 * N2), RX(L1 | 1), RY(L2 | 1), A((double*)smem + PAD),
+        dn(threadIdx.x, N1, blockDim.x), dw(threadIdx.x, W2, blockDim.x),
+        dl(threadIdx.x, L1, blockDim.x) {
+    const bool sq = N1 == N2;
+    mx = (int2*)(A + max(W2 * RX, L1 * RY) + PADE);
+    my = mx + (sq ? 0 : cmap_len(N1));
+    sx = (int*)(my + cmap_len(N2));
+    sy = sx + (sq ? 0 : smap_len(N1));
+    if (per) {
+      build_maps(mx, sx, N1, threadIdx.x, blockDim.x);
+      if (!sq) build_maps(my, sy, N2, threadIdx.x, blockDim.x);
+    }
+  }
+  // the thread's items, opaque: in a loop over planes, addresses and line-end
+  // masks made from them stay inside it (moved out, they spill)
+  __device__ __forceinline__ void opaque() {
+    asm volatile("" : "+v"(dn.ch), "+v"(dn.j), "+v"(dw.ch), "+v"(dw.j), "+v"(dl.ch), "+v"(dl.j));
+  }
+  // T's plane into the x rows, two values at a time (rows of 2 N1, planes of
+  // 4 N1 N2 values: 16-byte aligned)
+  __device__ __forceinline__ void load(const double* T) const {
     constexpr int UR = 4;
-    const int tot = N1 * W2;
+    const int tot = N1 * W2, nt = blockDim.x;
     const double2* src = (const double2*)T;
     ItDiv d = dn;
-    for (int i = tid; i < tot; i += nt * UR) {
+    for (int i = threadIdx.x; i < tot; i += nt * UR) {
       double2 v[UR];
 #pragma unroll
       for (int u = 0; u < UR; ++u) v[u] = src[min(i + u * nt, tot - 1)];
@@ -612,26 +615,53 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
       }
     }
   }
-  if (per) {
-    build_maps(mx, sx, N1, tid, nt);
-    if (!sq) build_maps(my, sy, N2, tid, nt);
-  }
-  __syncthreads();
-  double o[MI][8];
-  const ItDiv dw(tid, W2, nt), dl(tid, L1, nt);
-  // G_x on the rows j2, written as columns of the y rows
-  const int gx = (L1 + 7) >> 3, gy = (L2 + 7) >> 3;
-  each_item<MI>(dw, W2, gx, [&](int m, int ch, int j2) {
-    grow_row(A + j2 * RX, mx, N1, grow_k0(8 * ch, per), per, o[m]);
-  });
-  __syncthreads();
-  each_item<MI>(dw, W2, gx, [&](int m, int ch, int j2) {
-    double* a = A + 8 * ch * RY + j2;
+  // G_x on the rows j2, written as columns of the y rows (barriers: the plane
+  // is loaded before, the y rows are complete after)
+  template <int MI>
+  __device__ __forceinline__ void grow_x(double o[MI][8]) const {
+    const int gx = (L1 + 7) >> 3;
+    __syncthreads();
+    each_item<MI>(dw, W2, gx, [&](int m, int ch, int j2) {
+      grow_row(A + j2 * RX, mx, N1, grow_k0(8 * ch, per), per, o[m]);
+    });
+    __syncthreads();
+    each_item<MI>(dw, W2, gx, [&](int m, int ch, int j2) {
+      double* a = A + 8 * ch * RY + j2;
 #pragma unroll
-    for (int r = 0; r < 8; ++r)
-      if (8 * ch + r < L1) a[r * RY] = o[m][r];
-  });
-  __syncthreads();
+      for (int r = 0; r < 8; ++r)
+        if (8 * ch + r < L1) a[r * RY] = o[m][r];
+    });
+    __syncthreads();
+  }
+  __device__ __forceinline__ void grow_y(int ch, int p1, double o[8]) const {
+    grow_row(A + p1 * RY, my, N2, grow_k0(8 * ch, per), per, o);
+  }
+};
+
+// ---------------------------------------------------------------------------
+// TZ <- G_x^T G_y^T V G_y G_x TZ of the plane at fine z point p3, epot
+// partial
+// ---------------------------------------------------------------------------
+template <int NTM, int MI, int WPE>
+__global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileTable ft,
+                                                    double* part) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ double red[NTM / 64];
+  const int tile = tile_of(tt);
+  const int lb = find_box(tt, tile);
+  const int b = table_box(tt, lb);
+  const BoxDesc bd = B.box[b];
+  const int p3 = tile - box_first_tile(tt, lb);
+  const Plane P(bd, smem);
+  const int N1 = P.N1, N2 = P.N2, L1 = P.L1, L2 = P.L2, per = P.per;
+  const int W2 = P.W2, RX = P.RX, RY = P.RY;
+  double* A = P.A;
+  double* T = (double*)B.TZ + bd.tz_off + (long long)P.W1 * W2 * p3;
+  P.load(T);
+  double o[MI][8];
+  P.grow_x<MI>(o);
+  const ItDiv dw = P.dw, dl = P.dl;
+  const int gy = (L2 + 7) >> 3;
   // G_y and V on the rows p1.  V outside the potential box is zero, the
   // zeroing of psir there (potential.f90:874-947); those points read a value
   // of the box and discard it, so all loads of a chunk are in flight together
@@ -662,7 +692,7 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
       for (int r = 0; r < 8; ++r)
         v[r] = pot[v0 + pd1 * (unsigned)min(max(q20 + r, 0), bd.potdim[1] - 1)];
     }
-    grow_row(A + p1 * RY, my, N2, grow_k0(8 * ch, per), per, o[m]);
+    P.grow_y(ch, p1, o[m]);
     if (bd.conf_on || !whole) {
 #pragma unroll
       for (int r = 0; r < 8; ++r) {
@@ -690,7 +720,7 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
   // G_y^T on the rows p1, written as columns of the x rows
   const int cy = (N2 + 3) >> 2, cx = (N1 + 3) >> 2;
   each_item<MI>(dl, L1, cy, [&](int m, int ch, int p1) {
-    shrink_row(A + p1 * RY, sy, L2, 4 * ch, per, o[m]);
+    shrink_row(A + p1 * RY, P.sy, L2, 4 * ch, per, o[m]);
   });
   __syncthreads();
   each_item<MI>(dl, L1, cy, [&](int m, int ch, int p1) {
@@ -705,7 +735,7 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
   __syncthreads();
   // G_x^T on the rows j2
   each_item<MI>(dw, W2, cx, [&](int m, int ch, int j2) {
-    shrink_row(A + j2 * RX, sx, L1, 4 * ch, per, o[m]);
+    shrink_row(A + j2 * RX, P.sx, L1, 4 * ch, per, o[m]);
   });
   __syncthreads();
   each_item<MI>(dw, W2, cx, [&](int m, int ch, int j2) {
@@ -718,17 +748,74 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
       }
   });
   const double eps = block_sum_rt(ep, red);   // has the barriers
-  if (tid == 0) part[box_first_tile(ft, b) + p3] = eps;
+  if (threadIdx.x == 0) part[box_first_tile(ft, b) + p3] = eps;
   {
     const int tot = N1 * W2;
     double2* dst = (double2*)T;
-    ItDiv d = dn;
-    for (int i = tid; i < tot; i += nt) {
+    ItDiv d = P.dn;
+    for (int i = threadIdx.x; i < tot; i += (int)blockDim.x) {
       const double* a = A + d.ch * RX + 2 * d.j;
       dst[i] = make_double2(a[0], a[1]);
       d.next(N1);
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// density (local_partial_density, sumrho.f90:377-469): the planes p3 of TZ of
+// one group's orbitals (orbitals order[0 ..] of one spin, one box) in turn,
+// psir = G_y G_x, and sum hfac psir^2 kept in registers, written once as the
+// group's partial density.  Three items per thread (128 VGPRs) on 8 waves, two
+// work-groups per CU: with the sums beside the passes' outputs, two items at
+// 80 VGPRs spill (0.42 against 0.49 ms for 96 orbitals of a periodic 48^3
+// box).  That batch, 8.5e7 points: unpack 0.23, x-y planes 0.51, z lines 0.43
+// ms before, k_zgrow 0.27 and k_xyden 0.42 now (24 bytes per point for 40).
+// ---------------------------------------------------------------------------
+template <int NTM, int MI, int WPE>
+__global__ __launch_bounds__(NTM, WPE) void k_xyden(Batch B, DenArgs D) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const BoxDesc bd = B.box[0];
+  const int L3 = bd.L[2];
+  const int g = blockIdx.x / L3, p3 = blockIdx.x - g * L3;
+  Plane P(bd, smem);
+  const long long plane = (long long)P.W1 * P.W2;
+  const int gy = (P.L2 + 7) >> 3;
+  double acc[MI][8];
+#pragma unroll
+  for (int m = 0; m < MI; ++m)
+#pragma unroll
+    for (int r = 0; r < 8; ++r) acc[m][r] = 0.0;
+  const int o1 = D.gstart[g + 1];
+  for (int k = D.gstart[g]; k < o1; ++k) {
+    const double hf = D.hfac[k];
+    P.opaque();
+    P.load((const double*)B.TZ + B.box[D.order[k]].tz_off + plane * p3);
+    double o[MI][8];
+    P.grow_x<MI>(o);
+    each_item<MI>(P.dl, P.L1, gy, [&](int m, int ch, int p1) {
+      double v[8];
+      P.grow_y(ch, p1, v);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) acc[m][r] += hf * (v[r] * v[r]);
+    });
+    __syncthreads();
+  }
+  double* dst = D.part + (long long)g * D.nisf + (long long)P.L1 * P.L2 * p3;
+  each_item<MI>(P.dl, P.L1, gy, [&](int m, int ch, int p1) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      if (8 * ch + r < P.L2) dst[p1 + P.L1 * (8 * ch + r)] = acc[m][r];
+  });
+}
+
+// rho += sum of the group partials of a spin, groups in order
+__global__ __launch_bounds__(256) void k_xyden_sum(DenArgs D) {
+  const long long i = blockIdx.x * 256LL + threadIdx.x;
+  if (i >= D.nisf) return;
+  const int s = blockIdx.y;
+  double a = 0.0;
+  for (int g = s ? D.gspin : 0; g < (s ? D.ngroups : D.gspin); ++g) a += D.part[g * D.nisf + i];
+  D.rho[s * D.nisf + i] += a;
 }
 
 // ---------------------------------------------------------------------------
@@ -751,7 +838,7 @@ static size_t fp64_lds_pot(int N1, int N2, int L1, int L2) {
     maps = 8 * (size_t)cmap_len(N2) + 4 * (size_t)smap_len(N2);
     if (N1 != N2) maps += 8 * (size_t)cmap_len(N1) + 4 * (size_t)smap_len(N1);
   }
-  return 8 * ((x > y ? x : y) + 2 * PAD) + maps;
+  return 8 * ((x > y ? x : y) + PAD + PADE) + maps;
 }
 // Launch shapes of the in-plane kernels by items (8 values) of a plane's
 // largest pass and by the work-groups whose LDS fits a CU; work-groups of 4,
@@ -862,11 +949,26 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
   return hipGetLastError();
 }
 
+hipError_t launch_fp64_density(const Batch& B, const PassTables& PT, const DenArgs& D, int L3,
+                               hipStream_t s) {
+  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], PT.lds_cz, s);
+  if (e != hipSuccess) return e;
+  const int n = D.ngroups * L3;
+  const size_t lds = PT.lds_pbg[0];
+  if (PT.shape_pbg[0] >= 2)
+    k_xyden<512, 3, 4><<<n, std::min(512, PT.nthr_pbg[0]), lds, s>>>(B, D);
+  else
+    k_xyden<S1_NT, 3, 4><<<n, PT.nthr_pbg[0], lds, s>>>(B, D);
+  k_xyden_sum<<<dim3((unsigned)((D.nisf + 255) / 256), D.nspin), 256, 0, s>>>(D);
+  return hipGetLastError();
+}
+
 // raise the dynamic-LDS limit of the kernels to lds bytes
 void fp64_attributes(size_t lds) {
   const void* k[] = {(const void*)k_zgrow,         (const void*)k_zback<512, 1, 4>,
                      (const void*)k_zback<768, 1, 6>,   (const void*)k_zback<512, 2, 4>,
                      (const void*)k_zback<1024, 3, 4>,
+                     (const void*)k_xyden<512, 3, 4>, (const void*)k_xyden<S1_NT, 3, 4>,
                      (const void*)k_xykin<S2_NT, 2, 6>, (const void*)k_xypot<S2_NT, 2, 6>,
                      (const void*)k_xykin<S1_NT, 3, 4>, (const void*)k_xypot<S1_NT, 3, 4>};
   for (const void* f : k)

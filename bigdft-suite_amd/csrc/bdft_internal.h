@@ -493,6 +493,13 @@ struct DenArgs {
   double* rho;          // nspin x nisf, accumulated
   long long nisf;
   int norb, nspin, ngroups, gsize, nbund, nxt;
+  // FP64 planes (k_xyden): the orbitals with those of spin 0 first (order;
+  // hfac in that order), group g = order[gstart[g]] .. order[gstart[g + 1] -
+  // 1], all of one spin: groups below gspin of spin 0.  part holds one box
+  // per group.
+  const int* order;
+  const int* gstart;
+  int gspin;
 };
 
 // region transfers: one descriptor per local region, tiles of 256 points
@@ -601,6 +608,8 @@ struct PlaneFit {
 PlaneFit fp64_fit_kin(const BoxDesc& b, size_t plane_lds);
 PlaneFit fp64_fit_pot(const BoxDesc& b, size_t plane_lds);
 void fp64_attributes(size_t lds);
+hipError_t launch_fp64_density(const Batch& B, const PassTables& PT, const DenArgs& D, int L3,
+                               hipStream_t s);
 hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
                            hipEvent_t* ev);
 size_t plane_lds_fwd(int N1, int N2, int L1, int elem);
@@ -613,7 +622,6 @@ size_t plane_attributes();
 template <typename T>
 hipError_t launch_plane_fwd(const Batch& B, const TileTable& t, const TileTable& ft,
                             int ntiles, size_t lds, double* part, hipStream_t s);
-template <typename T>
 hipError_t launch_plane_grow(const Batch& B, const TileTable& t, int ntiles, size_t lds,
                              hipStream_t s);
 template <typename T>

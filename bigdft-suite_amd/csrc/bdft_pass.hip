@@ -1201,13 +1201,16 @@ static hipError_t launch_den(const Batch& B, const PassTables& PT, const DenArgs
     k_zero<T><<<(unsigned)(nb < 65536 ? nb : 65536), NT, 0, s>>>((T*)B.W, wtotal);
   }
   if (PT.ntiles[P_UNC] > 0) k_uncompress<T, false><<<PT.ntiles[P_UNC], NT, 0, s>>>(B, PT.t[P_UNC]);
-  if (PT.plane) {
+  bool fused = false;
+  if constexpr (sizeof(T) == 4) {
     // x and y grow of each plane in one pass through LDS
-    if (PT.ntiles[P_PF] > 0) {
-      const hipError_t e = launch_plane_grow<T>(B, PT.t[P_PF], PT.ntiles[P_PF], PT.lds_pf, s);
+    fused = PT.plane != 0;
+    if (fused && PT.ntiles[P_PF] > 0) {
+      const hipError_t e = launch_plane_grow(B, PT.t[P_PF], PT.ntiles[P_PF], PT.lds_pf, s);
       if (e != hipSuccess) return e;
     }
-  } else {
+  }
+  if (!fused) {
     if (PT.ntiles[P_XF] > 0) {
       if (PT.xbig) k_xfwd<T, true><<<PT.ntiles[P_XF], NT, lds, s>>>(B, PT.t[P_XF], PT.part[0]);
       else k_xfwd<T, false><<<PT.ntiles[P_XF], NT, lds, s>>>(B, PT.t[P_XF], PT.part[0]);

@@ -385,7 +385,7 @@ size_t plane_lds_bwd(int N1, int N2, int L1, int L2, int elem) {
 
 static hipError_t plane_setup(int bytes) {
   const void* k[] = {(const void*)k_plane_fwd<float>, (const void*)k_plane_fwd<float, false>,
-                     (const void*)k_plane_fwd<double, false>, (const void*)k_plane_bwd<float>,
+                     (const void*)k_plane_bwd<float>,
                      (const void*)k_plane_kin_pc<double>};
   for (const void* f : k) {
     const hipError_t e =
@@ -416,10 +416,9 @@ hipError_t launch_plane_fwd(const Batch& B, const TileTable& t, const TileTable&
   k_plane_fwd<T><<<ntiles, PlaneNT<T>::v, lds, s>>>(B, t, ft, part);
   return hipGetLastError();
 }
-template <typename T>
 hipError_t launch_plane_grow(const Batch& B, const TileTable& t, int ntiles, size_t lds,
                              hipStream_t s) {
-  k_plane_fwd<T, false><<<ntiles, PlaneNT<T>::v, lds, s>>>(B, t, t, nullptr);
+  k_plane_fwd<float, false><<<ntiles, PlaneNT<float>::v, lds, s>>>(B, t, t, nullptr);
   return hipGetLastError();
 }
 template <typename T>
@@ -430,10 +429,6 @@ hipError_t launch_plane_bwd(const Batch& B, const TileTable& t, int ntiles, size
 }
 template hipError_t launch_plane_fwd<float>(const Batch&, const TileTable&, const TileTable&,
                                             int, size_t, double*, hipStream_t);
-template hipError_t launch_plane_grow<double>(const Batch&, const TileTable&, int, size_t,
-                                              hipStream_t);
-template hipError_t launch_plane_grow<float>(const Batch&, const TileTable&, int, size_t,
-                                             hipStream_t);
 template hipError_t launch_plane_bwd<float>(const Batch&, const TileTable&, int, size_t,
                                             hipStream_t);
 

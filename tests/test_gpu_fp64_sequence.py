@@ -78,3 +78,32 @@ def test_launch_edges_match_the_oracle(ctx, geo, n, keys):
         assert rel_err(h - h0, ho - h0) < TOL
     assert rel_err(ek.cpu().numpy(), eo) < TOL
     assert rel_err(ep.cpu().numpy(), po) < TOL
+
+
+# (geo, n, spins): one work-group shape each, groups of one spin that are
+# full, partly full, single or (all orbitals spin down) missing
+DENSITY = [("P", (0, 0, 0), [0]), ("P", (4, 3, 5), [1, 0, 1]), ("P", (22, 21, 2), [1, 1]),
+           ("P", (38, 41, 0), [0, 1, 0, 0, 1]), ("P", (48, 48, 1), [0, 0]),
+           ("P", (49, 50, 0), [1, 0]), ("P", (63, 63, 0), [0, 1]),
+           ("F", (4, 3, 1), [0, 1]), ("F", (20, 21, 0), [1]), ("F", (35, 35, 0), [0, 1]),
+           ("F", (40, 30, 1), [0]), ("P", (1, 2, 2), [k % 2 for k in range(2000)])]
+
+
+@pytest.mark.parametrize("geo,n,spin", DENSITY,
+                         ids=[f"{g}{n[0]}x{n[1]}x{n[2]}-{len(s)}" for g, n, s in DENSITY])
+def test_density_launch_edges_match_the_oracle(ctx, geo, n, spin):
+    """rho += hfac psir^2 within 1e-12 of max rho: every point sums squares
+    of sums of 3 x 31 products"""
+    reg = dense_region(geo, n, (0.45, 0.4, 0.5))
+    norb = len(spin)
+    print(f"case {geo} n={n} norb={norb}", flush=True)
+    psi = random_psi(reg, norb, 41)
+    hfac = np.random.default_rng(42).uniform(0.1, 2.0, norb)
+    rho0 = np.random.default_rng(43).uniform(0.0, 1.0, (2, reg.n_isf))
+    lr = ctx.region(reg)
+    rho = dev(rho0)
+    ctx.density(lr, dev(psi), hfac, rho, spin=spin, nspin=2)
+    lr.close()
+    want = oracle.density(geo, reg.n, reg.nfl, reg.nfu, okeys(reg), psi, hfac, spin, 2)
+    got = rho.cpu().numpy() - rho0
+    assert np.abs(got - want.reshape(2, -1)).max() < TOL * max(np.abs(want).max(), 1.0)
