@@ -189,7 +189,8 @@ __global__ __launch_bounds__(ZG_NT) void k_zgrow(Batch B, TileTable tt) {
 // ---------------------------------------------------------------------------
 // hpsi += compress(G_z^T TZ + K + K_z W), ekin partial.  MI: chunks of four
 // coarse z per wave, their sums held in registers while the LDS rows change
-// from W to TZ to the records of hpsi.
+// from W to TZ to the records of hpsi.  The
+// first loads of K and TZ are issued before the passes ahead of them.
 // ---------------------------------------------------------------------------
 template <int ZB_NT, int MI, int WPE>
 __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, TileTable ft,
@@ -208,34 +209,48 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t ps = 4 * (size_t)(bd.N[0] * bd.N[1]);
+  // K of a chunk; the lines of TZ, TR rows of this wave at a time
+  const double* K = (const double*)B.K + bd.w_off + ct.at;
+  auto load_k = [&](int i0, double k[8]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int z = min(i0 + r, N3 - 1);
+      k[r] = K[ps * z];
+      k[4 + r] = K[ps * (N3 + z)];
+    }
+  };
+  constexpr int TR = 8;
+  const double* tz = (const double*)B.TZ + bd.tz_off + ct.at;
+  auto load_tz = [&](int pb, double v[TR]) {
+#pragma unroll
+    for (int u = 0; u < TR; ++u) v[u] = tz[ps * min(pb + u * NW, L3 - 1)];
+  };
+  double k0[8], tv[TR];
+  load_k(4 * w, k0);
   load_columns<ZB_NT>(lds, bd, B.psi, ct.q0, ct.nq);
   __syncthreads();
+  load_tz(w, tv);
   double o[MI][8];   // c, then d
   double ek = 0.0;
   {
     const double* c = lds + lane;
     const double* d = c + N3 * NL;
     const double ks = bd.kscale[2];
-    const double* K = (const double*)B.K + bd.w_off + ct.at;
 #pragma unroll
     for (int m = 0; m < MI; ++m) {
       const int i0 = 4 * (w + m * NW);
       if (i0 < N3) {
         double k[8];
+        if (m > 0) load_k(i0, k);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int z = min(i0 + r, N3 - 1);
-          k[r] = K[ps * z];
-          k[4 + r] = K[ps * (N3 + z)];
-          o[m][r] = o[m][4 + r] = 0.0;
-        }
+        for (int r = 0; r < 8; ++r) o[m][r] = 0.0;
         line_taps<32>(i0 - 14, N3, per, [&](int kk, int z) {
           kin_tap(kk, c[z * NL], d[z * NL], o[m], o[m] + 4);
         });
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          o[m][r] = fma(o[m][r], ks, k[r]);
-          o[m][4 + r] = fma(o[m][4 + r], ks, k[4 + r]);
+          o[m][r] = fma(o[m][r], ks, m > 0 ? k[r] : k0[r]);
+          o[m][4 + r] = fma(o[m][4 + r], ks, m > 0 ? k[4 + r] : k0[4 + r]);
           if (i0 + r < N3) {   // lanes off the box hold W = 0
             ek = fma(o[m][r], c[(i0 + r) * NL], ek);
             ek = fma(o[m][4 + r], d[(i0 + r) * NL], ek);
@@ -245,18 +260,11 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
     }
   }
   __syncthreads();
-  {
-    // the lines of TZ: one row of 64 values per wave and step
-    const double* src = (const double*)B.TZ + bd.tz_off + ct.at;
-    constexpr int UR = 8;
-    for (int pb = w; pb < L3; pb += NW * UR) {
-      double v[UR];
+  for (int pb = w; pb < L3; pb += NW * TR) {
+    if (pb > w) load_tz(pb, tv);
 #pragma unroll
-      for (int u = 0; u < UR; ++u) v[u] = src[ps * min(pb + u * NW, L3 - 1)];
-#pragma unroll
-      for (int u = 0; u < UR; ++u)
-        if (pb + u * NW < L3) lds[(pb + u * NW) * NL + lane] = v[u];
-    }
+    for (int u = 0; u < TR; ++u)
+      if (pb + u * NW < L3) lds[(pb + u * NW) * NL + lane] = tv[u];
   }
   __syncthreads();
 #pragma unroll
@@ -293,7 +301,7 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
   }
   __syncthreads();
   {
-    constexpr int ZS = ZB_NT / 128, UR = 4;
+    constexpr int ZS = ZB_NT / 128, UR = 8;
     const int e = threadIdx.x & 127, npl = bd.N[0] * bd.N[1];
     const RecElem re(e);
     if (re.col < ct.nq) {
