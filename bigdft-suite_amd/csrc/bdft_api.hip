@@ -2,6 +2,7 @@
 // upload), batch plans and their hipGraph capture.
 #include <algorithm>
 #include <map>
+#include <mutex>
 #include <tuple>
 #include <cstdarg>
 #include <cstdio>
@@ -209,6 +210,25 @@ static __device__ __align__(256) unsigned char scratch[BDFT_FIXED_BYTES];
 // ---------------------------------------------------------------------------
 // context
 // ---------------------------------------------------------------------------
+// LDS bytes a work-group may use on a device (current); the kernels'
+// dynamic-LDS limits, a property of the loaded code object, are raised to it
+// by the first context of the device (some 60 calls, 0.6 ms)
+static size_t kernel_lds(int device) {
+  static std::mutex mu;
+  static std::map<int, size_t> known;
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = known.find(device);
+  if (it != known.end()) return it->second;
+  const size_t lds = plane_attributes();
+  if (lds) {
+    mfma_attributes(lds);
+    line_attributes(lds);
+    fp64_attributes(lds);
+    known[device] = lds;
+  }
+  return lds;
+}
+
 extern "C" int bdft_ctx_create(int device, bdft_ctx** out) {
   if (!out) return BDFT_ERR_ARG;
   *out = nullptr;
@@ -223,12 +243,7 @@ extern "C" int bdft_ctx_create(int device, bdft_ctx** out) {
     return BDFT_ERR_HIP;
   }
   ctx->stream = ctx->own;
-  ctx->plane_lds = plane_attributes();
-  if (ctx->plane_lds) {
-    mfma_attributes(ctx->plane_lds);
-    line_attributes(ctx->plane_lds);
-    fp64_attributes(ctx->plane_lds);
-  }
+  ctx->plane_lds = kernel_lds(device);
   const char* env = getenv("BDFT_LINE_PASSES");
   ctx->force_lines = env && env[0] == '1';
   // this device's copy of the fixed array (its device is current here)
@@ -1157,14 +1172,16 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
             },
             T.pbg, T.nt_pbg, T.lds_pbg, T.shape_pbg, T.nthr_pbg, T.n_pbg, pb_off);
     }
-    // preconditioner plans (FP64): the x and y operator as one plane pass
-    // where the W and K planes of the largest box fit in LDS
-    size_t lk = 0;
-    for (int i = 0; i < norb; ++i)
-      lk = std::max(lk, plane_lds_kin(box[i].N[0], box[i].N[1], (int)sizeof(double)));
-    T.pc_plane = density && !grow_plane && !ctx->force_lines && !mfma && esz == 8 &&
-                 lk <= ctx->plane_lds;
-    T.lds_pc = lk;
+    // preconditioner plans (FP64): z lines and x-y planes where all boxes fit
+    T.pc_plane = density && !grow_plane && !ctx->force_lines && esz == 8;
+    for (int i = 0; i < norb && T.pc_plane; ++i) {
+      const size_t z = fp64_fit_z(box[i], ctx->plane_lds);
+      if (!z || !fp64_fit_kin(box[i], ctx->plane_lds).shape) T.pc_plane = 0;
+      T.lds_cz = std::max(T.lds_cz, z);
+    }
+    if (T.pc_plane)
+      group(P_PF, [&](const BoxDesc& b) { return fp64_fit_kin(b, ctx->plane_lds); }, T.pfg,
+            T.nt_pfg, T.lds_pfg, T.shape_pfg, T.nthr_pfg, T.n_pfg, pf_off);
   }
   // tile order: the z-line and line passes deal their tiles in contiguous
   // ranges per XCD (neighbouring bundles share cache lines); the plane and
@@ -1176,7 +1193,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     T.pf2.xcd = T.pb2.xcd = po;
     for (int k = 0; k < 4; ++k) T.vbg[k].xcd = T.pfg[k].xcd = T.pbg[k].xcd = po;
     // the two x-y kinetic planes of a coarse z read the same fine records
-    if (esz == 8 && !density) {
+    if (esz == 8 && (!density || T.pc_plane)) {
       T.t[P_PF].xcd = 1;
       for (int k = 0; k < 4; ++k) T.pfg[k].xcd = 1;
     }
@@ -1368,6 +1385,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   if (fp64_seq) wv = t2tot = t3tot = 0;
   else tztot = 0;
   if (fp64_seq && density) kv = 0;
+  if (T.pc_plane) wv = t1tot = t2tot = t3tot = 0;   // preconditioner: K
   T.xbig = xbig;
   T.zbig = zbig;
   T.zshort = maxL3 <= ZSHORT_L;
@@ -2107,7 +2125,8 @@ extern "C" int bdft_precond_cg_d(bdft_ctx* ctx, int norb, const bdft_lr* const* 
   auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
   const size_t nvec = sizeof(double) * (size_t)ntot;
   const size_t npc = sizeof(double) * pc.size(), nsc = sizeof(double) * 4 * (size_t)norb;
-  const size_t npart = sizeof(double) * std::max(1, plan->T.ntiles[P_UNC]);
+  const size_t npart =
+      sizeof(double) * std::max(1, std::max(plan->T.ntiles[P_UNC], plan->T.ntiles[P_PF]));
   DevBuf& buf = ctx->pc_buf;
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));  // the buffer may be reallocated
   int rc = dev_alloc(ctx, buf, 3 * al(nvec) + al(npc) + al(nsc) + al(npart));

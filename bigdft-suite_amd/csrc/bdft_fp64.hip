@@ -333,6 +333,95 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
 }
 
 // ---------------------------------------------------------------------------
+// Preconditioner, first half of A v = S (K + c) S v: K = c W + K_z W, W = S v.
+// MODE 0: v = x; 1: v = d; 2: v = d after the step's updates of the compressed
+// vectors, x += alpha d and d = r + beta d (the only kernel that reads whole
+// records of all three, so both updates ride on it: a conjugate-gradient step
+// moves 112 bytes per coefficient, in kernels of their own 144).  64 orbitals
+// of a periodic 48^3 box, six steps: 13.1 ms with the volumes W and K scattered
+// and gathered by kernels of their own, 9.0 now; this kernel 0.53 ms (48 bytes
+// per coefficient, 5.2 TB/s: bound by memory), k_xykin 0.57, the update of r
+// 0.23.
+// ---------------------------------------------------------------------------
+constexpr int PZ_NT = 512;
+template <int MODE>
+__global__ __launch_bounds__(PZ_NT, 6) void k_pcz(Batch B, TileTable tt, PcArgs P) {
+  constexpr int NW = PZ_NT / 64, ZS = PZ_NT / 128, UR = MODE == 2 ? 4 : 8;
+  extern __shared__ __align__(16) unsigned char smem[];
+  double* lds = (double*)smem;
+  const int tile = tile_of(tt);
+  const int b = find_box(tt, tile);
+  const BoxDesc bd = B.box[b];
+  const int N3 = bd.N[2], per = bd.per, npl = bd.N[0] * bd.N[1];
+  const ColTile ct(bd, tile - box_first_tile(tt, b));
+  {
+    const RecElem re(threadIdx.x & 127);
+    const bool on = re.col < ct.nq;
+    const int lin0 = ct.q0 + (on ? re.col : 0);
+    const int* inv = re.t == 0 ? bd.cinv : bd.finv;
+    const unsigned off = re.t == 0 ? 0u : 8u * (unsigned)(bd.nvctr_c + re.t - 1);
+    const unsigned mul = re.t == 0 ? 8u : 56u;
+    char *x = (char*)(P.x + bd.psi_off), *d = (char*)(P.d + bd.psi_off);
+    const char* r = (const char*)(P.r + bd.psi_off);
+    const double sc = P.pc[9 * b + 1 + re.t];
+    const double alpha = MODE == 2 ? P.sc[4 * b + 1] : 0.0;
+    const double beta = MODE == 2 ? P.sc[4 * b + 2] : 0.0;
+    double* dst = lds + (re.t >> 2) * N3 * NL + re.col + CC * (re.t & 3);
+    for (int zb = threadIdx.x >> 7; zb < N3; zb += ZS * UR) {
+      int e[UR];
+      double v[UR], rv[UR], xv[UR];
+#pragma unroll
+      for (int u = 0; u < UR; ++u) {
+        const int z = zb + u * ZS, lin = lin0 + npl * z;
+        e[u] = -1;
+        if (on && z < N3) e[u] = inv ? inv[lin] : lin;
+      }
+#pragma unroll
+      for (int u = 0; u < UR; ++u) {
+        const unsigned at = off + mul * (unsigned)e[u];
+        v[u] = e[u] >= 0 ? *(const double*)((MODE == 0 ? x : d) + at) : 0.0;
+        if (MODE == 2) {
+          rv[u] = e[u] >= 0 ? *(const double*)(r + at) : 0.0;
+          xv[u] = e[u] >= 0 ? *(const double*)(x + at) : 0.0;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < UR; ++u) {
+        if (MODE == 2 && e[u] >= 0) {
+          const unsigned at = off + mul * (unsigned)e[u];
+          *(double*)(x + at) = fma(alpha, v[u], xv[u]);
+          v[u] = fma(beta, v[u], rv[u]);
+          *(double*)(d + at) = v[u];
+        }
+        if (zb + u * ZS < N3) dst[(zb + u * ZS) * NL] = sc * v[u];
+      }
+    }
+  }
+  __syncthreads();
+  const double* c = lds + (threadIdx.x & 63);
+  const double* d = c + N3 * NL;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const size_t ps = 4 * (size_t)npl;
+  const double ks = bd.kscale[2], cp = P.pc[9 * b];
+  double* K = (double*)B.K + bd.w_off + ct.at;
+  for (int i0 = 4 * w; i0 < N3; i0 += 4 * NW) {
+    double o[8];
+#pragma unroll
+    for (int h = 0; h < 8; ++h) o[h] = 0.0;
+    line_taps<32>(i0 - 14, N3, per,
+                  [&](int kk, int z) { kin_tap(kk, c[z * NL], d[z * NL], o, o + 4); });
+    if (ct.on) {
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+        if (i0 + h < N3) {
+          K[ps * (i0 + h)] = fma(cp, c[(i0 + h) * NL], o[h] * ks);
+          K[ps * (N3 + i0 + h)] = fma(cp, d[(i0 + h) * NL], o[4 + h] * ks);
+        }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // in-plane passes.  One of a thread's work items is one chunk of a line, lanes along the
 // lines.  A pass keeps its items' outputs in registers (at most MI items of 8
 // values a thread) and writes them over the plane after a barrier, transposed
@@ -462,13 +551,20 @@ __device__ __forceinline__ void each_item(ItDiv d, int n, int nch, F f) {
 // planes of a coarse z are neighbouring tiles: they read the same fine
 // records).  K_y, along the columns, goes to memory first; K_x goes over the
 // plane in LDS and from there is added to it.
+//
+// PC: the last half of the preconditioner's A v = S (K + c) S v, W = S v of
+// the compressed vector v and c W + K_z W in K (k_pcz): S (K + K_x W + K_y W)
+// goes to the compressed vectors.  1, v = x: r = b - A x, d = r, partial
+// |r|^2; 2, v = d: q = A d, partial q d.
 // ---------------------------------------------------------------------------
-template <int NTM, int MI, int WPE>
-__global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt) {
+template <int NTM, int MI, int WPE, int PC = 0>
+__global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt, TileTable ft,
+                                                    PcArgs P) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int tile = tile_of(tt);
   const int lb = find_box(tt, tile);
-  const BoxDesc bd = B.box[table_box(tt, lb)];
+  const int b = table_box(tt, lb);
+  const BoxDesc bd = B.box[b];
   const int lt = tile - box_first_tile(tt, lb);
   const int N1 = bd.N[0], N2 = bd.N[1], N3 = bd.N[2], per = bd.per;
   const int s3 = lt & 1, i3 = lt >> 1;
@@ -478,16 +574,17 @@ __global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt) {
   int2* my = mx + map_len(N1);
   const int tid = threadIdx.x, nt = blockDim.x;
   // gather: thread's component c = s1 + 2 s2 of every (nt / 4)-th point
+  const int c = tid & 3, st = nt >> 2;
+  const bool cs = c == 0 && s3 == 0;
+  const unsigned off = cs ? 0u : 8u * (unsigned)(bd.nvctr_c + c + 4 * s3 - 1);
+  const unsigned mul = cs ? 8u : 56u;
+  const int* inv = cs ? bd.cinv : bd.finv;
+  const int lin0 = npl * i3;
+  const double sc = PC ? P.pc[9 * b + 1 + c + 4 * s3] : 1.0;
   {
     constexpr int UR = 8;
-    const int c = tid & 3, st = nt >> 2;
-    const bool cs = c == 0 && s3 == 0;
-    const char* src = (const char*)(B.psi + bd.psi_off);
-    const unsigned off = cs ? 0u : 8u * (unsigned)(bd.nvctr_c + c + 4 * s3 - 1);
-    const unsigned mul = cs ? 8u : 56u;
-    const int* inv = cs ? bd.cinv : bd.finv;
+    const char* src = (const char*)((PC == 0 ? B.psi : PC == 1 ? P.x : P.d) + bd.psi_off);
     const bool dense = !bd.cinv && !bd.finv;
-    const int lin0 = npl * i3;
     double* base = A + (c >> 1) * N2 * RA + (c & 1) * N1;
     ItDiv d(tid >> 2, N1, st);
     for (int pb = tid >> 2; pb < npl; pb += st * UR) {
@@ -510,7 +607,7 @@ __global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt) {
       }
 #pragma unroll
       for (int u = 0; u < UR; ++u) {
-        if (pb + u * st < npl) base[d.ch * RA + d.j] = v[u];
+        if (pb + u * st < npl) base[d.ch * RA + d.j] = PC ? sc * v[u] : v[u];
         d.next(N1);
       }
     }
@@ -526,13 +623,23 @@ __global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt) {
   each_item<MI>(ItDiv(tid, W1, nt), W1, cy, [&](int, int ch, int j1) {
     const int i0 = 4 * ch;
     double oc[4], od[4];
-    kin4_any(PLine<double>{A + j1, RA}, my, N2, i0, oc, od);
     const unsigned at = 8u * (unsigned)(j1 + W1 * i0);
+    auto kc = [&](int r) { return (double*)((char*)(K + W1 * r) + at); };
+    double k[8];   // K before, read ahead of the stencil
+    if (PC) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (i0 + r < N2) {
+          k[r] = *kc(r);
+          k[4 + r] = *kc(N2 + r);
+        }
+    }
+    kin4_any(PLine<double>{A + j1, RA}, my, N2, i0, oc, od);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       if (i0 + r < N2) {
-        *(double*)((char*)(K + W1 * r) + at) = oc[r] * ky;
-        *(double*)((char*)(K + W1 * (N2 + r)) + at) = od[r] * ky;
+        *kc(r) = PC ? fma(oc[r], ky, k[r]) : oc[r] * ky;
+        *kc(N2 + r) = PC ? fma(od[r], ky, k[4 + r]) : od[r] * ky;
       }
   });
   double o[MI][8];
@@ -551,6 +658,52 @@ __global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt) {
       }
   });
   __syncthreads();
+  if constexpr (PC != 0) {
+    // the plane's elements of the compressed vectors
+    __shared__ double red[NTM / 64];
+    constexpr int UR = 4;
+    const char* y = (const char*)((PC == 1 ? P.b : P.d) + bd.psi_off);
+    char* q = (char*)((PC == 1 ? P.r : P.q) + bd.psi_off);
+    char* dd = (char*)(P.d + bd.psi_off);
+    const int row0 = (c >> 1) * N2, col0 = (c & 1) * N1;
+    double acc = 0.0;
+    ItDiv d(tid >> 2, N1, st);
+    for (int pb = tid >> 2; pb < npl; pb += st * UR) {
+      int r[UR];
+      double k[UR], v[UR];
+      int a[UR];
+#pragma unroll
+      for (int u = 0; u < UR; ++u) {
+        const int p = pb + u * st;
+        r[u] = -1;
+        if (p < npl) r[u] = inv ? inv[lin0 + p] : lin0 + p;
+        a[u] = (row0 + d.ch) * RA + col0 + d.j;
+        k[u] = p < npl ? K[(row0 + d.ch) * W1 + col0 + d.j] : 0.0;
+        d.next(N1);
+      }
+#pragma unroll
+      for (int u = 0; u < UR; ++u)
+        v[u] = r[u] >= 0 ? *(const double*)(y + (off + mul * (unsigned)r[u])) : 0.0;
+#pragma unroll
+      for (int u = 0; u < UR; ++u)
+        if (r[u] >= 0) {
+          const double av = sc * (k[u] + A[a[u]]);
+          const unsigned at = off + mul * (unsigned)r[u];
+          if (PC == 1) {
+            const double rv = v[u] - av;
+            *(double*)(q + at) = rv;
+            *(double*)(dd + at) = rv;
+            acc = fma(rv, rv, acc);
+          } else {
+            *(double*)(q + at) = av;
+            acc = fma(av, v[u], acc);
+          }
+        }
+    }
+    const double sum = block_sum_rt(acc, red);
+    if (tid == 0) P.part[box_first_tile(ft, b) + lt] = sum;
+    return;
+  }
   // two values at a time (rows of 2 N1 values: 16-byte aligned)
   const int tot = N1 * W2;
   double2* K2 = (double2*)K;
@@ -831,6 +984,7 @@ __global__ __launch_bounds__(256) void k_xyden_sum(DenArgs D) {
 // ---------------------------------------------------------------------------
 // LDS bytes of the kernels for a box
 constexpr size_t LDS_STATIC = 128;   // the kernels' static LDS (reductions)
+static size_t lds_w(int N3) { return (size_t)NL * 2 * N3 * 8; }   // rows of W
 static size_t lds_z(int N3, int L3) { return (size_t)NL * (L3 > 2 * N3 ? L3 : 2 * N3) * 8; }
 size_t fp64_fit_z(const BoxDesc& b, size_t plane_lds) {
   const size_t v = lds_z(b.N[2], b.L[2]);
@@ -891,12 +1045,28 @@ static hipError_t launch_zback(const Batch& B, const TileTable& t, const TileTab
   else k_zback<1024, 3, 4><<<ntiles, 1024, lds, s>>>(B, t, ft, part);
   return hipGetLastError();
 }
-static hipError_t launch_xykin(const Batch& B, const TileTable& t, int ntiles, size_t lds,
-                               int nt, int shape, hipStream_t s) {
+template <int PC>
+static hipError_t launch_xykin(const Batch& B, const TileTable& t, const TileTable& ft,
+                               int ntiles, size_t lds, int nt, int shape, const PcArgs& P,
+                               hipStream_t s) {
   if (ntiles <= 0) return hipSuccess;
-  if (shape >= 2) k_xykin<S2_NT, 2, 6><<<ntiles, nt, lds, s>>>(B, t);
-  else k_xykin<S1_NT, 3, 4><<<ntiles, nt, lds, s>>>(B, t);
+  if (shape >= 2) k_xykin<S2_NT, 2, 6, PC><<<ntiles, nt, lds, s>>>(B, t, ft, P);
+  else k_xykin<S1_NT, 3, 4, PC><<<ntiles, nt, lds, s>>>(B, t, ft, P);
   return hipGetLastError();
+}
+// the x-y kinetic pass: one launch per group of boxes, or one over all
+template <int PC>
+static hipError_t xykin_pass(const Batch& B, const PassTables& PT, const PcArgs& P,
+                             hipStream_t s) {
+  const TileTable& ft = PT.t[P_PF];
+  if (PT.n_pfg == 0)
+    return launch_xykin<PC>(B, ft, ft, PT.ntiles[P_PF], PT.lds_pfg[0], PT.nthr_pfg[0],
+                            PT.shape_pfg[0], P, s);
+  hipError_t e = hipSuccess;
+  for (int k = 0; k < PT.n_pfg && e == hipSuccess; ++k)
+    e = launch_xykin<PC>(B, PT.pfg[k], ft, PT.nt_pfg[k], PT.lds_pfg[k], PT.nthr_pfg[k],
+                         PT.shape_pfg[k], P, s);
+  return e;
 }
 static hipError_t launch_xypot(const Batch& B, const TileTable& t, const TileTable& ft,
                                int ntiles, size_t lds, int nt, int shape, double* part,
@@ -914,16 +1084,11 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
     if (ev) (void)hipEventRecord(ev[2 * stage + end], s);
   };
   mark(S_ZG, 0);
-  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], PT.lds_cz, s);
+  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], lds_w(PT.maxN3), s);
   mark(S_ZG, 1);
   // one launch per group of boxes, or one over all of them
   mark(S_KXY, 0);
-  if (e == hipSuccess && PT.n_pfg == 0)
-    e = launch_xykin(B, PT.t[P_PF], PT.ntiles[P_PF], PT.lds_pfg[0], PT.nthr_pfg[0],
-                     PT.shape_pfg[0], s);
-  for (int k = 0; k < PT.n_pfg && e == hipSuccess; ++k)
-    e = launch_xykin(B, PT.pfg[k], PT.nt_pfg[k], PT.lds_pfg[k], PT.nthr_pfg[k],
-                     PT.shape_pfg[k], s);
+  if (e == hipSuccess) e = xykin_pass<0>(B, PT, PcArgs{}, s);
   mark(S_KXY, 1);
   mark(S_XYP, 0);
   if (e == hipSuccess && PT.n_pbg == 0)
@@ -959,7 +1124,7 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
 
 hipError_t launch_fp64_density(const Batch& B, const PassTables& PT, const DenArgs& D, int L3,
                                hipStream_t s) {
-  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], PT.lds_cz, s);
+  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], lds_w(PT.maxN3), s);
   if (e != hipSuccess) return e;
   const int n = D.ngroups * L3;
   const size_t lds = PT.lds_pbg[0];
@@ -971,6 +1136,21 @@ hipError_t launch_fp64_density(const Batch& B, const PassTables& PT, const DenAr
   return hipGetLastError();
 }
 
+// c W + K_z W + K_x W + K_y W of W = S v and the compressed sums that follow
+// (mode 0: v = x, r = d = b - A x; 1: v = d; 2: x and d of the step first)
+hipError_t launch_fp64_pc_apply(const Batch& B, const PassTables& PT, const PcArgs& P, int mode,
+                                hipStream_t s) {
+  const int n = PT.ntiles[P_CZ];
+  const TileTable& t = PT.t[P_CZ];
+  const size_t lds = lds_w(PT.maxN3);
+  if (mode == 0) k_pcz<0><<<n, PZ_NT, lds, s>>>(B, t, P);
+  else if (mode == 1) k_pcz<1><<<n, PZ_NT, lds, s>>>(B, t, P);
+  else k_pcz<2><<<n, PZ_NT, lds, s>>>(B, t, P);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return mode == 0 ? xykin_pass<1>(B, PT, P, s) : xykin_pass<2>(B, PT, P, s);
+}
+
 // raise the dynamic-LDS limit of the kernels to lds bytes
 void fp64_attributes(size_t lds) {
   const void* k[] = {(const void*)k_zgrow,         (const void*)k_zback<512, 1, 4>,
@@ -978,6 +1158,9 @@ void fp64_attributes(size_t lds) {
                      (const void*)k_zback<1024, 3, 4>,
                      (const void*)k_xyden<512, 3, 4>, (const void*)k_xyden<S1_NT, 3, 4>,
                      (const void*)k_xykin<S2_NT, 2, 6>, (const void*)k_xypot<S2_NT, 2, 6>,
+                     (const void*)k_xykin<S2_NT, 2, 6, 1>, (const void*)k_xykin<S2_NT, 2, 6, 2>,
+                     (const void*)k_xykin<S1_NT, 3, 4, 1>, (const void*)k_xykin<S1_NT, 3, 4, 2>,
+                     (const void*)k_pcz<0>, (const void*)k_pcz<1>, (const void*)k_pcz<2>,
                      (const void*)k_xykin<S1_NT, 3, 4>, (const void*)k_xypot<S1_NT, 3, 4>};
   for (const void* f : k)
     if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=

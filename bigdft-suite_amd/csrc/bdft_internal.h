@@ -443,9 +443,9 @@ struct PassTables {
   // z-line kernels of the FP64 sequence: LDS and longest line of the batch
   size_t lds_cz;
   int maxN3, maxL3;
-  // preconditioner: x and y operator in one plane pass (FP64 planes that fit)
+  // preconditioner: z lines and x-y planes of the compressed vectors
+  // (bdft_fp64.hip) where every box fits, else the line passes
   int pc_plane;
-  size_t lds_pc;
   // lines beyond the register-held outputs: x passes in their BIG forms
   // (some N1 > REG_N or L1 > REG_L), z potential pass in two kernels through
   // T3 (some L3 > REG_L)
@@ -608,16 +608,14 @@ struct PlaneFit {
 PlaneFit fp64_fit_kin(const BoxDesc& b, size_t plane_lds);
 PlaneFit fp64_fit_pot(const BoxDesc& b, size_t plane_lds);
 void fp64_attributes(size_t lds);
+hipError_t launch_fp64_pc_apply(const Batch& B, const PassTables& PT, const PcArgs& P, int mode,
+                                hipStream_t s);
 hipError_t launch_fp64_density(const Batch& B, const PassTables& PT, const DenArgs& D, int L3,
                                hipStream_t s);
 hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
                            hipEvent_t* ev);
 size_t plane_lds_fwd(int N1, int N2, int L1, int elem);
 size_t plane_lds_bwd(int N1, int N2, int L1, int L2, int elem);
-// preconditioner: K = c W + K_x W + K_y W per x-y plane (P_PF tiles)
-size_t plane_lds_kin(int N1, int N2, int elem);
-hipError_t launch_plane_kin_pc(const Batch& B, const TileTable& t, int ntiles, size_t lds,
-                               const double* pc, hipStream_t s);
 size_t plane_attributes();
 template <typename T>
 hipError_t launch_plane_fwd(const Batch& B, const TileTable& t, const TileTable& ft,

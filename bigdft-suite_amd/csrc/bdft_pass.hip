@@ -1689,14 +1689,37 @@ __global__ __launch_bounds__(NT) void k_pc_update(Batch B, TileTable tt, PcArgs 
   }
 }
 
-// x <- S x (scale_psi, OpenCL/Uncompress.c:377-470)
-__global__ __launch_bounds__(NT) void k_pc_final(Batch B, TileTable tt, PcArgs A) {
+// r -= alpha q, partial |r|^2
+__global__ __launch_bounds__(NT) void k_pc_residual(Batch B, TileTable tt, PcArgs A) {
+  __shared__ double red[NT / 64];
+  const int tile = tile_of(tt);
+  const int b = find_box(tt, tile);
+  const PcRange R = pc_range(B.box[b], tile - box_first_tile(tt, b));
+  const double alpha = A.sc[4 * b + 1];
+  double acc = 0.0;
+  for (int e = threadIdx.x; e < R.ne; e += NT) {
+    const long long i = R.e0 + e;
+    const double r = fma(-alpha, A.q[i], A.r[i]);
+    A.r[i] = r;
+    acc = fma(r, r, acc);
+  }
+  const double sum = block_sum(acc, red);
+  if (threadIdx.x == 0) A.part[tile] = sum;
+}
+
+// x <- S x (scale_psi, OpenCL/Uncompress.c:377-470); step, where x has not
+// taken its last step yet (pc_plane): x += alpha d first
+__global__ __launch_bounds__(NT) void k_pc_final(Batch B, TileTable tt, PcArgs A, int step) {
   const int tile = tile_of(tt);
   const int b = find_box(tt, tile);
   const BoxDesc bd = B.box[b];
   const PcRange R = pc_range(bd, tile - box_first_tile(tt, b));
-  for (int e = threadIdx.x; e < R.ne; e += NT)
-    A.x[R.e0 + e] *= pc_scal(A, b, R.fine ? 1 + e % 7 : 0);
+  const double alpha = step ? A.sc[4 * b + 1] : 0.0;
+  for (int e = threadIdx.x; e < R.ne; e += NT) {
+    const long long i = R.e0 + e;
+    const double x = step ? fma(alpha, A.d[i], A.x[i]) : A.x[i];
+    A.x[i] = x * pc_scal(A, b, R.fine ? 1 + e % 7 : 0);
+  }
 }
 
 // one block per box: s = sum of the box's tile partials (fixed order).
@@ -1728,23 +1751,39 @@ hipError_t launch_precond(const Batch& B, const PassTables& PT, int maxN, long l
   const size_t lds = lds_bytes(maxN, sizeof(double));
   const int nu = PT.ntiles[P_UNC];
   const TileTable& tu = PT.t[P_UNC];
+  if (nu > 0 && PT.pc_plane) {
+    // x and d are updated by the next step's first kernel, x once more at the
+    // end; partial sums by plane after an apply, by compressed tile after the
+    // update of r
+    const TileTable& tp = PT.t[P_PF];
+    hipError_t e = hipSuccess;
+    if (A.ncong > 0) {
+      e = launch_fp64_pc_apply(B, PT, A, 0, s);
+      k_pc_scalars<<<B.nbox, NT, 0, s>>>(tp, A, 0);
+    }
+    for (int it = 0; it < A.ncong && e == hipSuccess; ++it) {
+      e = launch_fp64_pc_apply(B, PT, A, it == 0 ? 1 : 2, s);
+      k_pc_scalars<<<B.nbox, NT, 0, s>>>(tp, A, 1);
+      if (it < A.ncong - 1) {
+        k_pc_residual<<<nu, NT, 0, s>>>(B, tu, A);
+        k_pc_scalars<<<B.nbox, NT, 0, s>>>(tu, A, 2);
+      }
+    }
+    k_pc_final<<<nu, NT, 0, s>>>(B, tu, A, A.ncong > 0);
+    return e != hipSuccess ? e : hipGetLastError();
+  }
   if (need_zero) {
     const long long nb = (wtotal + NT - 1) / NT;
     k_zero<double><<<(unsigned)(nb < 65536 ? nb : 65536), NT, 0, s>>>((double*)B.W, wtotal);
   }
   auto apply = [&](const double* src, int update) {
     if (nu > 0) k_pc_scatter<<<nu, NT, 0, s>>>(B, tu, A, src, update);
-    if (PT.pc_plane) {
-      // c W + K_x W + K_y W of each plane in one pass through LDS
-      (void)launch_plane_kin_pc(B, PT.t[P_PF], PT.ntiles[P_PF], PT.lds_pc, A.pc, s);
-    } else {
-      if (PT.ntiles[P_XF] > 0) {
-        if (PT.xbig) k_pc_kinx<true><<<PT.ntiles[P_XF], NT, lds, s>>>(B, PT.t[P_XF], A);
-        else k_pc_kinx<false><<<PT.ntiles[P_XF], NT, lds, s>>>(B, PT.t[P_XF], A);
-      }
-      if (PT.ntiles[P_KY] > 0)
-        k_kin<double, 1><<<PT.ntiles[P_KY], NT, lds, s>>>(B, PT.t[P_KY], PT.part[1]);
+    if (PT.ntiles[P_XF] > 0) {
+      if (PT.xbig) k_pc_kinx<true><<<PT.ntiles[P_XF], NT, lds, s>>>(B, PT.t[P_XF], A);
+      else k_pc_kinx<false><<<PT.ntiles[P_XF], NT, lds, s>>>(B, PT.t[P_XF], A);
     }
+    if (PT.ntiles[P_KY] > 0)
+      k_kin<double, 1><<<PT.ntiles[P_KY], NT, lds, s>>>(B, PT.t[P_KY], PT.part[1]);
     if (PT.ntiles[P_KZ] > 0)
       k_kin<double, 2><<<PT.ntiles[P_KZ], NT, lds, s>>>(B, PT.t[P_KZ], PT.part[2]);
   };
@@ -1760,7 +1799,7 @@ hipError_t launch_precond(const Batch& B, const PassTables& PT, int maxN, long l
     k_pc_update<<<nu, NT, 0, s>>>(B, tu, A, last);
     if (!last) k_pc_scalars<<<B.nbox, NT, 0, s>>>(tu, A, 2);
   }
-  k_pc_final<<<nu, NT, 0, s>>>(B, tu, A);
+  k_pc_final<<<nu, NT, 0, s>>>(B, tu, A, 0);
   return hipGetLastError();
 }
 

@@ -208,82 +208,6 @@ __global__ __launch_bounds__(PlaneNT<T>::v) void k_plane_fwd(Batch B, TileTable 
 }
 
 // ---------------------------------------------------------------------------
-// Preconditioner operator, x and y part, of one x-y plane of a box:
-//   K = c W + Ktilde_x W + Ktilde_y W      (c = cprecr of the box, pc[9 b])
-// the work of the x kinetic line pass (k_pc_kinx) and the y one (k_kin<1>)
-// in one read of the W plane and one write of K, in the same order of
-// operations (c W + K_x first, then + K_y)
-// ---------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(PlaneNT<T>::v) void k_plane_kin_pc(Batch B, TileTable tt,
-                                                                const double* pc) {
-  constexpr int NTP = PlaneNT<T>::v;
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int tile = tile_of(tt);
-  const int lb = find_box(tt, tile);
-  const int b = table_box(tt, lb);
-  const BoxDesc bd = B.box[b];
-  const int j3 = tile - box_first_tile(tt, lb);
-  const int N1 = bd.N[0], N2 = bd.N[1], per = bd.per;
-  const int W1 = 2 * N1, W2 = 2 * N2;
-  const int RA = W1 + 1;
-  T* A = (T*)smem;                  // W plane: A[j2*RA + j1]
-  T* C = A + (W2 + 1) * RA;         // K plane, same layout
-  int2* mx = (int2*)(smem + plane_maps_off(N1, N2, RA, sizeof(T)));
-  int2* mya = mx + map_len(N1);
-  const T* src = (const T*)B.W + bd.w_off + (long long)W1 * W2 * j3;
-  const int tid = threadIdx.x;
-  plane_load<T, NTP>(A, RA, src, W1, W2);
-  build_map(mx, N1, per, sizeof(T), W1, tid, NTP);
-  build_map(mya, N2, per, RA * sizeof(T), W2, tid, NTP);
-  plane_zero_slots<T, NTP>(A, RA, W1, W2, C, RA);
-  __syncthreads();
-  const T kx = (T)bd.kscale[0], ky = (T)bd.kscale[1], c = (T)pc[9 * b];
-  const int cx = (N1 + 3) >> 2;
-  for (ItDiv d(tid, W2, NTP); d.ch < cx; d.next(W2)) {
-    const int ch = d.ch, j2 = d.j;
-    const int i0 = 4 * ch;
-    T oc[4], od[4];
-    kin4_any(PLine<T>{A + j2 * RA, 1}, mx, N1, i0, oc, od);
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (i0 + r < N1) {
-        const int a = j2 * RA + i0 + r, d = j2 * RA + N1 + i0 + r;
-        C[a] = fma(c, A[a], oc[r] * kx);
-        C[d] = fma(c, A[d], od[r] * kx);
-      }
-  }
-  __syncthreads();
-  const int cy = (N2 + 3) >> 2;
-  for (ItDiv d(tid, W1, NTP); d.ch < cy; d.next(W1)) {
-    const int ch = d.ch, j1 = d.j;
-    const int i0 = 4 * ch;
-    T oc[4], od[4];
-    kin4_any(PLine<T>{A + j1, RA}, mya, N2, i0, oc, od);
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (i0 + r < N2) {
-        const int a = (i0 + r) * RA + j1, d = (N2 + i0 + r) * RA + j1;
-        C[a] += oc[r] * ky;
-        C[d] += od[r] * ky;
-      }
-  }
-  __syncthreads();
-  T* kd = (T*)B.K + bd.w_off + (long long)W1 * W2 * j3;
-  plane_store<T, NTP>(kd, C, RA, W1, W2);
-}
-
-size_t plane_lds_kin(int N1, int N2, int elem) {
-  return plane_maps_off(N1, N2, 2 * N1 + 1, elem) + 8 * (size_t)(map_len(N1) + map_len(N2));
-}
-
-hipError_t launch_plane_kin_pc(const Batch& B, const TileTable& t, int ntiles, size_t lds,
-                               const double* pc, hipStream_t s) {
-  if (ntiles > 0) k_plane_kin_pc<double><<<ntiles, PlaneNT<double>::v, lds, s>>>(B, t, pc);
-  return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
 // backward plane kernel with compress-accumulate
 // ---------------------------------------------------------------------------
 template <typename T>
@@ -385,8 +309,7 @@ size_t plane_lds_bwd(int N1, int N2, int L1, int L2, int elem) {
 
 static hipError_t plane_setup(int bytes) {
   const void* k[] = {(const void*)k_plane_fwd<float>, (const void*)k_plane_fwd<float, false>,
-                     (const void*)k_plane_bwd<float>,
-                     (const void*)k_plane_kin_pc<double>};
+                     (const void*)k_plane_bwd<float>};
   for (const void* f : k) {
     const hipError_t e =
         hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);

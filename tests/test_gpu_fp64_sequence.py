@@ -107,3 +107,31 @@ def test_density_launch_edges_match_the_oracle(ctx, geo, n, spin):
     want = oracle.density(geo, reg.n, reg.nfl, reg.nfu, okeys(reg), psi, hfac, spin, 2)
     got = rho.cpu().numpy() - rho0
     assert np.abs(got - want.reshape(2, -1)).max() < TOL * max(np.abs(want).max(), 1.0)
+
+
+@pytest.mark.parametrize("geo,n", [("P", (4, 3, 5)), ("P", (22, 22, 32)), ("P", (48, 48, 1)),
+                                   ("P", (49, 49, 2)), ("P", (63, 63, 0)), ("P", (70, 69, 0)),
+                                   ("F", (15, 16, 48)), ("F", (35, 36, 1)), ("F", (49, 50, 1)),
+                                   ("F", (2, 1, 144)), ("F", (2, 1, 147))],
+                         ids=lambda v: v if isinstance(v, str) else "x".join(map(str, v)))
+@pytest.mark.parametrize("keys", ["dense", "sparse"])
+def test_precond_launch_edges_match_the_oracle(ctx, geo, n, keys):
+    """three steps, every update in another kernel than the oracle's: 1e-10
+    of max|x|, the bar of the preconditioner's parity tests"""
+    reg = dense_region(geo, n, (0.45, 0.4, 0.5))
+    if keys == "sparse":
+        rng = np.random.default_rng(sum(n) + 7)
+        lg = rng.random(tuple(x + 1 for x in n)) < 0.6
+        lg[0, 0, 0] = True
+        reg = region_from_grids(geo, n, (0.45, 0.4, 0.5), lg, lg & (rng.random(lg.shape) < 0.5))
+    print(f"case {geo} n={n} {keys}", flush=True)
+    b, x0 = random_psi(reg, 2, 51), 0.05 * random_psi(reg, 2, 52)
+    cpr = [0.3, 0.9]
+    lr = ctx.region(reg)
+    x = dev(x0.ravel())
+    ctx.precond_cg([lr, lr], cpr, 3, x, dev(b.ravel()))
+    got = x.cpu().numpy().reshape(2, -1)
+    lr.close()
+    for i in range(2):
+        want = oracle.precond_cg(geo, reg.n, reg.hgrid, cpr[i], 3, okeys(reg), x0[i], b[i])
+        assert np.abs(got[i] - want).max() < 1e-10 * np.abs(want).max()
