@@ -721,6 +721,10 @@ static int box_tiles(const BoxDesc& b, int pass, int zg) {
     case P_ZPF: return cdiv((long long)L1 * L2, TW);
     case P_CZ: return cdiv((long long)N1 * N2, CCOL);
     case P_RP: return b.L[2];
+    case P_XK: return cdiv((long long)N2 * N3, CCOL);
+    case P_YK: return cdiv(N1, CCOL) * N3;
+    case P_XR: return cdiv(2LL * N2 * b.L[2], 64);
+    case P_YL: return cdiv((long long)L1 * b.L[2], 64);
   }
   return 0;
 }
@@ -736,6 +740,7 @@ struct PlanChoice {
   int zg;
   int fused, zvalu, bvalu;  // matrix-core sequence
   int plane;                // vector-unit sequence: plane-fused or line passes
+  int kin_lines, pot_lines; // FP64 sequence: x-y passes on lines
   int xbig, zbig;
   int nthr_rp[4];           // FP64 potential pass: threads by launch shape
                             // (they set the order of the epot sums)
@@ -780,7 +785,8 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   const bool f16 = precision == BDFT_PREC_F16X3;
   TabSet tabs;
   std::vector<BoxDesc> box((size_t)norb);
-  long long wtot = 0, t1tot = 0, t2tot = 0, t3tot = 0, tztot = 0, psi_run = 0;
+  long long wtot = 0, t1tot = 0, t2tot = 0, t3tot = 0, tztot = 0, txtot = 0,
+            psi_run = 0;
   int maxN = 0, maxN3 = 0;
   bool xbig = false, zbig = false;
   int maxL3 = 0;
@@ -855,6 +861,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     t2tot += (long long)b.L[0] * b.L[1] * 2 * b.N[2];
     t3tot += (long long)b.L[0] * b.L[1] * b.L[2];
     tztot += 4LL * b.N[0] * b.N[1] * b.L[2];
+    txtot += 2LL * b.N[1] * b.L[0] * b.L[2];
     xbig = xbig || b.N[0] > REG_N || b.L[0] > REG_L;
     zbig = zbig || b.L[2] > REG_L;
     maxL3 = std::max(maxL3, b.L[2]);
@@ -1079,12 +1086,15 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     bool plane = !ctx->force_lines && !mfma && (!density || grow_plane);
     const bool d64 = esz == 8;   // the FP64 sequence (bdft_fp64.hip)
     size_t lpf = 0, lpb = 0, lcz = 0;
-    bool fits = true;
+    // FP64 sequence: z lines fit; planes of every box fit, else lines do
+    bool fits = true, kp = true, pp = true, kl = true, pl = true;
     for (int i = 0; i < norb && plane; ++i) {
       const BoxDesc& b = box[i];
       if (d64) {
-        fits = fits && (density || fp64_fit_kin(b, ctx->plane_lds).shape) &&
-               fp64_fit_pot(b, ctx->plane_lds).shape;
+        kp = kp && fp64_fit_kin(b, ctx->plane_lds).shape;
+        pp = pp && fp64_fit_pot(b, ctx->plane_lds).shape;
+        kl = kl && fp64_kin_lines_ok(b, ctx->plane_lds);
+        pl = pl && fp64_pot_lines_ok(b, ctx->plane_lds);
         const size_t z = fp64_fit_z(b, ctx->plane_lds);
         fits = fits && z;
         lcz = std::max(lcz, z);
@@ -1093,14 +1103,27 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
         lpb = std::max(lpb, plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1], (int)esz));
       }
     }
+    if (d64) fits = fits && (density ? pp : (kp || kl) && (pp || pl));
     if (!fits || std::max(lpf, lpb) > ctx->plane_lds) plane = false;
     T.plane = plane ? 1 : 0;
-    if (force) T.plane = force->plane;
+    T.kin_lines = plane && d64 && !kp;
+    T.pot_lines = plane && d64 && !pp;
+    if (force) {
+      T.plane = force->plane;
+      T.kin_lines = force->kin_lines;
+      T.pot_lines = force->pot_lines;
+    }
     T.lds_pf = lpf;
     T.lds_pb = lpb;
     T.lds_cz = lcz;
     T.maxN3 = maxN3;
-    T.maxL3 = maxL3;
+    T.maxN1 = T.maxN2 = T.maxL1 = T.maxL2 = 0;
+    for (const BoxDesc& b : box) {
+      T.maxN1 = std::max(T.maxN1, b.N[0]);
+      T.maxN2 = std::max(T.maxN2, b.N[1]);
+      T.maxL1 = std::max(T.maxL1, b.L[0]);
+      T.maxL2 = std::max(T.maxL2, b.L[1]);
+    }
     // plane passes: the boxes grouped by how many of their work-groups fit a
     // CU (FP32, at most four) or by launch shape (FP64), one launch per group
     // with the group's largest LDS, so that the largest box does not set
@@ -1149,12 +1172,13 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     };
     T.n_pfg = T.n_pbg = 0;
     if (T.plane && d64) {
-      if (!density)
+      if (!density && !T.kin_lines)
         group(P_PF, [&](const BoxDesc& b) { return fp64_fit_kin(b, ctx->plane_lds); }, T.pfg,
               T.nt_pfg, T.lds_pfg, T.shape_pfg, T.nthr_pfg, T.n_pfg, pf_off);
-      group(P_RP, [&](const BoxDesc& b) { return fp64_fit_pot(b, ctx->plane_lds); }, T.pbg,
+      if (!T.pot_lines)
+        group(P_RP, [&](const BoxDesc& b) { return fp64_fit_pot(b, ctx->plane_lds); }, T.pbg,
             T.nt_pbg, T.lds_pbg, T.shape_pbg, T.nthr_pbg, T.n_pbg, pb_off);
-      for (int k = 0; k < std::max(1, T.n_pbg) && force; ++k)
+      for (int k = 0; k < std::max(1, T.n_pbg) && force && !T.pot_lines; ++k)
         T.nthr_pbg[k] = force->nthr_rp[T.shape_pbg[k] - 1];
     } else if (T.plane && !density && ctx->plane_lds > 0) {
       auto fit = [&](size_t v) {
@@ -1209,11 +1233,20 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     got->zvalu = ml.zvalu;
     got->bvalu = ml.bvalu;
     got->plane = T.plane;
+    got->kin_lines = T.kin_lines;
+    got->pot_lines = T.pot_lines;
     got->xbig = xbig;
     got->zbig = zbig;
     for (int k = 0; k < std::max(1, T.n_pbg); ++k)
-      if (esz == 8 && T.plane) got->nthr_rp[T.shape_pbg[k] - 1] = T.nthr_pbg[k];
+      if (esz == 8 && T.plane && !T.pot_lines) got->nthr_rp[T.shape_pbg[k] - 1] = T.nthr_pbg[k];
     return BDFT_OK;  // choices only: nothing allocated
+  }
+  if (T.plane && T.pot_lines) {
+    long long run = 0;
+    for (BoxDesc& b : box) {
+      b.t2_off = run;
+      run += 2LL * b.N[1] * b.L[0] * b.L[2];
+    }
   }
   bdft_plan* plan = new bdft_plan();
   plan->ctx = ctx;
@@ -1275,7 +1308,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   const bool fp64_seq = T.plane && esz == 8;
   if (fp64_seq) {
     epass[0] = P_CZ;
-    epass[3] = P_RP;
+    epass[3] = T.pot_lines ? P_YL : P_RP;
   } else if (T.plane) {
     epass[0] = P_PF;
   }
@@ -1380,10 +1413,14 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   // workspace: W | K | T1 | T2 | T3
   if (T.plane || mfma) t1tot = 0;
   if (!zbig) t3tot = 0;
-  // (FP64 sequence: K | TZ, density: TZ)
+  // (FP64 sequence: K | TZ, on lines also TX in T2's place; density: TZ)
   long long wv = wtot, kv = wtot;
-  if (fp64_seq) wv = t2tot = t3tot = 0;
-  else tztot = 0;
+  if (fp64_seq) {
+    wv = t3tot = 0;
+    t2tot = T.pot_lines ? txtot : 0;
+  } else {
+    tztot = 0;
+  }
   if (fp64_seq && density) kv = 0;
   if (T.pc_plane) wv = t1tot = t2tot = t3tot = 0;   // preconditioner: K
   T.xbig = xbig;

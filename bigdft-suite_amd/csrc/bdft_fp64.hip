@@ -31,6 +31,7 @@
 #include <algorithm>
 
 #include "bdft_internal.h"
+#include "../../include/bigdft_hip.h"
 #include "bdft_stencil.h"
 
 namespace bdft {
@@ -63,41 +64,46 @@ struct RecElem {
   }
 };
 
-template <int NT>
+// AX = 1: the y lines of 16 coarse x of one coarse z instead, rows s2 N2 +
+// i2, lines col + CC (s1 + 2 s3).  lin0: linear index of the first column's
+// first point.
+template <int NT, int AX = 2>
 __device__ __forceinline__ void load_columns(double* lds, const BoxDesc& bd, const double* psi,
-                                             int q0, int nq) {
+                                             int first, int nq) {
   constexpr int ZS = NT / 128, UR = 8;
-  const int N3 = bd.N[2], npl = bd.N[0] * bd.N[1];
+  const int n = bd.N[AX], step = AX == 2 ? bd.N[0] * bd.N[1] : bd.N[0];
   const RecElem re(threadIdx.x & 127);
   const int z0 = threadIdx.x >> 7;
   const bool on = re.col < nq;
-  const int lin0 = q0 + (on ? re.col : 0);
+  const int lin0 = first + (on ? re.col : 0);
   const char* src = (const char*)(psi + bd.psi_off);
   const unsigned off = re.t == 0 ? 0u : 8u * (unsigned)(bd.nvctr_c + re.t - 1);
   const unsigned mul = re.t == 0 ? 8u : 56u;
-  double* dst = lds + (re.t >> 2) * N3 * NL + re.col + CC * (re.t & 3);
+  const int sec = AX == 2 ? re.t >> 2 : (re.t >> 1) & 1;
+  const int ln = AX == 2 ? re.t & 3 : (re.t & 1) + 2 * (re.t >> 2);
+  double* dst = lds + sec * n * NL + re.col + CC * ln;
   if (!bd.cinv && !bd.finv) {
-    for (int zb = z0; zb < N3; zb += ZS * UR) {
+    for (int zb = z0; zb < n; zb += ZS * UR) {
       double v[UR];
 #pragma unroll
       for (int u = 0; u < UR; ++u) {
-        const int z = min(zb + u * ZS, N3 - 1);
-        v[u] = *(const double*)(src + (off + mul * (unsigned)(lin0 + npl * z)));
+        const int z = min(zb + u * ZS, n - 1);
+        v[u] = *(const double*)(src + (off + mul * (unsigned)(lin0 + step * z)));
       }
 #pragma unroll
       for (int u = 0; u < UR; ++u)
-        if (zb + u * ZS < N3) dst[(zb + u * ZS) * NL] = on ? v[u] : 0.0;
+        if (zb + u * ZS < n) dst[(zb + u * ZS) * NL] = on ? v[u] : 0.0;
     }
   } else {
     const int* inv = re.t == 0 ? bd.cinv : bd.finv;
-    for (int zb = z0; zb < N3; zb += ZS * UR) {
+    for (int zb = z0; zb < n; zb += ZS * UR) {
       int r[UR];
       double v[UR];
 #pragma unroll
       for (int u = 0; u < UR; ++u) {
-        const int z = zb + u * ZS, lin = lin0 + npl * z;
+        const int z = zb + u * ZS, lin = lin0 + step * z;
         r[u] = -1;
-        if (on && z < N3) r[u] = inv ? inv[lin] : lin;
+        if (on && z < n) r[u] = inv ? inv[lin] : lin;
       }
 #pragma unroll
       for (int u = 0; u < UR; ++u) {
@@ -106,7 +112,7 @@ __device__ __forceinline__ void load_columns(double* lds, const BoxDesc& bd, con
       }
 #pragma unroll
       for (int u = 0; u < UR; ++u)
-        if (zb + u * ZS < N3) dst[(zb + u * ZS) * NL] = v[u];
+        if (zb + u * ZS < n) dst[(zb + u * ZS) * NL] = v[u];
     }
   }
 }
@@ -155,7 +161,7 @@ struct ColTile {
 // ---------------------------------------------------------------------------
 // TZ = G_z W
 // ---------------------------------------------------------------------------
-constexpr int ZG_NT = 256;
+template <int ZG_NT>
 __global__ __launch_bounds__(ZG_NT) void k_zgrow(Batch B, TileTable tt) {
   extern __shared__ __align__(16) unsigned char smem[];
   double* lds = (double*)smem;
@@ -923,6 +929,352 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
 }
 
 // ---------------------------------------------------------------------------
+// Boxes whose planes do not fit in LDS (beyond 70 periodic, 55 or 70 free
+// coarse points on x and y): the x and y passes on tiles of 64 lines, a lane
+// per line and a wave per chunk as in the z kernels.
+//   k_xlines_grow    TX = G_x TZ, TX[p3][p1][j2] (y fastest: the lanes' lines
+//                    j2 are neighbours, and the y lines are rows again)
+//   k_ylines_pot     TX <- G_y^T V G_y TX in place, epot partial
+//   k_xlines_shrink  TZ = G_x^T TX
+//   k_xlines_kin     K = K_x W,  k_ylines_kin  K += K_y W
+// Rows of memory go through LDS as columns of stride LR (odd: neither side
+// meets a bank twice).  77x93x131, 8 orbitals (60 M points): 0.21, 0.42, 0.22,
+// 0.30 and 0.36 ms, 16 to 24 B per point at 2.2 to 4.8 TB/s; the apply 2.34 ms,
+// 5.50 ms on the line passes of bdft_pass.hip.  Per point the planes move
+// less (20 ps, these 25), so boxes whose planes fit keep them.
+// Work-groups of 12 or 16 waves, two on a CU while the lines leave LDS and
+// registers for two; the outputs that replace a tile's inputs are held in
+// registers, MI chunks per wave (with 8 waves and five chunks each the three
+// code paths of every chunk did not fit the instruction cache: k_xlines_kin
+// 0.64 ms).
+// ---------------------------------------------------------------------------
+constexpr int LR = NL + 1;
+
+// nr rows of n values (n even, 16-byte aligned) <-> LDS [x LR + row]
+template <bool STORE>
+__device__ __forceinline__ void rows_move(double* lds, double* mem, int nr, int n) {
+  constexpr int UR = 4;
+  const int h = n >> 1, tot = nr * h, nt = blockDim.x;
+  double2* m2 = (double2*)mem;
+  ItDiv d(threadIdx.x, h, nt);
+  for (int i = threadIdx.x; i < tot; i += nt * UR) {
+    double2 v[UR];
+    if (!STORE) {
+#pragma unroll
+      for (int u = 0; u < UR; ++u) v[u] = m2[min(i + u * nt, tot - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      double* a = lds + 2 * d.j * LR + d.ch;
+      if (i + u * nt < tot) {
+        if (STORE) {
+          m2[i + u * nt] = make_double2(a[0], a[LR]);
+        } else {
+          a[0] = v[u].x;
+          a[LR] = v[u].y;
+        }
+      }
+      d.next(h);
+    }
+  }
+}
+
+template <int NTM, int WPE>
+__global__ __launch_bounds__(NTM, WPE) void k_xlines_grow(Batch B, TileTable tt) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  double* lds = (double*)smem;
+  const int tile = tile_of(tt);
+  const int b = find_box(tt, tile);
+  const BoxDesc bd = B.box[b];
+  const int N1 = bd.N[0], L1 = bd.L[0], L3 = bd.L[2], per = bd.per;
+  const int W1 = 2 * N1, W2 = 2 * bd.N[1];
+  const int r0 = (tile - box_first_tile(tt, b)) * NL, nr = min(NL, W2 * L3 - r0);
+  rows_move<false>(lds, (double*)B.TZ + bd.tz_off + (long long)r0 * W1, nr, W1);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, r = r0 + min(lane, nr - 1);
+  const int p3 = r / W2, j2 = r - p3 * W2;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double* out = (double*)B.T2 + bd.t2_off + (long long)p3 * L1 * W2 + j2;
+  const double *c = lds + lane, *d = c + N1 * LR;
+  for (int p0 = 8 * w; p0 < L1; p0 += 8 * (NTM / 64)) {
+    double o[8] = {};
+    line_taps<19>(grow_k0(p0, per), N1, per,
+                  [&](int kk, int k) { grow_tap(kk, c[k * LR], d[k * LR], o); });
+    if (lane < nr) {
+#pragma unroll
+      for (int h = 0; h < 8; ++h)
+        if (p0 + h < L1) out[(size_t)W2 * (unsigned)(p0 + h)] = o[h];
+    }
+  }
+}
+
+template <int NTM, int MI, int WPE>
+__global__ __launch_bounds__(NTM, WPE) void k_ylines_pot(Batch B, TileTable tt, double* part) {
+  constexpr int NW = NTM / 64;
+  extern __shared__ __align__(16) unsigned char smem[];
+  double* lds = (double*)smem;
+  __shared__ double red[NW];
+  const int tile = tile_of(tt);
+  const int b = find_box(tt, tile);
+  const BoxDesc bd = B.box[b];
+  const int L1 = bd.L[0], N2 = bd.N[1], L2 = bd.L[1], L3 = bd.L[2], per = bd.per;
+  const int W2 = 2 * N2;
+  const int r0 = (tile - box_first_tile(tt, b)) * NL, nr = min(NL, L1 * L3 - r0);
+  double* T = (double*)B.T2 + bd.t2_off + (long long)r0 * W2;
+  rows_move<false>(lds, T, nr, W2);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, r = r0 + min(lane, nr - 1);
+  const int p3 = r / L1, p1 = r - p3 * L1;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // (lanes past the tile walk its last line again and store nothing)
+  const bool on = lane < nr;
+  double* col = lds + min(lane, nr - 1);
+  // V outside the potential box is zero; lanes off it read a value of the box
+  // and discard it
+  const int q1 = p1 - bd.ishift[0], q3 = p3 - bd.ishift[2];
+  const bool in13 = on && q1 >= 0 && q1 < bd.potdim[0] && q3 >= 0 && q3 < bd.potdim[2];
+  const unsigned pd1 = (unsigned)bd.potdim[0], pd2 = (unsigned)bd.potdim[1];
+  const unsigned v0 = in13 ? (unsigned)q1 + pd1 * pd2 * (unsigned)q3 : 0u;
+  const double* pot = B.pot + bd.pot_off;
+  const double cxz = bd.conf_on ? conf_axis2(bd, 0, p1) + conf_axis2(bd, 2, p3) : 0.0;
+  double o[MI][8];
+  double ep = 0.0;
+#pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    const int p0 = 8 * (w + m * NW);
+    if (p0 < L2) {
+      double v[8];
+#pragma unroll
+      for (int h = 0; h < 8; ++h) {
+        const int q2 = p0 + h - bd.ishift[1];
+        v[h] = pot[v0 + pd1 * (unsigned)min(max(q2, 0), bd.potdim[1] - 1)];
+        o[m][h] = 0.0;
+      }
+      line_taps<19>(grow_k0(p0, per), N2, per, [&](int kk, int k) {
+        grow_tap(kk, col[k * LR], col[(N2 + k) * LR], o[m]);
+      });
+#pragma unroll
+      for (int h = 0; h < 8; ++h) {
+        const int q2 = p0 + h - bd.ishift[1];
+        const bool ok = in13 && p0 + h < L2 && q2 >= 0 && q2 < bd.potdim[1];
+        double vr = ok ? v[h] : 0.0;
+        if (bd.conf_on && ok) vr += conf_term(bd, cxz + conf_axis2(bd, 1, p0 + h));
+        const double vp = vr * o[m][h];
+        ep = fma(vp, o[m][h], ep);
+        o[m][h] = vp;
+      }
+    }
+  }
+  const double eps = block_sum_rt(ep, red);   // starts with a barrier
+  if (threadIdx.x == 0) part[tile] = eps;
+#pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    const int p0 = 8 * (w + m * NW);
+#pragma unroll
+    for (int h = 0; h < 8; ++h)
+      if (on && p0 + h < L2) col[(p0 + h) * LR] = o[m][h];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    const int i0 = 4 * (w + m * NW);
+#pragma unroll
+    for (int h = 0; h < 8; ++h) o[m][h] = 0.0;
+    if (i0 < N2)
+      line_taps<37>(per ? 2 * i0 - 14 : 2 * i0, L2, per, [&](int qq, int p) {
+        shrink_tap<double, 4>(qq, col[p * LR], o[m], o[m] + 4);
+      });
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    const int i0 = 4 * (w + m * NW);
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+      if (on && i0 + h < N2) {
+        col[(i0 + h) * LR] = o[m][h];
+        col[(N2 + i0 + h) * LR] = o[m][4 + h];
+      }
+  }
+  __syncthreads();
+  rows_move<true>(lds, T, nr, W2);
+}
+
+template <int NTM, int MI, int WPE>
+__global__ __launch_bounds__(NTM, WPE) void k_xlines_shrink(Batch B, TileTable tt) {
+  constexpr int NW = NTM / 64, UR = 8;
+  extern __shared__ __align__(16) unsigned char smem[];
+  double* lds = (double*)smem;
+  const int tile = tile_of(tt);
+  const int b = find_box(tt, tile);
+  const BoxDesc bd = B.box[b];
+  const int N1 = bd.N[0], L1 = bd.L[0], L3 = bd.L[2], per = bd.per;
+  const int W1 = 2 * N1, W2 = 2 * bd.N[1];
+  const int r0 = (tile - box_first_tile(tt, b)) * NL, nr = min(NL, W2 * L3 - r0);
+  const int lane = threadIdx.x & 63, r = r0 + min(lane, nr - 1);
+  const int p3 = r / W2, j2 = r - p3 * W2;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const double* src = (const double*)B.T2 + bd.t2_off + (long long)p3 * L1 * W2 + j2;
+  double* col = lds + lane;
+  for (int pb = w; pb < L1; pb += NW * UR) {
+    double v[UR];
+#pragma unroll
+    for (int u = 0; u < UR; ++u) v[u] = src[(size_t)W2 * (unsigned)min(pb + u * NW, L1 - 1)];
+#pragma unroll
+    for (int u = 0; u < UR; ++u)
+      if (pb + u * NW < L1) col[(pb + u * NW) * LR] = v[u];
+  }
+  __syncthreads();
+  double o[MI][8];
+#pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    const int i0 = 4 * (w + m * NW);
+#pragma unroll
+    for (int h = 0; h < 8; ++h) o[m][h] = 0.0;
+    if (i0 < N1)
+      line_taps<37>(per ? 2 * i0 - 14 : 2 * i0, L1, per, [&](int qq, int p) {
+        shrink_tap<double, 4>(qq, col[p * LR], o[m], o[m] + 4);
+      });
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    const int i0 = 4 * (w + m * NW);
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+      if (i0 + h < N1) {
+        col[(i0 + h) * LR] = o[m][h];
+        col[(N1 + i0 + h) * LR] = o[m][4 + h];
+      }
+  }
+  __syncthreads();
+  rows_move<true>(lds, (double*)B.TZ + bd.tz_off + (long long)r0 * W1, nr, W1);
+}
+
+// x lines of 16 rows q = i2 + N2 i3 of coarse points: line row + 16 (s2 + 2
+// s3), gathered a row per wave (its records are contiguous)
+template <int NTM, int MI, int WPE>
+__global__ __launch_bounds__(NTM, WPE) void k_xlines_kin(Batch B, TileTable tt) {
+  constexpr int NW = NTM / 64, UR = 8, ZS = NTM / 128;
+  extern __shared__ __align__(16) unsigned char smem[];
+  double* lds = (double*)smem;
+  const int tile = tile_of(tt);
+  const int b = find_box(tt, tile);
+  const BoxDesc bd = B.box[b];
+  const int N1 = bd.N[0], N2 = bd.N[1], N3 = bd.N[2], per = bd.per;
+  const int W1 = 2 * N1, W2 = 2 * N2;
+  const int q0 = (tile - box_first_tile(tt, b)) * CC, nq = min(CC, N2 * N3 - q0);
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // 128 threads per 16 records of a row, as load_columns
+  const RecElem re(threadIdx.x & 127);
+  const int z0 = threadIdx.x >> 7, nit = CC * ((N1 + CC - 1) / CC);
+  const char* src = (const char*)(B.psi + bd.psi_off);
+  const unsigned off = re.t == 0 ? 0u : 8u * (unsigned)(bd.nvctr_c + re.t - 1);
+  const unsigned mul = re.t == 0 ? 8u : 56u;
+  const int* inv = re.t == 0 ? bd.cinv : bd.finv;
+  double* dst = lds + (re.t & 1) * N1 * LR + CC * (re.t >> 1);
+  for (int ib = z0; ib < nit; ib += ZS * UR) {
+    double v[UR];
+    int r[UR];
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      const int it = ib + u * ZS, row = it & (CC - 1), x = (it & -CC) + re.col;
+      r[u] = -1;
+      if (row < nq && x < N1) {
+        const int lin = (q0 + row) * N1 + x;
+        r[u] = inv ? inv[lin] : lin;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < UR; ++u)
+      v[u] = r[u] >= 0 ? *(const double*)(src + (off + mul * (unsigned)r[u])) : 0.0;
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      const int it = ib + u * ZS, row = it & (CC - 1), x = (it & -CC) + re.col;
+      if (it < nit && x < N1) dst[x * LR + row] = v[u];
+    }
+  }
+  __syncthreads();
+  double* col = lds + lane;
+  const double ks = bd.kscale[0];
+  double o[MI][8];
+#pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    const int i0 = 4 * (w + m * NW);
+#pragma unroll
+    for (int h = 0; h < 8; ++h) o[m][h] = 0.0;
+    if (i0 < N1)
+      line_taps<32>(i0 - 14, N1, per, [&](int kk, int k) {
+        kin_tap(kk, col[k * LR], col[(N1 + k) * LR], o[m], o[m] + 4);
+      });
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < MI; ++m) {
+    const int i0 = 4 * (w + m * NW);
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+      if (i0 + h < N1) {
+        col[(i0 + h) * LR] = o[m][h] * ks;
+        col[(N1 + i0 + h) * LR] = o[m][4 + h] * ks;
+      }
+  }
+  __syncthreads();
+  for (int l = w; l < NL; l += NW) {
+    const int row = l & (CC - 1), s = l / CC, q = q0 + row;
+    if (row < nq) {
+      const int i3 = q / N2, i2 = q - i3 * N2;
+      double* k = (double*)B.K + bd.w_off +
+                  (long long)W1 * (i2 + N2 * (s & 1) + W2 * (i3 + N3 * (s >> 1)));
+      for (int x = lane; x < W1; x += 64) k[x] = lds[x * LR + l];
+    }
+  }
+}
+
+// y lines of 16 coarse x of one coarse z: line col + 16 (s1 + 2 s3)
+template <int NTM, int WPE>
+__global__ __launch_bounds__(NTM, WPE) void k_ylines_kin(Batch B, TileTable tt) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  double* lds = (double*)smem;
+  const int tile = tile_of(tt);
+  const int b = find_box(tt, tile);
+  const BoxDesc bd = B.box[b];
+  const int N1 = bd.N[0], N2 = bd.N[1], N3 = bd.N[2], per = bd.per;
+  const int W1 = 2 * N1, W2 = 2 * N2, nx = (N1 + CC - 1) / CC;
+  const int lt = tile - box_first_tile(tt, b), i3 = lt / nx, x0 = (lt - i3 * nx) * CC;
+  const int nq = min(CC, N1 - x0);
+  load_columns<NTM, 1>(lds, bd, B.psi, x0 + N1 * N2 * i3, nq);
+  __syncthreads();
+  const int lane = threadIdx.x & 63, cl = lane & (CC - 1), s = lane / CC;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool on = cl < nq;
+  double* K = (double*)B.K + bd.w_off + (x0 + (on ? cl : 0) + N1 * (s & 1)) +
+              (long long)W1 * W2 * (i3 + N3 * (s >> 1));
+  const double *c = lds + lane, *d = c + N2 * NL;
+  const double ks = bd.kscale[1];
+  for (int i0 = 4 * w; i0 < N2; i0 += 4 * (NTM / 64)) {
+    double k[8], o[8] = {};
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const int i = min(i0 + h, N2 - 1);
+      k[h] = K[W1 * i];
+      k[4 + h] = K[W1 * (N2 + i)];
+    }
+    line_taps<32>(i0 - 14, N2, per,
+                  [&](int kk, int i) { kin_tap(kk, c[i * NL], d[i * NL], o, o + 4); });
+    if (on) {
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+        if (i0 + h < N2) {
+          K[W1 * (i0 + h)] = fma(o[h], ks, k[h]);
+          K[W1 * (N2 + i0 + h)] = fma(o[4 + h], ks, k[4 + h]);
+        }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // density (local_partial_density, sumrho.f90:377-469): the planes p3 of TZ of
 // one group's orbitals (orbitals order[0 ..] of one spin, one box) in turn,
 // psir = G_y G_x, and sum hfac psir^2 kept in registers, written once as the
@@ -1018,6 +1370,22 @@ static PlaneFit plane_fit(size_t lds, int items, size_t plane_lds) {
   return {0, 0, lds};
 }
 static int chunks(int n, int len) { return (n + len - 1) / len; }
+// do the line kernels hold a box's x and y lines?
+static size_t lds_rows(int n) { return 8 * (size_t)LR * n; }
+bool fp64_kin_lines_ok(const BoxDesc& b, size_t plane_lds) {
+  return std::max(lds_rows(2 * b.N[0]), lds_w(b.N[1])) <= plane_lds;
+}
+// (K, TZ and TX of a flat free box can take more than the grids of the line
+// passes, by which the fixed device array's entry admits it: half that array
+// or the line passes' bytes bound them)
+bool fp64_pot_lines_ok(const BoxDesc& b, size_t plane_lds) {
+  const size_t n1 = 2 * b.N[0], n2 = 2 * b.N[1], n3 = 2 * b.N[2];
+  const size_t l1 = b.L[0], l2 = b.L[1], l3 = b.L[2];
+  return lds_rows(std::max(b.L[0], b.L[1])) + LDS_STATIC <= plane_lds &&
+         n1 * n2 * (n3 + l3) + n2 * l1 * l3 <=
+             std::max<size_t>(BDFT_FIXED_BYTES / 16,
+                              2 * n1 * n2 * n3 + l1 * n2 * n3 + l1 * l2 * n3);
+}
 PlaneFit fp64_fit_kin(const BoxDesc& b, size_t plane_lds) {
   const int N1 = b.N[0], N2 = b.N[1];
   return plane_fit(fp64_lds_kin(N1, N2),
@@ -1031,9 +1399,14 @@ PlaneFit fp64_fit_pot(const BoxDesc& b, size_t plane_lds) {
                    plane_lds);
 }
 
-static hipError_t launch_zgrow(const Batch& B, const TileTable& t, int ntiles, size_t lds,
+// 256 threads; more where long lines leave LDS for few work-groups per CU
+static hipError_t launch_zgrow(const Batch& B, const TileTable& t, int ntiles, int maxN3,
                                hipStream_t s) {
-  if (ntiles > 0) k_zgrow<<<ntiles, ZG_NT, lds, s>>>(B, t);
+  const size_t lds = lds_w(maxN3);
+  if (ntiles <= 0) return hipSuccess;
+  if (maxN3 <= 64) k_zgrow<256><<<ntiles, 256, lds, s>>>(B, t);
+  else if (maxN3 <= 80) k_zgrow<512><<<ntiles, 512, lds, s>>>(B, t);
+  else k_zgrow<1024><<<ntiles, 1024, lds, s>>>(B, t);
   return hipGetLastError();
 }
 static hipError_t launch_zback(const Batch& B, const TileTable& t, const TileTable& ft,
@@ -1077,6 +1450,29 @@ static hipError_t launch_xypot(const Batch& B, const TileTable& t, const TileTab
   return hipGetLastError();
 }
 
+// the x-y kinetic and potential passes of boxes whose planes do not fit
+static hipError_t kin_lines_pass(const Batch& B, const PassTables& PT, hipStream_t s) {
+  const size_t lx = lds_rows(2 * PT.maxN1), ly = lds_w(PT.maxN2);
+  const int nx = PT.ntiles[P_XK], ny = PT.ntiles[P_YK];
+  if (nx <= 0) return hipSuccess;
+  if (PT.maxN1 <= 96) k_xlines_kin<768, 2, 6><<<nx, 768, lx, s>>>(B, PT.t[P_XK]);
+  else k_xlines_kin<1024, 3, 4><<<nx, 1024, lx, s>>>(B, PT.t[P_XK]);
+  if (PT.maxN2 <= 80) k_ylines_kin<768, 6><<<ny, 768, ly, s>>>(B, PT.t[P_YK]);
+  else k_ylines_kin<1024, 4><<<ny, 1024, ly, s>>>(B, PT.t[P_YK]);
+  return hipGetLastError();
+}
+static hipError_t pot_lines_pass(const Batch& B, const PassTables& PT, hipStream_t s) {
+  const size_t lg = lds_rows(2 * PT.maxN1), ly = lds_rows(PT.maxL2), lx = lds_rows(PT.maxL1);
+  const int nx = PT.ntiles[P_XR], ny = PT.ntiles[P_YL];
+  if (nx <= 0) return hipSuccess;
+  k_xlines_grow<1024, 8><<<nx, 1024, lg, s>>>(B, PT.t[P_XR]);
+  if (PT.maxL2 <= 256) k_ylines_pot<1024, 2, 4><<<ny, 1024, ly, s>>>(B, PT.t[P_YL], PT.part[3]);
+  else k_ylines_pot<1024, 3, 4><<<ny, 1024, ly, s>>>(B, PT.t[P_YL], PT.part[3]);
+  if (PT.maxN1 <= 96) k_xlines_shrink<768, 2, 6><<<nx, 768, lx, s>>>(B, PT.t[P_XR]);
+  else k_xlines_shrink<1024, 3, 4><<<nx, 1024, lx, s>>>(B, PT.t[P_XR]);
+  return hipGetLastError();
+}
+
 // ev: null, or 2 S_COUNT events recorded before / after each stage
 hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
                            hipEvent_t* ev) {
@@ -1084,14 +1480,16 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
     if (ev) (void)hipEventRecord(ev[2 * stage + end], s);
   };
   mark(S_ZG, 0);
-  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], lds_w(PT.maxN3), s);
+  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], PT.maxN3, s);
   mark(S_ZG, 1);
   // one launch per group of boxes, or one over all of them
   mark(S_KXY, 0);
-  if (e == hipSuccess) e = xykin_pass<0>(B, PT, PcArgs{}, s);
+  if (e == hipSuccess)
+    e = PT.kin_lines ? kin_lines_pass(B, PT, s) : xykin_pass<0>(B, PT, PcArgs{}, s);
   mark(S_KXY, 1);
   mark(S_XYP, 0);
-  if (e == hipSuccess && PT.n_pbg == 0)
+  if (e == hipSuccess && PT.pot_lines) e = pot_lines_pass(B, PT, s);
+  else if (e == hipSuccess && PT.n_pbg == 0)
     e = launch_xypot(B, PT.t[P_RP], PT.t[P_RP], PT.ntiles[P_RP], PT.lds_pbg[0],
                      PT.nthr_pbg[0], PT.shape_pbg[0], PT.part[3], s);
   for (int k = 0; k < PT.n_pbg && e == hipSuccess; ++k)
@@ -1107,7 +1505,7 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
   EnergyTables et;
   et.t[0] = PT.t[P_CZ];
   et.p[0] = PT.part[0];
-  et.t[1] = PT.t[P_RP];
+  et.t[1] = PT.t[PT.pot_lines ? P_YL : P_RP];
   et.p[1] = PT.part[3];
   et.nk = 1;
   et.n = 2;
@@ -1124,7 +1522,7 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
 
 hipError_t launch_fp64_density(const Batch& B, const PassTables& PT, const DenArgs& D, int L3,
                                hipStream_t s) {
-  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], lds_w(PT.maxN3), s);
+  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], PT.maxN3, s);
   if (e != hipSuccess) return e;
   const int n = D.ngroups * L3;
   const size_t lds = PT.lds_pbg[0];
@@ -1153,7 +1551,13 @@ hipError_t launch_fp64_pc_apply(const Batch& B, const PassTables& PT, const PcAr
 
 // raise the dynamic-LDS limit of the kernels to lds bytes
 void fp64_attributes(size_t lds) {
-  const void* k[] = {(const void*)k_zgrow,         (const void*)k_zback<512, 1, 4>,
+  const void* k[] = {(const void*)k_zgrow<256>,      (const void*)k_zgrow<512>,
+                     (const void*)k_zgrow<1024>,     (const void*)k_xlines_grow<1024, 8>,
+                     (const void*)k_ylines_pot<1024, 2, 4>,  (const void*)k_ylines_pot<1024, 3, 4>,
+                     (const void*)k_xlines_shrink<768, 2, 6>,
+                     (const void*)k_xlines_shrink<1024, 3, 4>,
+                     (const void*)k_xlines_kin<768, 2, 6>, (const void*)k_xlines_kin<1024, 3, 4>,
+                     (const void*)k_ylines_kin<768, 6>, (const void*)k_ylines_kin<1024, 4>, (const void*)k_zback<512, 1, 4>,
                      (const void*)k_zback<768, 1, 6>,   (const void*)k_zback<512, 2, 4>,
                      (const void*)k_zback<1024, 3, 4>,
                      (const void*)k_xyden<512, 3, 4>, (const void*)k_xyden<S1_NT, 3, 4>,

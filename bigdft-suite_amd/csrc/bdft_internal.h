@@ -46,7 +46,8 @@ struct BoxDesc {
   double kscale[3];     // -1/2/h_d^2, coarse grid spacing
   long long w_off;      // offset of the wavelet volume (8 N1 N2 N3)
   long long t1_off;     // offset of (L1, 2N2, 2N3)
-  long long t2_off;     // offset of (L1, L2, 2N3)
+  long long t2_off;     // offset of (L1, L2, 2N3); FP64 sequence on lines: of
+                        // TX (2N2, L1, L3)
   long long tz_off;     // offset of (2N1, 2N2, L3) (FP64 sequence)
   long long t3_off;     // offset of the real volume (L1, L2, L3): z lines
                         // longer than 192 points only (k_zgrowpot)
@@ -401,9 +402,11 @@ __device__ __forceinline__ float t2_line_unscale(const Batch& B, const BoxDesc& 
 // lines as one run x + L1 y, 32 consecutive lines per tile (a tile may span
 // two rows), so that only a box's last tile is partly empty (k_zpot).
 // P_CZ: runs of CCOL coarse columns (z lines of the FP64 sequence); P_RP:
-// real-z planes of its potential pass.
+// real-z planes of its potential pass; where planes do not fit in LDS, P_XK:
+// runs of CCOL rows of coarse points (x lines), P_YK: CCOL coarse x of one
+// coarse z (y lines), P_XR: 64 x lines of TZ, P_YL: 64 y lines of (L1, L3).
 enum Pass { P_UNC = 0, P_XF, P_YF, P_KY, P_KZ, P_ZP, P_YB, P_XB, P_PF, P_PB, P_KZG, P_ZPG,
-            P_ZPF, P_CZ, P_RP, P_COUNT };
+            P_ZPF, P_CZ, P_RP, P_XK, P_YK, P_XR, P_YL, P_COUNT };
 constexpr int CCOL = 16;    // coarse columns (64 z lines) per P_CZ tile
 constexpr int ZGROUP = 3;   // bundles per z-line tile unless LDS asks for 2
 
@@ -442,7 +445,10 @@ struct PassTables {
   int n_pbg;
   // z-line kernels of the FP64 sequence: LDS and longest line of the batch
   size_t lds_cz;
-  int maxN3, maxL3;
+  int maxN1, maxN2, maxN3, maxL1, maxL2;
+  // FP64 sequence: x-y kinetic, potential pass on lines (some plane does not
+  // fit in LDS)
+  int kin_lines, pot_lines;
   // preconditioner: z lines and x-y planes of the compressed vectors
   // (bdft_fp64.hip) where every box fits, else the line passes
   int pc_plane;
@@ -607,6 +613,8 @@ struct PlaneFit {
 };
 PlaneFit fp64_fit_kin(const BoxDesc& b, size_t plane_lds);
 PlaneFit fp64_fit_pot(const BoxDesc& b, size_t plane_lds);
+bool fp64_kin_lines_ok(const BoxDesc& b, size_t plane_lds);
+bool fp64_pot_lines_ok(const BoxDesc& b, size_t plane_lds);
 void fp64_attributes(size_t lds);
 hipError_t launch_fp64_pc_apply(const Batch& B, const PassTables& PT, const PcArgs& P, int mode,
                                 hipStream_t s);

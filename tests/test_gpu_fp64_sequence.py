@@ -1,7 +1,7 @@
 """The FP64 plane-fused sequence (bdft_fp64.hip) against the oracle at the
 edges of its launch rules: extents where an in-plane work-group changes its
-shape (8, 12 or 16 waves, one or more per CU) or the planes stop fitting and
-the batch takes the line passes, z lines where the z kernels change their
+shape (8, 12 or 16 waves, one or more per CU), where the planes stop fitting
+and x and y go as tiles of 64 lines, where those lines stop fitting, z lines where the z kernels change their
 chunks per wave or stop fitting, and coarse planes that leave a partly empty
 last run of 16 columns.
 
@@ -34,6 +34,12 @@ def dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
+def lr_dims(reg):
+    """real-space grid points per axis"""
+    extra = 0 if reg.geocode == "P" else 29
+    return tuple(2 * (x + 1) + extra for x in reg.n)
+
+
 # n (coarse points - 1) per axis
 SIZES = [("P", n) for n in [
     (0, 0, 0), (15, 0, 4), (4, 3, 1), (7, 15, 2), (16, 16, 1),   # column runs, 4 waves
@@ -41,10 +47,12 @@ SIZES = [("P", n) for n in [
     (48, 48, 1), (49, 49, 1), (54, 55, 0),                       # half a CU's LDS, 12 waves
     (63, 63, 0), (69, 69, 0), (70, 70, 0), (84, 40, 0),          # 16 waves, beyond
     (1, 2, 31), (2, 1, 32), (1, 2, 47), (2, 1, 48), (1, 2, 63), (2, 1, 64),
-    (1, 0, 158), (0, 1, 159)]] + [("F", n) for n in [
+    (1, 0, 158), (0, 1, 159), (71, 70, 3), (127, 128, 0), (156, 90, 0), (90, 156, 0),
+    (157, 90, 0), (90, 157, 0)]] + [("F", n) for n in [
     (0, 0, 0), (4, 3, 1), (15, 16, 1), (20, 21, 0), (25, 26, 1),
     (35, 35, 0), (36, 36, 0), (40, 30, 1), (55, 55, 0), (56, 57, 0),
-    (1, 2, 31), (2, 1, 32), (1, 2, 48), (2, 1, 64), (1, 0, 144), (0, 1, 146)]]
+    (1, 2, 31), (2, 1, 32), (1, 2, 48), (2, 1, 64), (1, 0, 144), (0, 1, 146),
+    (57, 63, 2), (141, 60, 0), (60, 141, 0), (142, 60, 0), (60, 142, 0)]]
 
 
 @pytest.mark.parametrize("geo,n", SIZES, ids=[f"{g}{n[0]}x{n[1]}x{n[2]}" for g, n in SIZES])
@@ -78,6 +86,64 @@ def test_launch_edges_match_the_oracle(ctx, geo, n, keys):
         assert rel_err(h - h0, ho - h0) < TOL
     assert rel_err(ek.cpu().numpy(), eo) < TOL
     assert rel_err(ep.cpu().numpy(), po) < TOL
+
+
+def test_large_and_small_boxes_of_one_batch(ctx):
+    """boxes beyond LDS planes and small ones in one batch (all on x and y
+    lines): a potential box smaller than the grid and offset from it, and a
+    confining term, each against the oracle; the batch through the fixed
+    device array gives the same bits"""
+    import bigdft_hip
+    regs = [dense_region("P", (71, 72, 2), (0.45, 0.4, 0.5)),
+            dense_region("F", (5, 4, 3), (0.45, 0.4, 0.5)),
+            dense_region("P", (40, 90, 3), (0.45, 0.4, 0.5))]
+    psi = [random_psi(r, 1, 61 + i)[0] for i, r in enumerate(regs)]
+    dims = [lr_dims(r) for r in regs]
+    assert [r.n_isf for r in regs] == [int(np.prod(d)) for d in dims]
+    # potential boxes: four points less on x and y, offset by one and two
+    pots = [random_pot(r, 71 + i).reshape(d[::-1]) for i, (r, d) in enumerate(zip(regs, dims))]
+    sub = [np.ascontiguousarray(p[:, 2:-2, 1:-3]) for p in pots]
+    full = [np.zeros_like(p) for p in pots]
+    for a, b in zip(full, sub):
+        a[:, 2:-2, 1:-3] = b
+    lrs = [ctx.region(r) for r in regs]
+
+    def run(ps, conf=None, fixed=False, **kw):
+        off = np.cumsum([0] + [p.size for p in ps[:-1]])
+        po = np.cumsum([0] + [p.size for p in psi[:-1]])
+        x = dev(np.concatenate(psi))
+        h = torch.zeros_like(x)
+        ek = torch.zeros(3, dtype=torch.float64, device="cuda")
+        ep = torch.zeros_like(ek)
+        fn = ctx.locham_batch_fixed if fixed else ctx.locham_batch
+        if conf is not None:
+            kw["conf"] = conf
+        fn(lrs, dev(np.concatenate([p.ravel() for p in ps])), x, h, ek, ep, pot_off=off,
+           psi_off=po, **kw)
+        ctx.sync()
+        return np.split(h.cpu().numpy(), po[1:]), ek.cpu().numpy(), ep.cpu().numpy()
+
+    kw = dict(potdim=np.array([s.shape[::-1] for s in sub], dtype=np.int32).ravel(),
+              ishift=np.array([(1, 2, 0)] * 3, dtype=np.int32).ravel())
+    confs = [dict(args=(4, 1e-4, (0.2,) * 3, (3.0, 4.0, 1.0), (-1, -15, 2)[i:i + 1] * 3))
+             for i in range(3)]
+    gconf = np.concatenate([bigdft_hip.confpot(*c["args"]) for c in confs])
+    got = [run(sub, **kw), run(pots, conf=gconf)]
+    for g, ps, cf in ((got[0], full, None), (got[1], pots, confs)):
+        for i, r in enumerate(regs):
+            print(f"box {i} conf={cf is not None}", flush=True)
+            h, ek, ep = oracle.locham(r.geocode, r.n, r.nfl, r.nfu, r.hgrid, okeys(r),
+                                      ps[i].ravel(), psi[i][None],
+                                      conf=oracle.confpot(*cf[i]["args"]) if cf else None)
+            assert np.abs(g[0][i] - h[0]).max() < TOL * np.abs(h).max()
+            assert rel_err(g[1][i:i + 1], ek) < TOL
+            assert rel_err(g[2][i:i + 1], ep) < TOL
+    fx = run(sub, fixed=True, **kw)
+    for a, b in zip(fx[0], got[0][0]):
+        assert np.array_equal(a, b)
+    assert np.array_equal(fx[1], got[0][1]) and np.array_equal(fx[2], got[0][2])
+    for lr in lrs:
+        lr.close()
 
 
 # (geo, n, spins): one work-group shape each, groups of one spin that are
