@@ -2021,6 +2021,8 @@ static int xfer(bdft_ctx* ctx, const bdft_lr* glr, int norb, const bdft_lr* cons
     x.nvctr_f = L->nvctr_f;
     x.m1 = L->n[0] + 1;
     x.m2 = L->n[1] + 1;
+    xfer_magic(x.m1, x.q1, x.s1);
+    xfer_magic(x.m2, x.q2, x.s2);
     for (int k = 0; k < 3; ++k) x.ns[k] = ns[3 * i + k];
     const long long lnc = (long long)L->nvctr_c + 7LL * L->nvctr_f;
     if (to_local) {

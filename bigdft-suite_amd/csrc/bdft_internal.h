@@ -515,10 +515,24 @@ struct XferDesc {
   const int* fmap;
   int nvctr_c, nvctr_f;
   int m1, m2;           // local points per axis 1, 2 (n + 1)
+  unsigned q1, q2;      // division by m1, m2: n / m = umulhi(n, q) >> s
+  int s1, s2;           // (xfer_magic; q 0: m is 1)
   int ns[3];            // local box origin in the global box
-  long long loff, goff; // offsets of the local and global orbitals
   int tile0;
+  long long loff, goff; // offsets of the local and global orbitals
 };
+// n / m for 0 <= n < 2^31 as umulhi(n, q) >> s: q = floor(2^(31 + l) / m) + 1
+// with l = ceil(log2 m), s = l - 1 (q < 2^32; the error of q adds less than
+// n / 2^(31 + l) < 1 / m to the quotient).  m = 1: q = 0, n itself.
+inline void xfer_magic(int m, unsigned& q, int& s) {
+  q = 0;
+  s = 0;
+  if (m <= 1) return;
+  int l = 0;
+  while ((1LL << l) < m) ++l;
+  q = (unsigned)((1ULL << (31 + l)) / (unsigned)m + 1);
+  s = l - 1;
+}
 struct XferArgs {
   const XferDesc* d;
   int nd;

@@ -117,3 +117,39 @@ def test_transfers_sphere_batch_round_trip(ctx):
     for l in cache.values():
         l.close()
     g.close()
+
+
+@pytest.mark.parametrize("nl", [(0, 0, 0), (1, 0, 2), (2, 6, 0), (0, 7, 8), (8, 1, 6), (15, 16, 3),
+                                (16, 14, 17)], ids=lambda v: "x".join(map(str, v)))
+def test_transfers_box_extents(ctx, nl):
+    """local grids of one point, powers of two and their neighbours along x
+    and y (the split of a grid index), a tile's remainder in the coarse and
+    the fine part, a local box without fine points: bit-exact"""
+    from bigdft_hip.descriptors import dense_region, region_from_grids
+    h = (0.4, 0.4, 0.4)
+    ng = (19, 18, 20)
+    glob = dense_region("F", ng, h)
+    rng = np.random.default_rng(sum(nl) + 3)
+    cm = rng.random(tuple(x + 1 for x in nl)) < 0.7
+    cm[0, 0, 0] = True
+    locs = [dense_region("F", nl, h), region_from_grids("F", nl, h, cm, np.zeros_like(cm)),
+            region_from_grids("F", nl, h, cm, cm & (rng.random(cm.shape) < 0.5))]
+    ns = [[int(rng.integers(0, ng[d] - nl[d] + 1)) for d in range(3)] for _ in locs]
+    g, lrs = ctx.region(glob), [ctx.region(r) for r in locs]
+    gpsi = rng.standard_normal((3, glob.ncoef))
+    lnc = [r.ncoef for r in locs]
+    lp = torch.full((sum(lnc),), np.nan, dtype=torch.float64, device="cuda")
+    ctx.psi_to_locreg(g, lrs, np.array(ns, dtype=np.int32), dev(gpsi), lp)
+    base = rng.standard_normal((3, glob.ncoef))
+    back = dev(base)
+    ctx.locreg_to_psi(g, lrs, np.array(ns, dtype=np.int32), lp, back)
+    got = np.split(lp.cpu().numpy(), np.cumsum(lnc)[:-1])
+    for i, r in enumerate(locs):
+        exp = oracle.psi_to_locreg2(nl, ng, ns[i], okeys(r), okeys(glob), gpsi[i])
+        assert np.array_equal(got[i], exp)
+        full, n = oracle.lpsi_to_global2(nl, ng, ns[i], okeys(r), okeys(glob), exp, base[i])
+        assert n == r.nvctr_c + r.nvctr_f
+        assert np.array_equal(back[i].cpu().numpy(), full)
+    for lr in lrs:
+        lr.close()
+    g.close()
