@@ -755,10 +755,17 @@ struct Plane {
       if (!sq) build_maps(my, sy, N2, threadIdx.x, blockDim.x);
     }
   }
-  // the thread's items, opaque: in a loop over planes, addresses and line-end
-  // masks made from them stay inside it (moved out, they spill)
+  // the thread's items, opaque: addresses and line-end masks made from them
+  // are neither moved out of a loop over planes nor shared between passes
+  // (either way they spill; a kernel that uses scratch memory starts 0.13 ms
+  // late on a queue that has run none: the first apply on a new stream of one
+  // 16^3 orbital took 0.32 to 0.45 ms in place of 0.20)
   __device__ __forceinline__ void opaque() {
-    asm volatile("" : "+v"(dn.ch), "+v"(dn.j), "+v"(dw.ch), "+v"(dw.j), "+v"(dl.ch), "+v"(dl.j));
+    asm volatile("" : "+v"(dn.ch), "+v"(dn.j));
+    opaque_xy();
+  }
+  __device__ __forceinline__ void opaque_xy() {
+    asm volatile("" : "+v"(dw.ch), "+v"(dw.j), "+v"(dl.ch), "+v"(dl.j));
   }
   // T's plane into the x rows, two values at a time (rows of 2 N1, planes of
   // 4 N1 N2 values: 16-byte aligned)
@@ -819,7 +826,7 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
   const int b = table_box(tt, lb);
   const BoxDesc bd = B.box[b];
   const int p3 = tile - box_first_tile(tt, lb);
-  const Plane P(bd, smem);
+  Plane P(bd, smem);
   const int N1 = P.N1, N2 = P.N2, L1 = P.L1, L2 = P.L2, per = P.per;
   const int W2 = P.W2, RX = P.RX, RY = P.RY;
   double* A = P.A;
@@ -827,7 +834,7 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
   P.load(T);
   double o[MI][8];
   P.grow_x<MI>(o);
-  const ItDiv dw = P.dw, dl = P.dl;
+  P.opaque_xy();
   const int gy = (L2 + 7) >> 3;
   // G_y and V on the rows p1.  V outside the potential box is zero, the
   // zeroing of psir there (potential.f90:874-947); those points read a value
@@ -841,7 +848,7 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
                           (unsigned)min(max(q3, 0), bd.potdim[2] - 1);
   const double cz = bd.conf_on ? conf_axis2(bd, 2, p3) : 0.0;
   double ep = 0.0;
-  each_item<MI>(dl, L1, gy, [&](int m, int ch, int p1) {
+  each_item<MI>(P.dl, L1, gy, [&](int m, int ch, int p1) {
     const int q1 = p1 - bd.ishift[0], q20 = 8 * ch - bd.ishift[1];
     // rows of the chunk inside the box and the potential box
     const bool in13 = in3 && q1 >= 0 && q1 < bd.potdim[0];
@@ -877,20 +884,21 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
     }
   });
   __syncthreads();
-  each_item<MI>(dl, L1, gy, [&](int m, int ch, int p1) {
+  each_item<MI>(P.dl, L1, gy, [&](int m, int ch, int p1) {
     double* a = A + p1 * RY + 8 * ch;
 #pragma unroll
     for (int r = 0; r < 8; ++r)
       if (8 * ch + r < L2) a[r] = o[m][r];
   });
   __syncthreads();
+  P.opaque_xy();
   // G_y^T on the rows p1, written as columns of the x rows
   const int cy = (N2 + 3) >> 2, cx = (N1 + 3) >> 2;
-  each_item<MI>(dl, L1, cy, [&](int m, int ch, int p1) {
+  each_item<MI>(P.dl, L1, cy, [&](int m, int ch, int p1) {
     shrink_row(A + p1 * RY, P.sy, L2, 4 * ch, per, o[m]);
   });
   __syncthreads();
-  each_item<MI>(dl, L1, cy, [&](int m, int ch, int p1) {
+  each_item<MI>(P.dl, L1, cy, [&](int m, int ch, int p1) {
     double* a = A + 4 * ch * RX + p1;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -900,12 +908,13 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
       }
   });
   __syncthreads();
+  P.opaque_xy();
   // G_x^T on the rows j2
-  each_item<MI>(dw, W2, cx, [&](int m, int ch, int j2) {
+  each_item<MI>(P.dw, W2, cx, [&](int m, int ch, int j2) {
     shrink_row(A + j2 * RX, P.sx, L1, 4 * ch, per, o[m]);
   });
   __syncthreads();
-  each_item<MI>(dw, W2, cx, [&](int m, int ch, int j2) {
+  each_item<MI>(P.dw, W2, cx, [&](int m, int ch, int j2) {
     double* a = A + j2 * RX + 4 * ch;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -919,8 +928,10 @@ __global__ __launch_bounds__(NTM, WPE) void k_xypot(Batch B, TileTable tt, TileT
   {
     const int tot = N1 * W2;
     double2* dst = (double2*)T;
-    ItDiv d = P.dn;
-    for (int i = threadIdx.x; i < tot; i += (int)blockDim.x) {
+    int tid = threadIdx.x;   // opaque: counted anew, not held through the passes
+    asm volatile("" : "+v"(tid));
+    ItDiv d(tid, N1, blockDim.x);
+    for (int i = tid; i < tot; i += (int)blockDim.x) {
       const double* a = A + d.ch * RX + 2 * d.j;
       dst[i] = make_double2(a[0], a[1]);
       d.next(N1);

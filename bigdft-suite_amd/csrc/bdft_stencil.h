@@ -20,7 +20,7 @@ struct ItDiv {
   __device__ __forceinline__ ItDiv(int tid, int n, int step) {
     ch = tid / n;
     j = tid - ch * n;
-    dch = step / n;
+    dch = __builtin_amdgcn_readfirstlane(step / n);   // n, step: the same in all threads
     dj = step - dch * n;
   }
   __device__ __forceinline__ void next(int n) {
