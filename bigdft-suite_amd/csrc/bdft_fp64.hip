@@ -162,10 +162,9 @@ struct ColTile {
 // TZ = G_z W
 // ---------------------------------------------------------------------------
 template <int ZG_NT>
-__global__ __launch_bounds__(ZG_NT) void k_zgrow(Batch B, TileTable tt) {
-  extern __shared__ __align__(16) unsigned char smem[];
+__device__ __forceinline__ void zgrow_tile(const Batch& B, const TileTable& tt, int tile,
+                                           unsigned char* smem) {
   double* lds = (double*)smem;
-  const int tile = tile_of(tt);
   const int lb = find_box(tt, tile);
   const BoxDesc bd = B.box[table_box(tt, lb)];
   const int N3 = bd.N[2], L3 = bd.L[2], per = bd.per;
@@ -190,6 +189,11 @@ __global__ __launch_bounds__(ZG_NT) void k_zgrow(Batch B, TileTable tt) {
         if (p0 + r < L3) q[ps * r] = o[r];
     }
   }
+}
+template <int ZG_NT>
+__global__ __launch_bounds__(ZG_NT) void k_zgrow(Batch B, TileTable tt) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  zgrow_tile<ZG_NT>(B, tt, tile_of(tt), smem);
 }
 
 // ---------------------------------------------------------------------------
@@ -563,11 +567,10 @@ __device__ __forceinline__ void each_item(ItDiv d, int n, int nch, F f) {
 // goes to the compressed vectors.  1, v = x: r = b - A x, d = r, partial
 // |r|^2; 2, v = d: q = A d, partial q d.
 // ---------------------------------------------------------------------------
-template <int NTM, int MI, int WPE, int PC = 0>
-__global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt, TileTable ft,
-                                                    PcArgs P) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int tile = tile_of(tt);
+template <int NTM, int MI, int PC>
+__device__ __forceinline__ void xykin_tile(const Batch& B, const TileTable& tt,
+                                           const TileTable& ft, const PcArgs& P, int tile,
+                                           unsigned char* smem) {
   const int lb = find_box(tt, tile);
   const int b = table_box(tt, lb);
   const BoxDesc bd = B.box[b];
@@ -728,6 +731,26 @@ __global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt, TileT
       d.next(N1);
     }
   }
+}
+
+template <int NTM, int MI, int WPE, int PC = 0>
+__global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt, TileTable ft,
+                                                    PcArgs P) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  xykin_tile<NTM, MI, PC>(B, tt, ft, P, tile_of(tt), smem);
+}
+
+// Both kernels that read psi alone in one launch: nx planes of k_xykin, then
+// the tiles of k_zgrow.
+template <int NTM>
+__global__ __launch_bounds__(NTM, 6) void k_zgrow_xykin(Batch B, TileTable tz, TileTable tx,
+                                                        int nx) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int b = blockIdx.x;
+  if (b < nx)
+    xykin_tile<NTM, 2, 0>(B, tx, tx, PcArgs{}, tx.xcd ? xcd_tile(b, nx) : b, smem);
+  else
+    zgrow_tile<NTM>(B, tz, tz.xcd ? xcd_tile(b - nx, gridDim.x - nx) : b - nx, smem);
 }
 
 // ---------------------------------------------------------------------------
@@ -1490,14 +1513,34 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
   auto mark = [&](int stage, int end) {
     if (ev) (void)hipEventRecord(ev[2 * stage + end], s);
   };
-  mark(S_ZG, 0);
-  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], PT.maxN3, s);
-  mark(S_ZG, 1);
-  // one launch per group of boxes, or one over all of them
-  mark(S_KXY, 0);
-  if (e == hipSuccess)
-    e = PT.kin_lines ? kin_lines_pass(B, PT, s) : xykin_pass<0>(B, PT, PcArgs{}, s);
-  mark(S_KXY, 1);
+  hipError_t e = hipSuccess;
+  // k_zgrow and k_xykin share a launch, unless stages are timed: it saves a
+  // launch and the first kernel's last, partly empty wave of work-groups, 6 to
+  // 10 us for one orbital of 16^3 to 40^3 (60 of 66, 84 of 94 us), 15 to 25 us
+  // for ten to sixty (32^3 x 60: 420 of 445 us; 40^3 x 40: 584 of 607).  From
+  // ZX_MAX work-groups on the gain is lost in the mix of two kinds of
+  // work-group on a CU (32^3 x 300: 1.955 of 1.960 ms, 40^3 x 128: 1.760 of
+  // 1.745).
+  constexpr int ZX_MAX = 16384;
+  const int nz = PT.ntiles[P_CZ], nx = PT.ntiles[P_PF];
+  if (!ev && !PT.kin_lines && PT.n_pfg == 0 && PT.shape_pfg[0] >= 2 && nz + nx <= ZX_MAX) {
+    const size_t lds = std::max(lds_w(PT.maxN3), PT.lds_pfg[0]);
+    const TileTable &tz = PT.t[P_CZ], &tx = PT.t[P_PF];
+    if (nz + nx <= 0) return hipSuccess;
+    if (PT.nthr_pfg[0] <= 256) k_zgrow_xykin<256><<<nz + nx, 256, lds, s>>>(B, tz, tx, nx);
+    else if (PT.nthr_pfg[0] <= 512) k_zgrow_xykin<512><<<nz + nx, 512, lds, s>>>(B, tz, tx, nx);
+    else k_zgrow_xykin<S2_NT><<<nz + nx, S2_NT, lds, s>>>(B, tz, tx, nx);
+    e = hipGetLastError();
+  } else {
+    mark(S_ZG, 0);
+    e = launch_zgrow(B, PT.t[P_CZ], nz, PT.maxN3, s);
+    mark(S_ZG, 1);
+    // one launch per group of boxes, or one over all of them
+    mark(S_KXY, 0);
+    if (e == hipSuccess)
+      e = PT.kin_lines ? kin_lines_pass(B, PT, s) : xykin_pass<0>(B, PT, PcArgs{}, s);
+    mark(S_KXY, 1);
+  }
   mark(S_XYP, 0);
   if (e == hipSuccess && PT.pot_lines) e = pot_lines_pass(B, PT, s);
   else if (e == hipSuccess && PT.n_pbg == 0)
@@ -1563,7 +1606,9 @@ hipError_t launch_fp64_pc_apply(const Batch& B, const PassTables& PT, const PcAr
 // raise the dynamic-LDS limit of the kernels to lds bytes
 void fp64_attributes(size_t lds) {
   const void* k[] = {(const void*)k_zgrow<256>,      (const void*)k_zgrow<512>,
-                     (const void*)k_zgrow<1024>,     (const void*)k_xlines_grow<1024, 8>,
+                     (const void*)k_zgrow<1024>,     (const void*)k_zgrow_xykin<256>,
+                     (const void*)k_zgrow_xykin<512>, (const void*)k_zgrow_xykin<S2_NT>,
+                     (const void*)k_xlines_grow<1024, 8>,
                      (const void*)k_ylines_pot<1024, 2, 4>,  (const void*)k_ylines_pot<1024, 3, 4>,
                      (const void*)k_xlines_shrink<768, 2, 6>,
                      (const void*)k_xlines_shrink<1024, 3, 4>,

@@ -201,3 +201,38 @@ def test_precond_launch_edges_match_the_oracle(ctx, geo, n, keys):
     for i in range(2):
         want = oracle.precond_cg(geo, reg.n, reg.hgrid, cpr[i], 3, okeys(reg), x0[i], b[i])
         assert np.abs(got[i] - want).max() < 1e-10 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("geo,n,norb", [("P", (0, 0, 0), 1), ("P", (15, 15, 15), 1),
+                                        ("P", (22, 20, 21), 6), ("P", (31, 31, 3), 5),
+                                        ("P", (32, 31, 9), 2), ("P", (40, 44, 2), 2),
+                                        ("P", (54, 53, 1), 1), ("P", (55, 54, 1), 1),
+                                        ("P", (3, 3, 0), 5461), ("P", (3, 3, 0), 5462),
+                                        ("F", (3, 2, 47), 2), ("F", (9, 8, 7), 11)],
+                         ids=lambda v: v if isinstance(v, str) else str(v).replace(", ", "x"))
+def test_small_batches_share_the_first_launch(ctx, geo, n, norb):
+    """small batches run G_z and the x-y kinetic in one launch of 256, 512 or
+    768 threads, up to 16384 work-groups (5461 of the three of a 4x4x1 box);
+    with stage timing on every kernel has its own: the same sums in the same
+    order, so the same bits"""
+    reg = dense_region(geo, n, (0.45, 0.4, 0.5))
+    print(f"case {geo} n={n} norb={norb}", flush=True)
+    psi, pot, lr = dev(random_psi(reg, norb, 81)), dev(random_pot(reg, 82)), ctx.region(reg)
+
+    def run():
+        h = torch.zeros_like(psi)
+        ek = torch.zeros(norb, dtype=torch.float64, device="cuda")
+        ep = torch.zeros_like(ek)
+        ctx.locham(lr, pot, psi, h, ek, ep)
+        ctx.sync()
+        return h, ek, ep
+    one = run()
+    ctx.profile(True)
+    try:
+        each = run()
+    finally:
+        ctx.profile_read()
+        ctx.profile(False)
+    lr.close()
+    for a, b in zip(one, each):
+        assert torch.equal(a, b)
