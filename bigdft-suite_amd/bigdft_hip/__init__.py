@@ -207,20 +207,26 @@ class LocReg:
             pass
 
 
-def _stream_ordered(method):
+def _stream_ordered(method, complete=False):
     """Device-array entry points run on the context's stream: it first waits
     for the work already queued on torch's current stream (tensors the
     caller just allocated or filled), and torch's current stream then waits
-    for the call, so results read through torch see it complete."""
+    for the call, so results read through torch see it complete (complete:
+    the library has waited for it by the time it returns)."""
     def wrapped(self, *args, **kwargs):
         ctx = self if isinstance(self, Context) else self.ctx
         ctx._enter()
         try:
             return method(self, *args, **kwargs)
         finally:
-            ctx._leave()
+            if not complete:
+                ctx._leave()
     wrapped.__name__, wrapped.__doc__ = method.__name__, method.__doc__
     return wrapped
+
+
+def _stream_ordered_complete(method):
+    return _stream_ordered(method, complete=True)
 
 
 class Plan:
@@ -419,7 +425,7 @@ class Context:
             None if sp is None else sp.ctypes.data_as(ctypes.c_void_p),
             nspin, _dev(rho, "rho", int(np.prod(lr.region.nfine)) * nspin), precision))
 
-    @_stream_ordered
+    @_stream_ordered_complete
     def _xfer(self, fn, glr, llrs, ns, src, soff, dst, doff):
         arr = (ctypes.c_void_p * len(llrs))(*[l.handle.value for l in llrs])
         nsa = np.ascontiguousarray(ns, dtype=np.int32).ravel()

@@ -540,6 +540,7 @@ struct XferArgs {
   const int* gfinv;
   int g1, g2, g3;       // global points per axis
   int gnvctr_c;
+  int* flag;            // host memory: set to 1 where a point is missing
   const double* src;
   double* dst;
   int to_local;         // 1: local = global(map), 0: global(map) = local

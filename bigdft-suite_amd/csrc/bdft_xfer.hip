@@ -77,7 +77,10 @@ __device__ __forceinline__ void xfer_tile(const XferArgs& A, const XferDesc& D, 
     if (e >= ne) continue;
     if (A.to_local) dst[lb + e] = v[u];
     else if (gi[u] >= 0) dst[gb + (FINE ? 7LL * gi[u] + t : gi[u])] = v[u];
-    else if (t == 0) atomicAdd(A.miss, 1);   // once per point
+    else if (t == 0) {   // once per point
+      atomicAdd(A.miss, 1);
+      __hip_atomic_store(A.flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
 }
 

@@ -153,3 +153,36 @@ def test_transfers_box_extents(ctx, nl):
     for lr in lrs:
         lr.close()
     g.close()
+
+
+def test_missing_points_are_counted_on_every_call(ctx):
+    """the count of points without a counterpart is that of the one call:
+    failing, good and failing calls in turn, on one batch and on another"""
+    import bigdft_hip
+    from bigdft_hip.descriptors import dense_region, region_from_grids
+    h = (0.4, 0.4, 0.4)
+    full = np.ones((9, 8, 7), dtype=bool)
+    holes = full.copy()
+    holes[2:4, 3, 1:6] = False
+    glob = region_from_grids("F", (8, 7, 6), h, holes, np.zeros_like(full))
+    g = ctx.region(glob)
+    small, big = dense_region("F", (1, 1, 1), h), dense_region("F", (8, 7, 6), h)
+    for loc, ns, missing in [(big, (0, 0, 0), (9 * 8 * 7 * 2) - glob.nvctr_c),
+                             (small, (2, 3, 1), 12), (big, (0, 0, 0), 9 * 8 * 7 * 2 - glob.nvctr_c)]:
+        lr = ctx.region(loc)
+        lp = dev(np.ones(loc.ncoef))
+        out = torch.zeros(glob.ncoef, dtype=torch.float64, device="cuda")
+        for _ in range(2):
+            with pytest.raises(bigdft_hip.BigDFTError, match=f"{missing} local points"):
+                ctx.locreg_to_psi(g, [lr], np.array(ns, dtype=np.int32), lp, out)
+            # to the local region the missing points are zeros, not an error
+            ctx.psi_to_locreg(g, [lr], np.array(ns, dtype=np.int32), out, lp)
+            lp.fill_(1.0)
+        lr.close()
+    ok = region_from_grids("F", (8, 7, 6), h, holes, np.zeros_like(full))
+    lr = ctx.region(ok)
+    out = torch.zeros(glob.ncoef, dtype=torch.float64, device="cuda")
+    ctx.locreg_to_psi(g, [lr], np.zeros(3, dtype=np.int32), dev(np.ones(ok.ncoef)), out)
+    assert torch.equal(out, torch.ones_like(out))
+    lr.close()
+    g.close()
