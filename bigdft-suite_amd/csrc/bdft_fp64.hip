@@ -141,6 +141,44 @@ __device__ __forceinline__ void line_taps(int k0, int n, int per, F tap) {
   }
 }
 
+// The 32 taps of a kinetic chunk from both ends inwards: tap 31 - kk has the
+// mirror of tap kk's coefficients (the filters are symmetric or each other's
+// mirror), so each pair shares its constants.  In ascending order they stay
+// live from one half to the other, more than the scalar registers hold, and
+// a tenth of the vector instructions are their spills.
+template <typename F>
+__device__ __forceinline__ void kin_order(F tap) {
+#pragma unroll
+  for (int kk = 0; kk < 16; ++kk) {
+    tap(kk);
+    tap(31 - kk);
+  }
+}
+// ... on a line of n values from k0 (as line_taps)
+template <typename F>
+__device__ __forceinline__ void kin_taps(int k0, int n, int per, F tap) {
+  if (k0 >= 0 && k0 + 32 <= n) {
+    kin_order([&](int kk) { tap(kk, k0 + kk); });
+  } else if (per) {
+    int ka = k0, kb = k0 + 31;
+    while (ka < 0) ka += n;
+    while (ka >= n) ka -= n;
+    while (kb < 0) kb += n;
+    while (kb >= n) kb -= n;
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk) {
+      tap(kk, ka);
+      tap(31 - kk, kb);
+      ka = ka + 1 == n ? 0 : ka + 1;
+      kb = kb == 0 ? n - 1 : kb - 1;
+    }
+  } else {
+    kin_order([&](int kk) {
+      if (k0 + kk >= 0 && k0 + kk < n) tap(kk, k0 + kk);
+    });
+  }
+}
+
 // a tile's lines: first column, columns, and this lane's line
 struct ColTile {
   int q0, nq;
@@ -254,7 +292,7 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
         if (m > 0) load_k(i0, k);
 #pragma unroll
         for (int r = 0; r < 8; ++r) o[m][r] = 0.0;
-        line_taps<32>(i0 - 14, N3, per, [&](int kk, int z) {
+        kin_taps(i0 - 14, N3, per, [&](int kk, int z) {
           kin_tap(kk, c[z * NL], d[z * NL], o[m], o[m] + 4);
         });
 #pragma unroll
@@ -418,7 +456,7 @@ __global__ __launch_bounds__(PZ_NT, 6) void k_pcz(Batch B, TileTable tt, PcArgs 
     double o[8];
 #pragma unroll
     for (int h = 0; h < 8; ++h) o[h] = 0.0;
-    line_taps<32>(i0 - 14, N3, per,
+    kin_taps(i0 - 14, N3, per,
                   [&](int kk, int z) { kin_tap(kk, c[z * NL], d[z * NL], o, o + 4); });
     if (ct.on) {
 #pragma unroll
@@ -495,20 +533,6 @@ __device__ __forceinline__ void grow_row(const double* ln, const int2* m, int N,
       [&](int kk, double2 x) { grow_tap(kk, x.x, x.y, o); });
 }
 
-// wavelet-basis kinetic (unscaled) of a wavelet row: coarse outputs i0 .. i0
-// + 3 (c in o[0..3], d in o[4..7])
-__device__ __forceinline__ void kin_row(const double* ln, const int2* m, int N, int i0, int per,
-                                        double o[8]) {
-#pragma unroll
-  for (int r = 0; r < 8; ++r) o[r] = 0.0;
-  const double *c = ln + i0 - 14, *d = ln + N + i0 - 14;
-  const int2* mm = m + (i0 - 14 + MOFF);
-  row_taps<32>(
-      i0 - 14, N, per, [&](int kk) { return make_double2(c[kk], d[kk]); },
-      [&](int kk) { return at2(ln, mm[kk]); },
-      [&](int kk, double2 x) { kin_tap(kk, x.x, x.y, o, o + 4); });
-}
-
 // G^T of a fine row of L values: coarse outputs i0 .. i0 + 3; m: fine line
 // map (periodic)
 __device__ __forceinline__ void shrink_row(const double* ln, const int* m, int L, int i0,
@@ -559,15 +583,85 @@ __device__ __forceinline__ void each_item(ItDiv d, int n, int nch, F f) {
 // ---------------------------------------------------------------------------
 // K = K_x W + K_y W of one x-y plane (wavelet z index i3 + N3 s3; the two
 // planes of a coarse z are neighbouring tiles: they read the same fine
-// records).  K_y, along the columns, goes to memory first; K_x goes over the
-// plane in LDS and from there is added to it.
+// records).
+//
+// Eight lanes take the 64 values of a 4 x 4 block of coarse points: for K_x
+// a lane per row (o, s2), its results the eight columns (o1, s1); for K_y a
+// lane per column, its results the eight rows.  An 8 x 8 transposition between
+// lanes and registers brings K_x into K_y's layout and the sum goes to memory
+// once, 16 neighbouring columns per half-row of lanes.  The plane in LDS is
+// only read, so its one barrier is after the load, and K makes no second trip:
+// K_y written, read back and added to K_x moved 32 B per point in place of 16
+// (50 in place of 34 with PC), at 4.2 to 4.8 TB/s.  40^3 x 128 (65 M points):
+// 0.50 -> 0.47 ms, 64^3 x 48: 0.96 -> 0.80, PC 2 of 48^3 x 64: 0.63 -> 0.53;
+// bound by the vector units, three quarters of whose instructions are the
+// stencils.
+//
+// LDS: rows j2, c and d of a coarse x side by side (one 16-byte read per tap
+// of K_x), a stride of an odd number of such pairs.  Lane bits: o 0-1, s 4,
+// blocks 2, 3, 5: 16 lanes of K_x read four rows of four neighbouring blocks,
+// 32 lanes of K_y 32 neighbouring values, all in distinct banks.
 //
 // PC: the last half of the preconditioner's A v = S (K + c) S v, W = S v of
 // the compressed vector v and c W + K_z W in K (k_pcz): S (K + K_x W + K_y W)
 // goes to the compressed vectors.  1, v = x: r = b - A x, d = r, partial
-// |r|^2; 2, v = d: q = A d, partial q d.
+// |r|^2; 2, v = d: q = A d, partial q d = (K + K_x W + K_y W) W.
 // ---------------------------------------------------------------------------
-template <int NTM, int MI, int PC>
+__host__ __device__ constexpr int pair_stride(int N) { return 2 * ((N + 1) | 1); }
+
+// register pair (a, b) <-> lane bit 0 or 1 (CTRL: the quad_perm of that
+// exchange), bit: this lane's value of it
+template <int CTRL>
+__device__ __forceinline__ unsigned quad_lane(unsigned x) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ void swap_quad(double& a, double& b, bool bit) {
+  const uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
+  // every lane takes part in the exchange, then chooses
+  const uint2 u = make_uint2(quad_lane<CTRL>(x.x), quad_lane<CTRL>(x.y));
+  const uint2 w = make_uint2(quad_lane<CTRL>(y.x), quad_lane<CTRL>(y.y));
+  const uint2 p = make_uint2(bit ? w.x : x.x, bit ? w.y : x.y);
+  const uint2 q = make_uint2(bit ? y.x : u.x, bit ? y.y : u.y);
+  a = __builtin_bit_cast(double, p);
+  b = __builtin_bit_cast(double, q);
+}
+// ... <-> lane bit 4
+__device__ __forceinline__ void swap_row16(double& a, double& b) {
+  const uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
+  const auto lo = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+  a = __builtin_bit_cast(double, make_uint2(lo[0], hi[0]));
+  b = __builtin_bit_cast(double, make_uint2(lo[1], hi[1]));
+}
+// v[4 s + o] of lane (s', o') <-> v[4 s' + o'] of lane (s, o)
+__device__ __forceinline__ void transpose8(double v[8]) {
+  const bool o0 = threadIdx.x & 1, o1 = threadIdx.x & 2;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) swap_row16(v[r], v[4 + r]);
+#pragma unroll
+  for (int r = 0; r < 8; r += 2) swap_quad<0xb1>(v[r], v[r + 1], o0);
+#pragma unroll
+  for (int r = 0; r < 8; r += 4) {
+    swap_quad<0x4e>(v[r], v[r + 2], o1);
+    swap_quad<0x4e>(v[r + 1], v[r + 3], o1);
+  }
+}
+
+// Component t = s1 + 2 s2 + 4 s3 of the compressed vectors: index of a grid
+// point's record (t = 0: scaling coefficient), -1 where it has none, and the
+// byte offset of its value
+struct Comp {
+  const int* inv;
+  unsigned off, mul;
+  __device__ __forceinline__ Comp(const BoxDesc& bd, int t)
+      : inv(t == 0 ? bd.cinv : bd.finv), off(t == 0 ? 0u : 8u * (unsigned)(bd.nvctr_c + t - 1)),
+        mul(t == 0 ? 8u : 56u) {}
+  __device__ __forceinline__ int index(int lin) const { return inv ? inv[lin] : lin; }
+  __device__ __forceinline__ unsigned at(int i) const { return off + mul * (unsigned)i; }
+};
+
+template <int NTM, int PC>
 __device__ __forceinline__ void xykin_tile(const Batch& B, const TileTable& tt,
                                            const TileTable& ft, const PcArgs& P, int tile,
                                            unsigned char* smem) {
@@ -577,167 +671,186 @@ __device__ __forceinline__ void xykin_tile(const Batch& B, const TileTable& tt,
   const int lt = tile - box_first_tile(tt, lb);
   const int N1 = bd.N[0], N2 = bd.N[1], N3 = bd.N[2], per = bd.per;
   const int s3 = lt & 1, i3 = lt >> 1;
-  const int W1 = 2 * N1, W2 = 2 * N2, RA = W1 + 1, npl = N1 * N2;
+  const int W1 = 2 * N1, W2 = 2 * N2, RA = pair_stride(N1), npl = N1 * N2;
   double* A = (double*)smem;
-  int2* mx = (int2*)(A + (W2 + 1) * RA);
-  int2* my = mx + map_len(N1);
+  int2* my = (int2*)(A + (W2 + 1) * RA);
+  int* mx = (int*)(my + map_len(N2));
   const int tid = threadIdx.x, nt = blockDim.x;
-  // gather: thread's component c = s1 + 2 s2 of every (nt / 4)-th point
-  const int c = tid & 3, st = nt >> 2;
-  const bool cs = c == 0 && s3 == 0;
-  const unsigned off = cs ? 0u : 8u * (unsigned)(bd.nvctr_c + c + 4 * s3 - 1);
-  const unsigned mul = cs ? 8u : 56u;
-  const int* inv = cs ? bd.cinv : bd.finv;
   const int lin0 = npl * i3;
-  const double sc = PC ? P.pc[9 * b + 1 + c + 4 * s3] : 1.0;
+  const int st = nt >> 2;
   {
+    // gather: thread's component c = s1 + 2 s2 of every (nt / 4)-th point
     constexpr int UR = 8;
+    const int c = tid & 3;
+    const Comp cp(bd, c + 4 * s3);
+    const double sc = PC ? P.pc[9 * b + 1 + c + 4 * s3] : 1.0;
     const char* src = (const char*)((PC == 0 ? B.psi : PC == 1 ? P.x : P.d) + bd.psi_off);
     const bool dense = !bd.cinv && !bd.finv;
-    double* base = A + (c >> 1) * N2 * RA + (c & 1) * N1;
+    double* base = A + (c >> 1) * N2 * RA + (c & 1);
     ItDiv d(tid >> 2, N1, st);
     for (int pb = tid >> 2; pb < npl; pb += st * UR) {
       double v[UR];
       if (dense) {
 #pragma unroll
         for (int u = 0; u < UR; ++u)
-          v[u] = *(const double*)(src + (off + mul * (unsigned)(lin0 + min(pb + u * st, npl - 1))));
+          v[u] = *(const double*)(src + cp.at(lin0 + min(pb + u * st, npl - 1)));
       } else {
         int r[UR];
 #pragma unroll
         for (int u = 0; u < UR; ++u) {
           const int p = pb + u * st;
           r[u] = -1;
-          if (p < npl) r[u] = inv ? inv[lin0 + p] : lin0 + p;
+          if (p < npl) r[u] = cp.index(lin0 + p);
         }
 #pragma unroll
         for (int u = 0; u < UR; ++u)
-          v[u] = r[u] >= 0 ? *(const double*)(src + (off + mul * (unsigned)r[u])) : 0.0;
+          v[u] = r[u] >= 0 ? *(const double*)(src + cp.at(r[u])) : 0.0;
       }
 #pragma unroll
       for (int u = 0; u < UR; ++u) {
-        if (pb + u * st < npl) base[d.ch * RA + d.j] = PC ? sc * v[u] : v[u];
+        if (pb + u * st < npl) base[d.ch * RA + 2 * d.j] = PC ? sc * v[u] : v[u];
         d.next(N1);
       }
     }
   }
-  build_map(mx, N1, per, sizeof(double), W1, tid, nt);
   build_map(my, N2, per, RA * sizeof(double), W2, tid, nt);
-  for (int i = tid; i < W2; i += nt) A[i * RA + W1] = 0.0;
+  for (int e = tid; e < map_len(N1); e += nt) {
+    int k = e - MOFF;
+    if (per) {
+      while (k < 0) k += N1;
+      while (k >= N1) k -= N1;
+    } else if ((unsigned)k >= (unsigned)N1) {
+      k = N1;   // a pair of zeros
+    }
+    mx[e] = 16 * k;
+  }
+  for (int i = tid; i < W2; i += nt) *(double2*)(A + i * RA + W1) = make_double2(0.0, 0.0);
   for (int i = tid; i < RA; i += nt) A[W2 * RA + i] = 0.0;
   __syncthreads();
-  double* K = (double*)B.K + bd.w_off + (long long)W1 * W2 * (i3 + N3 * s3);
   const double kx = bd.kscale[0], ky = bd.kscale[1];
-  const int cy = (N2 + 3) >> 2, cx = (N1 + 3) >> 2;
-  each_item<MI>(ItDiv(tid, W1, nt), W1, cy, [&](int, int ch, int j1) {
-    const int i0 = 4 * ch;
-    double oc[4], od[4];
-    const unsigned at = 8u * (unsigned)(j1 + W1 * i0);
-    auto kc = [&](int r) { return (double*)((char*)(K + W1 * r) + at); };
-    double k[8];   // K before, read ahead of the stencil
+  const int cx = (N1 + 3) >> 2, nblk = cx * ((N2 + 3) >> 2);
+  const float icx = 1.0f / (float)cx;
+  double* K = (double*)B.K + bd.w_off + (long long)W1 * W2 * (i3 + N3 * s3);
+  double sum = 0.0;
+  for (int b0 = 8 * __builtin_amdgcn_readfirstlane(tid >> 6); b0 < nblk; b0 += nt >> 3) {
+    int l = tid;   // opaque: what follows from it is not held over the loop
+    asm volatile("" : "+v"(l));
+    const int o = l & 3, s = (l >> 4) & 1, g = ((l >> 2) & 3) + 4 * ((l >> 5) & 1);
+    const int blk = min(b0 + g, nblk - 1);
+    const int chy = qdiv(blk, cx, icx), i1 = 4 * (blk - chy * cx), i2 = 4 * chy;
+    const int x = min(i1 + o, N1 - 1);                     // lane's column
+    const int row = s * N2 + min(i2 + o, N2 - 1);          // and row
+    // results of this lane: rows i2 + r (s2 = 0: h = r, 1: h = 4 + r)
+    const int nrow = b0 + g < nblk && i1 + o < N1 ? N2 - i2 : 0;
+    // byte offset of the first of them from the plane's K (uniform base)
+    const unsigned at = 8u * (unsigned)(x + N1 * s + W1 * i2);
+    auto kp = [&](int h) {
+      return (double*)((char*)K + (at + 8u * (unsigned)(W1 * ((h & 3) + (h >> 2) * N2))));
+    };
+    double vx[8], vy[8];
+#pragma unroll
+    for (int h = 0; h < 8; ++h) vx[h] = vy[h] = 0.0;
+    {
+      const char* a = (const char*)(A + row * RA);
+      const int* m = mx + (i1 - 14 + MOFF);
+      kin_order([&](int kk) {
+        const double2 w = *(const double2*)(a + m[kk]);
+        kin_tap(kk, w.x, w.y, vx, vx + 4);
+      });
+    }
+    transpose8(vx);
+    const double* col = A + 2 * x + s;
+    if (__all(i2 >= 14 && i2 + 17 < N2)) {
+      const double *yc = col + (i2 - 14) * RA, *yd = yc + N2 * RA;
+      kin_order([&](int kk) { kin_tap(kk, yc[kk * RA], yd[kk * RA], vy, vy + 4); });
+    } else {
+      const int2* m = my + (i2 - 14 + MOFF);
+      kin_order([&](int kk) {
+        const double2 w = at2(col, m[kk]);
+        kin_tap(kk, w.x, w.y, vy, vy + 4);
+      });
+    }
     if (PC) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (i0 + r < N2) {
-          k[r] = *kc(r);
-          k[4 + r] = *kc(N2 + r);
-        }
+      for (int h = 0; h < 8; ++h) vx[h] = fma(vy[h], ky, vx[h] * kx);
+      double k[8];
+#pragma unroll
+      for (int h = 0; h < 8; ++h) k[h] = (h & 3) < nrow ? *kp(h) : 0.0;
+#pragma unroll
+      for (int h = 0; h < 8; ++h) vx[h] += k[h];
+    } else {
+#pragma unroll
+      for (int h = 0; h < 8; ++h) vx[h] = fma(vy[h], ky, vx[h] * kx);
     }
-    kin4_any(PLine<double>{A + j1, RA}, my, N2, i0, oc, od);
+    if (PC < 2) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (i0 + r < N2) {
-        *kc(r) = PC ? fma(oc[r], ky, k[r]) : oc[r] * ky;
-        *kc(N2 + r) = PC ? fma(od[r], ky, k[4 + r]) : od[r] * ky;
-      }
-  });
-  double o[MI][8];
-  const ItDiv d2(tid, W2, nt);
-  each_item<MI>(d2, W2, cx, [&](int m, int ch, int j2) {
-    kin4_any(PLine<double>{A + j2 * RA, 1}, mx, N1, 4 * ch, o[m], o[m] + 4);
-  });
-  __syncthreads();
-  each_item<MI>(d2, W2, cx, [&](int m, int ch, int j2) {
-    double* a = A + j2 * RA + 4 * ch;
+      for (int h = 0; h < 8; ++h)
+        if ((h & 3) < nrow) *kp(h) = vx[h];
+    } else {
+      char* q = (char*)(P.q + bd.psi_off);
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (4 * ch + r < N1) {
-        a[r] = o[m][r] * kx;
-        a[N1 + r] = o[m][4 + r] * kx;
+      for (int h = 0; h < 8; ++h) {
+        const int r = h & 3, s2 = h >> 2, t = s + 2 * s2 + 4 * s3;
+        const Comp cp(bd, t);
+        int i = -1;
+        if (r < nrow) i = cp.index(lin0 + x + N1 * (i2 + r));
+        if (i >= 0) {
+          *(double*)(q + cp.at(i)) = P.pc[9 * b + 1 + t] * vx[h];
+          sum = fma(vx[h], col[(s2 * N2 + i2 + r) * RA], sum);
+        }
       }
-  });
-  __syncthreads();
-  if constexpr (PC != 0) {
-    // the plane's elements of the compressed vectors
-    __shared__ double red[NTM / 64];
+    }
+  }
+  if constexpr (PC == 1) {
+    // r and d in the order of the records: three streams of single values from
+    // the blocks' lanes took 0.89 ms, K through memory 0.66
+    __syncthreads();
     constexpr int UR = 4;
-    const char* y = (const char*)((PC == 1 ? P.b : P.d) + bd.psi_off);
-    char* q = (char*)((PC == 1 ? P.r : P.q) + bd.psi_off);
+    int to = tid;   // opaque, as in the loop
+    asm volatile("" : "+v"(to));
+    const int c = to & 3;
+    const Comp cp(bd, c + 4 * s3);
+    const double sc = P.pc[9 * b + 1 + c + 4 * s3];
+    const char* y = (const char*)(P.b + bd.psi_off);
+    char* rr = (char*)(P.r + bd.psi_off);
     char* dd = (char*)(P.d + bd.psi_off);
-    const int row0 = (c >> 1) * N2, col0 = (c & 1) * N1;
-    double acc = 0.0;
-    ItDiv d(tid >> 2, N1, st);
-    for (int pb = tid >> 2; pb < npl; pb += st * UR) {
+    const double* kc = K + (size_t)((c >> 1) * N2) * W1 + (c & 1) * N1;
+    ItDiv d(to >> 2, N1, st);
+    for (int pb = to >> 2; pb < npl; pb += st * UR) {
       int r[UR];
       double k[UR], v[UR];
-      int a[UR];
 #pragma unroll
       for (int u = 0; u < UR; ++u) {
         const int p = pb + u * st;
         r[u] = -1;
-        if (p < npl) r[u] = inv ? inv[lin0 + p] : lin0 + p;
-        a[u] = (row0 + d.ch) * RA + col0 + d.j;
-        k[u] = p < npl ? K[(row0 + d.ch) * W1 + col0 + d.j] : 0.0;
+        if (p < npl) r[u] = cp.index(lin0 + p);
+        k[u] = p < npl ? kc[d.ch * W1 + d.j] : 0.0;
         d.next(N1);
       }
 #pragma unroll
-      for (int u = 0; u < UR; ++u)
-        v[u] = r[u] >= 0 ? *(const double*)(y + (off + mul * (unsigned)r[u])) : 0.0;
+      for (int u = 0; u < UR; ++u) v[u] = r[u] >= 0 ? *(const double*)(y + cp.at(r[u])) : 0.0;
 #pragma unroll
       for (int u = 0; u < UR; ++u)
         if (r[u] >= 0) {
-          const double av = sc * (k[u] + A[a[u]]);
-          const unsigned at = off + mul * (unsigned)r[u];
-          if (PC == 1) {
-            const double rv = v[u] - av;
-            *(double*)(q + at) = rv;
-            *(double*)(dd + at) = rv;
-            acc = fma(rv, rv, acc);
-          } else {
-            *(double*)(q + at) = av;
-            acc = fma(av, v[u], acc);
-          }
+          const double rv = v[u] - sc * k[u];
+          *(double*)(rr + cp.at(r[u])) = rv;
+          *(double*)(dd + cp.at(r[u])) = rv;
+          sum = fma(rv, rv, sum);
         }
     }
-    const double sum = block_sum_rt(acc, red);
-    if (tid == 0) P.part[box_first_tile(ft, b) + lt] = sum;
-    return;
   }
-  // two values at a time (rows of 2 N1 values: 16-byte aligned)
-  const int tot = N1 * W2;
-  double2* K2 = (double2*)K;
-  ItDiv d(tid, N1, nt);
-  constexpr int UR = 4;
-  for (int i = tid; i < tot; i += nt * UR) {
-    double2 v[UR];
-#pragma unroll
-    for (int u = 0; u < UR; ++u) v[u] = K2[min(i + u * nt, tot - 1)];
-#pragma unroll
-    for (int u = 0; u < UR; ++u) {
-      if (i + u * nt < tot) {
-        const double* a = A + d.ch * RA + 2 * d.j;
-        K2[i + u * nt] = make_double2(v[u].x + a[0], v[u].y + a[1]);
-      }
-      d.next(N1);
-    }
+  if constexpr (PC != 0) {
+    __shared__ double red[NTM / 64];
+    const double v = block_sum_rt(sum, red);
+    if (tid == 0) P.part[box_first_tile(ft, b) + lt] = v;
   }
 }
 
-template <int NTM, int MI, int WPE, int PC = 0>
+template <int NTM, int WPE, int PC>
 __global__ __launch_bounds__(NTM, WPE) void k_xykin(Batch B, TileTable tt, TileTable ft,
                                                     PcArgs P) {
   extern __shared__ __align__(16) unsigned char smem[];
-  xykin_tile<NTM, MI, PC>(B, tt, ft, P, tile_of(tt), smem);
+  xykin_tile<NTM, PC>(B, tt, ft, P, tile_of(tt), smem);
 }
 
 // Both kernels that read psi alone in one launch: nx planes of k_xykin, then
@@ -748,7 +861,7 @@ __global__ __launch_bounds__(NTM, 6) void k_zgrow_xykin(Batch B, TileTable tz, T
   extern __shared__ __align__(16) unsigned char smem[];
   const int b = blockIdx.x;
   if (b < nx)
-    xykin_tile<NTM, 2, 0>(B, tx, tx, PcArgs{}, tx.xcd ? xcd_tile(b, nx) : b, smem);
+    xykin_tile<NTM, 0>(B, tx, tx, PcArgs{}, tx.xcd ? xcd_tile(b, nx) : b, smem);
   else
     zgrow_tile<NTM>(B, tz, tz.xcd ? xcd_tile(b - nx, gridDim.x - nx) : b - nx, smem);
 }
@@ -1239,7 +1352,7 @@ __global__ __launch_bounds__(NTM, WPE) void k_xlines_kin(Batch B, TileTable tt) 
 #pragma unroll
     for (int h = 0; h < 8; ++h) o[m][h] = 0.0;
     if (i0 < N1)
-      line_taps<32>(i0 - 14, N1, per, [&](int kk, int k) {
+      kin_taps(i0 - 14, N1, per, [&](int kk, int k) {
         kin_tap(kk, col[k * LR], col[(N1 + k) * LR], o[m], o[m] + 4);
       });
   }
@@ -1295,7 +1408,7 @@ __global__ __launch_bounds__(NTM, WPE) void k_ylines_kin(Batch B, TileTable tt) 
       k[h] = K[W1 * i];
       k[4 + h] = K[W1 * (N2 + i)];
     }
-    line_taps<32>(i0 - 14, N2, per,
+    kin_taps(i0 - 14, N2, per,
                   [&](int kk, int i) { kin_tap(kk, c[i * NL], d[i * NL], o, o + 4); });
     if (on) {
 #pragma unroll
@@ -1377,7 +1490,7 @@ size_t fp64_fit_z(const BoxDesc& b, size_t plane_lds) {
   return v + LDS_STATIC <= plane_lds ? v : 0;
 }
 static size_t fp64_lds_kin(int N1, int N2) {
-  return 8 * ((size_t)(2 * N2 + 1) * (2 * N1 + 1) + map_len(N1) + map_len(N2));
+  return 8 * ((size_t)(2 * N2 + 1) * pair_stride(N1) + map_len(N2)) + 4 * map_len(N1);
 }
 static size_t fp64_lds_pot(int N1, int N2, int L1, int L2) {
   const size_t x = (size_t)2 * N2 * (L1 | 1), y = (size_t)L1 * (L2 | 1);
@@ -1421,9 +1534,14 @@ bool fp64_pot_lines_ok(const BoxDesc& b, size_t plane_lds) {
                               2 * n1 * n2 * n3 + l1 * n2 * n3 + l1 * l2 * n3);
 }
 PlaneFit fp64_fit_kin(const BoxDesc& b, size_t plane_lds) {
-  const int N1 = b.N[0], N2 = b.N[1];
-  return plane_fit(fp64_lds_kin(N1, N2),
-                   std::max(2 * N1 * chunks(N2, 4), 2 * N2 * chunks(N1, 4)), plane_lds);
+  // a wave takes eight blocks of 4 x 4 points, any number of times
+  const int nblk = chunks(b.N[0], 4) * chunks(b.N[1], 4);
+  const size_t lds = fp64_lds_kin(b.N[0], b.N[1]);
+  plane_lds -= std::min(plane_lds, LDS_STATIC);
+  if (lds <= plane_lds / 4) return {4, nblk <= 32 ? 128 : 256, lds};
+  if (lds <= plane_lds / 3) return {3, 512, lds};
+  if (lds <= plane_lds / 2) return {2, S2_NT, lds};
+  return {lds <= plane_lds ? 1 : 0, S1_NT, lds};
 }
 PlaneFit fp64_fit_pot(const BoxDesc& b, size_t plane_lds) {
   const int N1 = b.N[0], N2 = b.N[1], L1 = b.L[0], L2 = b.L[1];
@@ -1457,8 +1575,8 @@ static hipError_t launch_xykin(const Batch& B, const TileTable& t, const TileTab
                                int ntiles, size_t lds, int nt, int shape, const PcArgs& P,
                                hipStream_t s) {
   if (ntiles <= 0) return hipSuccess;
-  if (shape >= 2) k_xykin<S2_NT, 2, 6, PC><<<ntiles, nt, lds, s>>>(B, t, ft, P);
-  else k_xykin<S1_NT, 3, 4, PC><<<ntiles, nt, lds, s>>>(B, t, ft, P);
+  if (shape >= 2) k_xykin<S2_NT, 6, PC><<<ntiles, nt, lds, s>>>(B, t, ft, P);
+  else k_xykin<S1_NT, 4, PC><<<ntiles, nt, lds, s>>>(B, t, ft, P);
   return hipGetLastError();
 }
 // the x-y kinetic pass: one launch per group of boxes, or one over all
@@ -1617,11 +1735,11 @@ void fp64_attributes(size_t lds) {
                      (const void*)k_zback<768, 1, 6>,   (const void*)k_zback<512, 2, 4>,
                      (const void*)k_zback<1024, 3, 4>,
                      (const void*)k_xyden<512, 3, 4>, (const void*)k_xyden<S1_NT, 3, 4>,
-                     (const void*)k_xykin<S2_NT, 2, 6>, (const void*)k_xypot<S2_NT, 2, 6>,
-                     (const void*)k_xykin<S2_NT, 2, 6, 1>, (const void*)k_xykin<S2_NT, 2, 6, 2>,
-                     (const void*)k_xykin<S1_NT, 3, 4, 1>, (const void*)k_xykin<S1_NT, 3, 4, 2>,
+                     (const void*)k_xykin<S2_NT, 6, 0>, (const void*)k_xypot<S2_NT, 2, 6>,
+                     (const void*)k_xykin<S2_NT, 6, 1>, (const void*)k_xykin<S2_NT, 6, 2>,
+                     (const void*)k_xykin<S1_NT, 4, 1>, (const void*)k_xykin<S1_NT, 4, 2>,
                      (const void*)k_pcz<0>, (const void*)k_pcz<1>, (const void*)k_pcz<2>,
-                     (const void*)k_xykin<S1_NT, 3, 4>, (const void*)k_xypot<S1_NT, 3, 4>};
+                     (const void*)k_xykin<S1_NT, 4, 0>, (const void*)k_xypot<S1_NT, 3, 4>};
   for (const void* f : k)
     if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
         hipSuccess)
