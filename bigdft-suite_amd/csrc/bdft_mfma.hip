@@ -24,6 +24,7 @@
 // not fit in LDS.
 #include "bdft_internal.h"
 #include "../../include/bigdft_hip.h"
+#include "bdft_stencil.h"
 
 namespace bdft {
 
@@ -712,6 +713,41 @@ __global__ __launch_bounds__(NTMP) void k_mshrink_plane(Batch B, TileTable tt) {
   }
 }
 
+// A plane of h rows of w floats (w even, 8-byte aligned) times sc into LDS as
+// split pieces [row * (KX + 8) + x], zero for w <= x < KX and h <= row < nR:
+// two x-neighbours per load and per LDS store, eight loads in flight, row and
+// column counted on instead of divided out (48^3, 256 orbitals: k_mbwd 1.42 ->
+// 1.37 ms with pairs in place of single values, k_mfwd 1.04 -> 1.01).
+template <int M>
+__device__ __forceinline__ void stage_plane(const float* src, int w, int h, int KX, int nR,
+                                            float sc, __bf16* rh, __bf16* rl) {
+  constexpr int UR = 8;
+  const float2* s2 = (const float2*)src;
+  const int hp = KX / 2, tot = nR * hp;
+  ItDiv d(threadIdx.x, hp, NTMP);
+  for (int i0 = threadIdx.x; i0 < tot; i0 += NTMP * UR) {
+    float2 v[UR];
+    int at[UR];
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      at[u] = d.ch * (KX + 8) + 2 * d.j;
+      const bool in = d.ch < h && 2 * d.j < w;   // rows beyond nR too
+      v[u] = in ? s2[d.ch * (w >> 1) + d.j] : make_float2(0.0f, 0.0f);
+      d.next(hp);
+    }
+#pragma unroll
+    for (int u = 0; u < UR; ++u) {
+      if (i0 + u * NTMP < tot) {
+        __bf16 h0, l0, h1, l1;
+        split2<M>(v[u].x * sc, h0, l0);
+        split2<M>(v[u].y * sc, h1, l1);
+        *(bf16x2*)(rh + at[u]) = bf16x2{h0, h1};
+        *(bf16x2*)(rl + at[u]) = bf16x2{l0, l1};
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Plane-fused forward pass, one work-group per x-y plane j3 of a box:
 //   K  = (Ktilde_x + Ktilde_y) W      (kinetic of the plane)
@@ -750,37 +786,9 @@ __global__ __launch_bounds__(NTMP, 4) void k_mfwd(Batch B, TileTable tt) {
   __bf16* rl = rh + nR * XR;
   __bf16* ch = rl + nR * XR;   // [p1 * XC + j2]
   __bf16* cl = ch + nC * XC;
-  // load the plane, two x-neighbours per thread (W1 is even)
-  {
-    const float2* src =
-        (const float2*)((const float*)B.W + bd.w_off + (long long)W1 * W2 * j3);
-    const int hp = KX / 2;
-    const float ihp = 1.0f / (float)hp;
-    const int tot = nR * hp;
-    for (int i0 = threadIdx.x; i0 < tot; i0 += NTMP * 8) {
-      float2 v[8];
-      int jj[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int i = i0 + u * NTMP;
-        const int j2 = qdiv(i, hp, ihp), j1 = 2 * (i - j2 * hp);
-        jj[u] = j2 * XR + j1;
-        v[u] = (i < tot && j2 < W2 && j1 < W1) ? src[(j2 * W1 + j1) >> 1]
-                                                : make_float2(0.0f, 0.0f);
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int i = i0 + u * NTMP;
-        if (i < tot) {
-          __bf16 h0, l0, h1, l1;
-          split2<NT4>(v[u].x * sc, h0, l0);
-          split2<NT4>(v[u].y * sc, h1, l1);
-          *(bf16x2*)(rh + jj[u]) = bf16x2{h0, h1};
-          *(bf16x2*)(rl + jj[u]) = bf16x2{l0, l1};
-        }
-      }
-    }
-  }
+  // load the plane (W1 is even)
+  stage_plane<NT4>((const float*)B.W + bd.w_off + (long long)W1 * W2 * j3, W1, W2, KX, nR, sc, rh,
+                   rl);
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -906,8 +914,10 @@ __global__ __launch_bounds__(NTMP) void k_mbwd(Batch B, TileTable tt) {
   __bf16* rl = rh + nR * XR;
   __bf16* ch = rl + nR * XR;   // [j1 * XC + p2]
   __bf16* cl = ch + nC * XC;
-  {
-    const float* src = (const float*)B.T2 + bd.t2_off + (long long)L1 * L2 * j3;
+  const float* src = (const float*)B.T2 + bd.t2_off + (long long)L1 * L2 * j3;
+  if ((L1 & 1) == 0) {
+    stage_plane<BM>(src, L1, L2, KX, nR, 1.0f, rh, rl);
+  } else {
     const int tot = nR * KX;
     const float ikx = 1.0f / (float)KX;
     for (int i0 = threadIdx.x; i0 < tot; i0 += NTMP * 8) {
