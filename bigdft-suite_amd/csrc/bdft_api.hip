@@ -747,6 +747,7 @@ struct PlanChoice {
   int xbig, zbig;
   int nthr_rp[4];           // FP64 potential pass: threads by launch shape
                             // (they set the order of the epot sums)
+  int rp_one;               // its one launch shape, 0: by box
 };
 
 // point the plan's grids at their places in a workspace of ws_need bytes
@@ -1133,7 +1134,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     // every work-group's LDS.  One group (n = 0) runs as a single launch
     // over t[pass], with entry 0's shape, threads and LDS.
     auto group = [&](int pass, auto fit_of, TileTable* tg, int* nt, size_t* lg, int* shape,
-                     int* nthr, int& n, int off[4][2]) {
+                     int* nthr, int& n, int off[4][2], bool one = false) {
       n = 0;
       std::vector<int> grp[4];
       PlaneFit most[4] = {};
@@ -1145,14 +1146,15 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
         most[c].lds = std::max(most[c].lds, f.lds);
       }
       int ng = 0;
-      for (int c = 0; c < 4; ++c)
+      lg[0] = 0;
+      for (int c = 3; c >= 0; --c)
         if (!grp[c].empty()) {
           ++ng;
-          shape[0] = c + 1;
+          shape[0] = c + 1;   // of the largest boxes
           nthr[0] = most[c].nt;
-          lg[0] = most[c].lds;
+          lg[0] = std::max(lg[0], most[c].lds);
         }
-      if (ng < 2) return;
+      if (ng < 2 || one) return;
       for (int c = 4; c >= 1; --c)
         if (!grp[c - 1].empty()) {
           const int k = n++;
@@ -1175,14 +1177,29 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     };
     T.n_pfg = T.n_pbg = 0;
     if (T.plane && d64) {
+      // One launch over all boxes, in the largest boxes' shape, while launches
+      // and their last waves of work-groups cost more than the occupancy of the
+      // smaller boxes: the x-y kinetic up to where it shares a launch with G_z
+      // (free boxes of 16 to 40 points an axis: 4 of them 144 -> 116 us, 16:
+      // 249 -> 228, 64: 645 -> 616; 256: 2.02 -> 2.07 ms), the potential pass
+      // up to two planes per CU (4 boxes 116 -> 101 us, 8: 136 -> 133, 16: 224
+      // -> 245).
+      long long work = 0;   // work-groups of the x-y kinetic and of G_z
+      for (const BoxDesc& b : box) work += box_tiles(b, P_PF, zg) + box_tiles(b, P_CZ, zg);
       if (!density && !T.kin_lines)
         group(P_PF, [&](const BoxDesc& b) { return fp64_fit_kin(b, ctx->plane_lds); }, T.pfg,
-              T.nt_pfg, T.lds_pfg, T.shape_pfg, T.nthr_pfg, T.n_pfg, pf_off);
-      if (!T.pot_lines)
+              T.nt_pfg, T.lds_pfg, T.shape_pfg, T.nthr_pfg, T.n_pfg, pf_off,
+              work <= FP64_JOIN);
+      if (!T.pot_lines) {
+        work = 0;
+        for (const BoxDesc& b : box) work += box_tiles(b, P_RP, zg);
+        T.rp_one = force ? force->rp_one > 0 : work <= 512;
         group(P_RP, [&](const BoxDesc& b) { return fp64_fit_pot(b, ctx->plane_lds); }, T.pbg,
-            T.nt_pbg, T.lds_pbg, T.shape_pbg, T.nthr_pbg, T.n_pbg, pb_off);
-      for (int k = 0; k < std::max(1, T.n_pbg) && force && !T.pot_lines; ++k)
-        T.nthr_pbg[k] = force->nthr_rp[T.shape_pbg[k] - 1];
+              T.nt_pbg, T.lds_pbg, T.shape_pbg, T.nthr_pbg, T.n_pbg, pb_off, T.rp_one);
+        if (force && T.rp_one) T.shape_pbg[0] = force->rp_one;
+        for (int k = 0; k < std::max(1, T.n_pbg) && force; ++k)
+          T.nthr_pbg[k] = force->nthr_rp[T.shape_pbg[k] - 1];
+      }
     } else if (T.plane && !density && ctx->plane_lds > 0) {
       auto fit = [&](size_t v) {
         const size_t c = ctx->plane_lds / std::max(v, (size_t)1);
@@ -1240,6 +1257,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     got->pot_lines = T.pot_lines;
     got->xbig = xbig;
     got->zbig = zbig;
+    got->rp_one = esz == 8 && T.plane && !T.pot_lines && T.rp_one ? T.shape_pbg[0] : 0;
     for (int k = 0; k < std::max(1, T.n_pbg); ++k)
       if (esz == 8 && T.plane && !T.pot_lines) got->nthr_rp[T.shape_pbg[k] - 1] = T.nthr_pbg[k];
     return BDFT_OK;  // choices only: nothing allocated

@@ -1636,12 +1636,11 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
   // launch and the first kernel's last, partly empty wave of work-groups, 6 to
   // 10 us for one orbital of 16^3 to 40^3 (60 of 66, 84 of 94 us), 15 to 25 us
   // for ten to sixty (32^3 x 60: 420 of 445 us; 40^3 x 40: 584 of 607).  From
-  // ZX_MAX work-groups on the gain is lost in the mix of two kinds of
+  // FP64_JOIN work-groups on the gain is lost in the mix of two kinds of
   // work-group on a CU (32^3 x 300: 1.955 of 1.960 ms, 40^3 x 128: 1.760 of
   // 1.745).
-  constexpr int ZX_MAX = 16384;
   const int nz = PT.ntiles[P_CZ], nx = PT.ntiles[P_PF];
-  if (!ev && !PT.kin_lines && PT.n_pfg == 0 && PT.shape_pfg[0] >= 2 && nz + nx <= ZX_MAX) {
+  if (!ev && !PT.kin_lines && PT.n_pfg == 0 && PT.shape_pfg[0] >= 2 && nz + nx <= FP64_JOIN) {
     const size_t lds = std::max(lds_w(PT.maxN3), PT.lds_pfg[0]);
     const TileTable &tz = PT.t[P_CZ], &tx = PT.t[P_PF];
     if (nz + nx <= 0) return hipSuccess;

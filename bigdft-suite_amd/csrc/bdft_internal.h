@@ -449,6 +449,7 @@ struct PassTables {
   // FP64 sequence: x-y kinetic, potential pass on lines (some plane does not
   // fit in LDS)
   int kin_lines, pot_lines;
+  int rp_one;   // planes of all boxes' potential pass in one launch shape
   // preconditioner: z lines and x-y planes of the compressed vectors
   // (bdft_fp64.hip) where every box fits, else the line passes
   int pc_plane;
@@ -628,6 +629,8 @@ struct PlaneFit {
 };
 PlaneFit fp64_fit_kin(const BoxDesc& b, size_t plane_lds);
 PlaneFit fp64_fit_pot(const BoxDesc& b, size_t plane_lds);
+// work-groups of k_xykin and k_zgrow up to which they share a launch
+constexpr int FP64_JOIN = 16384;
 bool fp64_kin_lines_ok(const BoxDesc& b, size_t plane_lds);
 bool fp64_pot_lines_ok(const BoxDesc& b, size_t plane_lds);
 void fp64_attributes(size_t lds);

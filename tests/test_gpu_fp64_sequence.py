@@ -236,3 +236,45 @@ def test_small_batches_share_the_first_launch(ctx, geo, n, norb):
     lr.close()
     for a, b in zip(one, each):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("copies", [1, 2, 5])
+def test_uneven_batches_in_one_and_in_several_launches(ctx, copies):
+    """boxes of every launch shape in one batch: few planes (one launch per
+    pass), more than 512 (potential pass by shape), against the oracle, and
+    cut into chunks the same bits"""
+    ns = [(4, 3, 5), (20, 17, 9), (27, 30, 12), (36, 35, 20), (49, 51, 7)]
+    regs = [dense_region("F", n, (0.4, 0.4, 0.4)) for n in ns]
+    psi = [random_psi(r, 1, 91 + i)[0] for i, r in enumerate(regs)]
+    pots = [random_pot(r, 95 + i) for i, r in enumerate(regs)]
+    lrs = [ctx.region(r) for r in regs] * copies
+    po = np.cumsum([0] + [p.size for p in pots])
+    so = np.cumsum([0] + [p.size for p in psi * copies])
+    x, pot = dev(np.concatenate(psi * copies)), dev(np.concatenate(pots))
+
+    def run():
+        h = torch.zeros_like(x)
+        ek = torch.zeros(len(lrs), dtype=torch.float64, device="cuda")
+        ep = torch.zeros_like(ek)
+        ctx.locham_batch(lrs, pot, x, h, ek, ep, pot_off=np.tile(po[:-1], copies), psi_off=so[:-1])
+        ctx.sync()
+        return h.cpu().numpy(), ek.cpu().numpy(), ep.cpu().numpy()
+    got = run()
+    ctx.set_option("chunk_mb", 8)
+    try:
+        cut = run()
+    finally:
+        ctx.set_option("chunk_mb", 0)
+    for a, b in zip(got, cut):
+        assert np.array_equal(a, b)
+    h = np.split(got[0], so[1:-1])
+    for i, r in enumerate(regs):
+        print(f"box {i} of {copies}", flush=True)
+        ho, eo, vo = oracle.locham("F", r.n, r.nfl, r.nfu, r.hgrid, okeys(r), pots[i],
+                                   psi[i][None])
+        for k in range(i, len(lrs), len(regs)):
+            assert np.abs(h[k] - ho[0]).max() < TOL * np.abs(ho).max()
+            assert rel_err(got[1][k:k + 1], eo) < TOL
+            assert rel_err(got[2][k:k + 1], vo) < TOL
+    for lr in lrs[:len(regs)]:
+        lr.close()
