@@ -163,10 +163,10 @@ def build_batch(cfg, seed, device):
 
 
 # Algorithmic FP64 bytes per coefficient and CG step of the preconditioner
-# (dense keys: one working-grid point per coefficient): d = r + beta d and
-# W = S d (32), K = c W + K_x W (16), K += K_y W, K_z W (24 + 24), q = S K and
-# q.d (24), x += alpha d, r -= alpha q, |r|^2 (48).
-PC_BYTES_PER_COEF_STEP = 168
+# (dense keys: one working-grid point per coefficient): x += alpha d, d = r +
+# beta d, K = c W + K_z W (48), q = S (K + K_x W + K_y W) and q.d (24),
+# r -= alpha q, |r|^2 (24).
+PC_BYTES_PER_COEF_STEP = 96
 
 
 def bench_precond(args, cfg, batch, ctx, lrs, stream):
@@ -197,7 +197,7 @@ def bench_precond(args, cfg, batch, ctx, lrs, stream):
     gbs = PC_BYTES_PER_COEF_STEP * ncoef * applies / (ms * 1e-3) / 1e9
     roof = {"bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
             "frac": gbs / PEAK_HBM_GBS, "traffic": None,
-            "kernel": "whole call (scatter, kinetic x/y/z, gather, update per CG step)",
+            "kernel": "whole call (x, d and z kinetic; x-y kinetic; r per CG step)",
             "bytes_per_coef_step": PC_BYTES_PER_COEF_STEP}
     cpu = None
     if not args.no_cpu:
@@ -292,8 +292,7 @@ def bench_density(args, cfg, batch, ctx, lrs, stream):
         roof = {"bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                 "frac": gbs / PEAK_HBM_GBS, "flop_TFLOPs": tfs}
     roof.update({"traffic": None, "bytes_per_pt": bpp, "flops_per_pt": fpp,
-                 "kernel": "whole call (uncompress, x and y grow, z grow + hfac psir^2, "
-                           "group reduction)"})
+                 "kernel": "whole call (z grow, x and y grow + hfac psir^2, group sum)"})
     cpu = None
     if not args.no_cpu:
         sys.path.insert(0, os.path.join(ROOT, "oracle"))

@@ -20,11 +20,12 @@
 // x-y-z order's kernels before: uncompress 183 us, forward planes 1085, z
 // kinetic 553, z potential 413, backward planes 689, an apply 2.65 ms; now
 // k_zgrow 0.24 ms (16 B per point: 4.4 TB/s, a large copy runs at 4.9),
-// k_xykin 0.52 and k_xypot 0.52 (3.5 and 3.7 times the time of their FMAs at
-// the FP64 peak; waits at barriers and LDS loads), k_zback 0.68 (40 B per
-// point: 3.9 TB/s), an apply 1.80 ms.  48 orbitals of a 64^3 box, whose pairs
-// of planes did not fit in LDS (line passes): 4.64 -> 2.99 ms; 256 free boxes
-// of 16 to 40 points an axis 2.70 -> 2.19 ms.
+// k_xykin 0.47 and k_xypot 0.49 (three times the time of their FMAs at the
+// FP64 peak; a quarter of their vector instructions are addresses, the rest
+// waits at barriers and LDS loads), k_zback 0.60 (40 B per point: 4.4 TB/s),
+// an apply 1.71 ms.  48 orbitals of a 64^3 box, whose pairs of planes did not
+// fit in LDS (line passes): 4.61 -> 2.84 ms; 256 free boxes of 16 to 40 points
+// an axis 2.66 -> 2.03 ms.
 //
 // Grid TZ of a box (tz_off): plane p3 = 0 .. L3 - 1, in it the wavelet plane
 // [j1 + 2 N1 j2]; K (w_off): the wavelet volume.
@@ -385,10 +386,10 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
 // MODE 0: v = x; 1: v = d; 2: v = d after the step's updates of the compressed
 // vectors, x += alpha d and d = r + beta d (the only kernel that reads whole
 // records of all three, so both updates ride on it: a conjugate-gradient step
-// moves 112 bytes per coefficient, in kernels of their own 144).  64 orbitals
+// moves 96 bytes per coefficient, in kernels of their own 128).  64 orbitals
 // of a periodic 48^3 box, six steps: 13.1 ms with the volumes W and K scattered
-// and gathered by kernels of their own, 9.0 now; this kernel 0.53 ms (48 bytes
-// per coefficient, 5.2 TB/s: bound by memory), k_xykin 0.57, the update of r
+// and gathered by kernels of their own, 8.3 now; this kernel 0.53 ms (48 bytes
+// per coefficient, 5.2 TB/s: bound by memory), k_xykin 0.53, the update of r
 // 0.23.
 // ---------------------------------------------------------------------------
 constexpr int PZ_NT = 512;
@@ -592,7 +593,7 @@ __device__ __forceinline__ void each_item(ItDiv d, int n, int nch, F f) {
 // once, 16 neighbouring columns per half-row of lanes.  The plane in LDS is
 // only read, so its one barrier is after the load, and K makes no second trip:
 // K_y written, read back and added to K_x moved 32 B per point in place of 16
-// (50 in place of 34 with PC), at 4.2 to 4.8 TB/s.  40^3 x 128 (65 M points):
+// (50 in place of 26 with PC), at 4.2 to 4.8 TB/s.  40^3 x 128 (65 M points):
 // 0.50 -> 0.47 ms, 64^3 x 48: 0.96 -> 0.80, PC 2 of 48^3 x 64: 0.63 -> 0.53;
 // bound by the vector units, three quarters of whose instructions are the
 // stencils.
