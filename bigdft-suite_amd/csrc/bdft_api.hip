@@ -748,6 +748,8 @@ struct PlanChoice {
   int nthr_rp[4];           // FP64 potential pass: threads by launch shape
                             // (they set the order of the epot sums)
   int rp_one;               // its one launch shape, 0: by box
+  int zb_n3;                // FP64 back pass: the longest z line its launch shape is
+                            // for (it sets the order of the ekin sums)
 };
 
 // point the plan's grids at their places in a workspace of ws_need bytes
@@ -1121,6 +1123,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     T.lds_pb = lpb;
     T.lds_cz = lcz;
     T.maxN3 = maxN3;
+    T.zb_n3 = force ? force->zb_n3 : maxN3;
     T.maxN1 = T.maxN2 = T.maxL1 = T.maxL2 = 0;
     for (const BoxDesc& b : box) {
       T.maxN1 = std::max(T.maxN1, b.N[0]);
@@ -1257,6 +1260,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     got->pot_lines = T.pot_lines;
     got->xbig = xbig;
     got->zbig = zbig;
+    got->zb_n3 = T.zb_n3;
     got->rp_one = esz == 8 && T.plane && !T.pot_lines && T.rp_one ? T.shape_pbg[0] : 0;
     for (int k = 0; k < std::max(1, T.n_pbg); ++k)
       if (esz == 8 && T.plane && !T.pot_lines) got->nthr_rp[T.shape_pbg[k] - 1] = T.nthr_pbg[k];

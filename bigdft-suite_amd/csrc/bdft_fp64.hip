@@ -1562,12 +1562,15 @@ static hipError_t launch_zgrow(const Batch& B, const TileTable& t, int ntiles, i
   else k_zgrow<1024><<<ntiles, 1024, lds, s>>>(B, t);
   return hipGetLastError();
 }
+// The launch shape says which chunks of a line a wave adds to its ekin sum, so
+// it follows the longest line n3 of the whole batch: a part of a chunked batch
+// that chose by its own lines summed 33 to 64 points in another order.
 static hipError_t launch_zback(const Batch& B, const TileTable& t, const TileTable& ft,
-                               int ntiles, size_t lds, int maxN3, double* part, hipStream_t s) {
+                               int ntiles, size_t lds, int n3, double* part, hipStream_t s) {
   if (ntiles <= 0) return hipSuccess;
-  if (maxN3 <= 32) k_zback<512, 1, 4><<<ntiles, 512, lds, s>>>(B, t, ft, part);
-  else if (maxN3 <= 48) k_zback<768, 1, 6><<<ntiles, 768, lds, s>>>(B, t, ft, part);
-  else if (maxN3 <= 64) k_zback<512, 2, 4><<<ntiles, 512, lds, s>>>(B, t, ft, part);
+  if (n3 <= 32) k_zback<512, 1, 4><<<ntiles, 512, lds, s>>>(B, t, ft, part);
+  else if (n3 <= 48) k_zback<768, 1, 6><<<ntiles, 768, lds, s>>>(B, t, ft, part);
+  else if (n3 <= 64) k_zback<512, 2, 4><<<ntiles, 512, lds, s>>>(B, t, ft, part);
   else k_zback<1024, 3, 4><<<ntiles, 1024, lds, s>>>(B, t, ft, part);
   return hipGetLastError();
 }
@@ -1670,7 +1673,7 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
   mark(S_XYP, 1);
   mark(S_ZB, 0);
   if (e == hipSuccess)
-    e = launch_zback(B, PT.t[P_CZ], PT.t[P_CZ], PT.ntiles[P_CZ], PT.lds_cz, PT.maxN3,
+    e = launch_zback(B, PT.t[P_CZ], PT.t[P_CZ], PT.ntiles[P_CZ], PT.lds_cz, PT.zb_n3,
                      PT.part[0], s);
   mark(S_ZB, 1);
   if (e != hipSuccess) return e;

@@ -446,6 +446,8 @@ struct PassTables {
   // z-line kernels of the FP64 sequence: LDS and longest line of the batch
   size_t lds_cz;
   int maxN1, maxN2, maxN3, maxL1, maxL2;
+  int zb_n3;    // longest z line that k_zback's launch shape is chosen for (of
+                // the whole batch where it runs in parts)
   // FP64 sequence: x-y kinetic, potential pass on lines (some plane does not
   // fit in LDS)
   int kin_lines, pot_lines;

@@ -278,3 +278,45 @@ def test_uneven_batches_in_one_and_in_several_launches(ctx, copies):
             assert rel_err(got[2][k:k + 1], vo) < TOL
     for lr in lrs[:len(regs)]:
         lr.close()
+
+
+@pytest.mark.parametrize("how", ["chunks", "fixed"])
+def test_parts_of_a_batch_sum_ekin_as_the_whole(ctx, how):
+    """z lines of 40, 60 and 75 points in one batch: the back pass's launch
+    shape decides which chunks of a line one wave sums, so a part that holds
+    only shorter lines than the batch's longest has to run the whole batch's
+    shape.  The same bits as in one piece, for cuts into parts of one length,
+    of two, and of all"""
+    # 1.2, 1.8 and 2.3 MB of grids a box: chunks of 4 MiB, or 128 MiB of the fixed array
+    times = 1 if how == "chunks" else 30
+    regs = {k: dense_region("P", (12, 8, k - 1), (0.45, 0.4, 0.5)) for k in (40, 60, 75)}
+    lr = {k: ctx.region(r) for k, r in regs.items()}
+    psi = {k: random_psi(r, 1, 101 + k)[0] for k, r in regs.items()}
+    pot = {k: random_pot(r, 103 + k) for k, r in regs.items()}
+    for lens in ([40] * 7 + [60] * 3, [60, 40, 40, 40, 40, 40, 40], [75, 40, 40, 60, 60, 60, 40]):
+        print(f"case {how} {lens}", flush=True)
+        lens = [k for k in lens for _ in range(times)]
+        so = np.cumsum([0] + [psi[k].size for k in lens])[:-1]
+        po = np.cumsum([0] + [pot[k].size for k in lens])[:-1]
+        x, v = dev(np.concatenate([psi[k] for k in lens])), dev(np.concatenate([pot[k] for k in lens]))
+
+        def run(fn):
+            h = torch.zeros_like(x)
+            ek = torch.zeros(len(lens), dtype=torch.float64, device="cuda")
+            ep = torch.zeros_like(ek)
+            fn([lr[k] for k in lens], v, x, h, ek, ep, pot_off=po, psi_off=so)
+            ctx.sync()
+            return h, ek, ep
+        whole = run(ctx.locham_batch)
+        if how == "chunks":
+            ctx.set_option("chunk_mb", 4)
+            try:
+                cut = run(ctx.locham_batch)
+            finally:
+                ctx.set_option("chunk_mb", 0)
+        else:
+            cut = run(ctx.locham_batch_fixed)
+        for a, b in zip(whole, cut):
+            assert torch.equal(a, b)
+    for l in lr.values():
+        l.close()
