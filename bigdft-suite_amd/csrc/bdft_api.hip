@@ -722,7 +722,7 @@ static int box_tiles(const BoxDesc& b, int pass, int zg) {
     case P_KZG: return cdiv((long long)cdiv(4LL * N1 * N2, TW), zg);
     case P_ZPG: return cdiv((long long)cdiv(L1, TW) * L2, zg);
     case P_ZPF: return cdiv((long long)L1 * L2, TW);
-    case P_CZ: return cdiv((long long)N1 * N2, CCOL);
+    case P_CZ: return cdiv((long long)N1 * N2, b.zcol ? b.zcol : CCOL);
     case P_RP: return b.L[2];
     case P_XK: return cdiv((long long)N2 * N3, CCOL);
     case P_YK: return cdiv(N1, CCOL) * N3;
@@ -793,7 +793,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   std::vector<BoxDesc> box((size_t)norb);
   long long wtot = 0, t1tot = 0, t2tot = 0, t3tot = 0, tztot = 0, txtot = 0,
             psi_run = 0;
-  int maxN = 0, maxN3 = 0;
+  int maxN = 0;
   bool xbig = false, zbig = false;
   int maxL3 = 0;
   bool need_zero = false;
@@ -871,7 +871,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     xbig = xbig || b.N[0] > REG_N || b.L[0] > REG_L;
     zbig = zbig || b.L[2] > REG_L;
     maxL3 = std::max(maxL3, b.L[2]);
-    maxN3 = std::max(maxN3, b.N[2]);
+    b.zcol = fp64_zcols(b, ctx->plane_lds);
     if (!lr->dense) need_zero = true;
   }
   // bundles per z-line tile of the matrix-core sequence: three, unless a
@@ -1001,6 +1001,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   int g_off[4] = {-1, -1, -1, -1};  // small starts, small map, large starts, large map
   int pf_off[4][2] = {{-1, -1}, {-1, -1}, {-1, -1}, {-1, -1}};  // forward plane groups
   int pb_off[4][2] = {{-1, -1}, {-1, -1}, {-1, -1}, {-1, -1}};  // backward plane groups
+  int zg_off[4][2] = {{-1, -1}, {-1, -1}, {-1, -1}, {-1, -1}};  // z-line groups
   int vb_off[4][2] = {{-1, -1}, {-1, -1}, {-1, -1}, {-1, -1}};  // FP32 backward groups
   if (mfma && ml.fused) {
     const size_t half = ctx->plane_lds / 2;
@@ -1091,7 +1092,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     // preconditioner's plans keep the line passes
     bool plane = !ctx->force_lines && !mfma && (!density || grow_plane);
     const bool d64 = esz == 8;   // the FP64 sequence (bdft_fp64.hip)
-    size_t lpf = 0, lpb = 0, lcz = 0;
+    size_t lpf = 0, lpb = 0;
     // FP64 sequence: z lines fit; planes of every box fit, else lines do
     bool fits = true, kp = true, pp = true, kl = true, pl = true;
     for (int i = 0; i < norb && plane; ++i) {
@@ -1101,9 +1102,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
         pp = pp && fp64_fit_pot(b, ctx->plane_lds).shape;
         kl = kl && fp64_kin_lines_ok(b, ctx->plane_lds);
         pl = pl && fp64_pot_lines_ok(b, ctx->plane_lds);
-        const size_t z = fp64_fit_z(b, ctx->plane_lds);
-        fits = fits && z;
-        lcz = std::max(lcz, z);
+        fits = fits && b.zcol;
       } else {
         lpf = std::max(lpf, plane_lds_fwd(b.N[0], b.N[1], b.L[0], (int)esz));
         lpb = std::max(lpb, plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1], (int)esz));
@@ -1121,9 +1120,9 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     }
     T.lds_pf = lpf;
     T.lds_pb = lpb;
-    T.lds_cz = lcz;
-    T.maxN3 = maxN3;
-    T.zb_n3 = force ? force->zb_n3 : maxN3;
+    T.zb_n3 = force ? force->zb_n3 : 0;
+    for (const BoxDesc& b : box)
+      if (!force && b.zcol == CCOL) T.zb_n3 = std::max(T.zb_n3, b.N[2]);
     T.maxN1 = T.maxN2 = T.maxL1 = T.maxL2 = 0;
     for (const BoxDesc& b : box) {
       T.maxN1 = std::max(T.maxN1, b.N[0]);
@@ -1178,8 +1177,16 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
           lg[k] = most[c - 1].lds;
         }
     };
-    T.n_pfg = T.n_pbg = 0;
+    T.n_pfg = T.n_pbg = T.n_zg = 0;
+    auto zgroup = [&] {
+      group(P_CZ,
+            [&](const BoxDesc& b) {
+              return PlaneFit{b.zcol == CCOL ? 2 : 1, b.N[2], fp64_lds_z(b, b.zcol)};
+            },
+            T.zg, T.nt_zg, T.lds_zg, T.shape_zg, T.len_zg, T.n_zg, zg_off);
+    };
     if (T.plane && d64) {
+      zgroup();
       // One launch over all boxes, in the largest boxes' shape, while launches
       // and their last waves of work-groups cost more than the occupancy of the
       // smaller boxes: the x-y kinetic up to where it shares a launch with G_z
@@ -1221,14 +1228,13 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     }
     // preconditioner plans (FP64): z lines and x-y planes where all boxes fit
     T.pc_plane = density && !grow_plane && !ctx->force_lines && esz == 8;
-    for (int i = 0; i < norb && T.pc_plane; ++i) {
-      const size_t z = fp64_fit_z(box[i], ctx->plane_lds);
-      if (!z || !fp64_fit_kin(box[i], ctx->plane_lds).shape) T.pc_plane = 0;
-      T.lds_cz = std::max(T.lds_cz, z);
-    }
-    if (T.pc_plane)
+    for (int i = 0; i < norb && T.pc_plane; ++i)
+      if (!box[i].zcol || !fp64_fit_kin(box[i], ctx->plane_lds).shape) T.pc_plane = 0;
+    if (T.pc_plane) {
+      zgroup();
       group(P_PF, [&](const BoxDesc& b) { return fp64_fit_kin(b, ctx->plane_lds); }, T.pfg,
             T.nt_pfg, T.lds_pfg, T.shape_pfg, T.nthr_pfg, T.n_pfg, pf_off);
+    }
   }
   // tile order: the z-line and line passes deal their tiles in contiguous
   // ranges per XCD (neighbouring bundles share cache lines); the plane and
@@ -1239,6 +1245,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     T.t[P_PF].xcd = T.t[P_PB].xcd = T.t[P_UNC].xcd = po;
     T.pf2.xcd = T.pb2.xcd = po;
     for (int k = 0; k < 4; ++k) T.vbg[k].xcd = T.pfg[k].xcd = T.pbg[k].xcd = po;
+    for (int k = 0; k < 4; ++k) T.zg[k].xcd = 1;
     // the two x-y kinetic planes of a coarse z read the same fine records
     if (esz == 8 && (!density || T.pc_plane)) {
       T.t[P_PF].xcd = 1;
@@ -1290,6 +1297,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   int tb_v[4] = {-1, -1, -1, -1};  // the FP32 backward groups
   int tb_f[4] = {-1, -1, -1, -1};  // the forward plane groups
   int tb_b[4] = {-1, -1, -1, -1};  // the backward plane groups
+  int tb_z[4] = {-1, -1, -1, -1};  // the z-line groups
   {
     constexpr int TB_MAX = 1 << 22;
     auto tiles_of = [&](int so, int nb) {
@@ -1311,6 +1319,8 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
       tb_f[k] = T.nt_pfg[k] <= TB_MAX ? tiles_of(pf_off[k][0], T.pfg[k].nbox) : -1;
     for (int k = 0; k < T.n_pbg; ++k)
       tb_b[k] = T.nt_pbg[k] <= TB_MAX ? tiles_of(pb_off[k][0], T.pbg[k].nbox) : -1;
+    for (int k = 0; k < T.n_zg; ++k)
+      tb_z[k] = T.nt_zg[k] <= TB_MAX ? tiles_of(zg_off[k][0], T.zg[k].nbox) : -1;
   }
   // work queue of the persistent z potential pass: the boxes in order of
   // decreasing work (fine points), each box's tiles together
@@ -1413,6 +1423,11 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     T.pbg[k].start = dst + pb_off[k][0];
     T.pbg[k].bmap = dst + pb_off[k][1];
     T.pbg[k].tbox = tb_b[k] >= 0 ? dst + tb_b[k] : nullptr;
+  }
+  for (int k = 0; k < T.n_zg; ++k) {
+    T.zg[k].start = dst + zg_off[k][0];
+    T.zg[k].bmap = dst + zg_off[k][1];
+    T.zg[k].tbox = tb_z[k] >= 0 ? dst + tb_z[k] : nullptr;
   }
   T.zq = zq_off >= 0 ? dst + zq_off : nullptr;
   T.zq_grid = 0;

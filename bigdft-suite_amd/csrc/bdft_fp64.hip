@@ -38,29 +38,49 @@
 namespace bdft {
 
 // ---------------------------------------------------------------------------
-// z-line tiles: CC coarse columns q = i1 + N1 i2 of a box, each with its four
-// z lines (s1, s2): line l = col + CC (s1 + 2 s2), one lane per line.  A wave
+// z-line tiles: C = 16 coarse columns q = i1 + N1 i2 of a box, each with its
+// four z lines (s1, s2): line l = col + C (s1 + 2 s2), one lane per line.  A wave
 // works on one chunk of outputs of all 64 lines, so the chunk's rows are
 // uniform over the wave: LDS rows are read without bank conflicts at
 // immediate offsets, and a line end costs scalar instructions only.
+//
+// Lines whose 64-line tile does not fit in LDS (beyond 159 periodic, 145 free
+// points): C = 8 columns, 32 lines, and each half of a wave takes a chunk of
+// its own (up to the library's 256 points, 138 KB).  The longer lines of a
+// batch have launches of their own.  16 orbitals of 24 x 24 x 200 points: 0.51
+// ms, on the line passes of bdft_pass.hip 2.04 (density 0.27 and 1.09 ms,
+// four preconditioner steps 1.86 and 5.12).
 // ---------------------------------------------------------------------------
 constexpr int CC = CCOL;
-constexpr int NL = 4 * CC;      // lines of a tile
+constexpr int NL = 4 * CC;      // lines of a tile of 16 columns
 static_assert(NL == 64, "one lane per line");
 
+// this lane's line and its chunk among the SUB a wave takes at a time
+template <int C>
+struct ZLane {
+  static constexpr int NLC = 4 * C, SUB = CC / C;
+  int line, sub;
+  __device__ __forceinline__ ZLane() {
+    const int lane = threadIdx.x & 63;
+    line = SUB == 1 ? lane : lane & (NLC - 1);
+    sub = SUB == 1 ? 0 : lane / NLC;
+  }
+};
+
 // W of the tile's columns into LDS: row s3 N3 + i3 (wavelet z index),
-// lane l.  Thread e = tid mod 128 moves element e of every (tid / 128)-th coarse
-// z: columns' scaling coefficients for e < 16, else component (e - 16) mod 7
-// of column (e - 16) / 7, the order the records have in memory.
+// lane l.  Thread e = tid mod 8 C moves element e of every (tid / 8 C)-th coarse
+// z: columns' scaling coefficients for e < C, else component (e - C) mod 7
+// of column (e - C) / 7, the order the records have in memory.
+template <int C = CC>
 struct RecElem {
   int col, t;                   // column and component 0..7
   __device__ __forceinline__ explicit RecElem(int e) {
-    if (e < CC) {
+    if (e < C) {
       col = e;
       t = 0;
     } else {
-      col = (e - CC) / 7;
-      t = e - CC - 7 * col + 1;
+      col = (e - C) / 7;
+      t = e - C - 7 * col + 1;
     }
   }
 };
@@ -68,13 +88,13 @@ struct RecElem {
 // AX = 1: the y lines of 16 coarse x of one coarse z instead, rows s2 N2 +
 // i2, lines col + CC (s1 + 2 s3).  lin0: linear index of the first column's
 // first point.
-template <int NT, int AX = 2>
+template <int NT, int AX = 2, int C = CC>
 __device__ __forceinline__ void load_columns(double* lds, const BoxDesc& bd, const double* psi,
                                              int first, int nq) {
-  constexpr int ZS = NT / 128, UR = 8;
+  constexpr int NL = 4 * C, EL = 8 * C, ZS = NT / EL, UR = 8;
   const int n = bd.N[AX], step = AX == 2 ? bd.N[0] * bd.N[1] : bd.N[0];
-  const RecElem re(threadIdx.x & 127);
-  const int z0 = threadIdx.x >> 7;
+  const RecElem<C> re(threadIdx.x & (EL - 1));
+  const int z0 = threadIdx.x / EL;
   const bool on = re.col < nq;
   const int lin0 = first + (on ? re.col : 0);
   const char* src = (const char*)(psi + bd.psi_off);
@@ -82,7 +102,7 @@ __device__ __forceinline__ void load_columns(double* lds, const BoxDesc& bd, con
   const unsigned mul = re.t == 0 ? 8u : 56u;
   const int sec = AX == 2 ? re.t >> 2 : (re.t >> 1) & 1;
   const int ln = AX == 2 ? re.t & 3 : (re.t & 1) + 2 * (re.t >> 2);
-  double* dst = lds + sec * n * NL + re.col + CC * ln;
+  double* dst = lds + sec * n * NL + re.col + C * ln;
   if (!bd.cinv && !bd.finv) {
     for (int zb = z0; zb < n; zb += ZS * UR) {
       double v[UR];
@@ -118,12 +138,13 @@ __device__ __forceinline__ void load_columns(double* lds, const BoxDesc& bd, con
   }
 }
 
-// The taps of rows k0 .. k0 + NK - 1 of a line, k0 uniform over the wave:
-// tap(kk, k) with k a valid row.  Rows past a line end wrap (periodic) or
+// The taps of rows k0 .. k0 + NK - 1 of a line, k0 uniform over the lanes of a
+// chunk: tap(kk, k) with k a valid row.  Rows past a line end wrap (periodic) or
 // are left out (free: they hold zeros).
-template <int NK, typename F>
+template <int NK, int SUB = 1, typename F>
 __device__ __forceinline__ void line_taps(int k0, int n, int per, F tap) {
-  if (k0 >= 0 && k0 + NK <= n) {
+  // (SUB > 1: the chunks of the whole wave)
+  if (SUB == 1 ? k0 >= 0 && k0 + NK <= n : (bool)__all(k0 >= 0 && k0 + NK <= n)) {
 #pragma unroll
     for (int kk = 0; kk < NK; ++kk) tap(kk, k0 + kk);
   } else if (per) {
@@ -156,9 +177,9 @@ __device__ __forceinline__ void kin_order(F tap) {
   }
 }
 // ... on a line of n values from k0 (as line_taps)
-template <typename F>
+template <int SUB = 1, typename F>
 __device__ __forceinline__ void kin_taps(int k0, int n, int per, F tap) {
-  if (k0 >= 0 && k0 + 32 <= n) {
+  if (SUB == 1 ? k0 >= 0 && k0 + 32 <= n : (bool)__all(k0 >= 0 && k0 + 32 <= n)) {
     kin_order([&](int kk) { tap(kk, k0 + kk); });
   } else if (per) {
     int ka = k0, kb = k0 + 31;
@@ -181,15 +202,16 @@ __device__ __forceinline__ void kin_taps(int k0, int n, int per, F tap) {
 }
 
 // a tile's lines: first column, columns, and this lane's line
+template <int C = CC>
 struct ColTile {
   int q0, nq;
   bool on;       // this lane's column is one of the box
   unsigned at;   // its line in a wavelet plane, j1 + 2 N1 j2
   __device__ __forceinline__ ColTile(const BoxDesc& bd, int lt) {
     const int N1 = bd.N[0], N2 = bd.N[1];
-    q0 = lt * CC;
-    nq = min(CC, N1 * N2 - q0);
-    const int lane = threadIdx.x & 63, col = lane & (CC - 1), s = lane / CC;
+    q0 = lt * C;
+    nq = min(C, N1 * N2 - q0);
+    const int line = ZLane<C>().line, col = line & (C - 1), s = line / C;
     on = col < nq;
     const int q = q0 + (on ? col : 0);
     const int i2 = qdiv(q, N1, 1.0f / (float)N1), i1 = q - i2 * N1;
@@ -200,27 +222,30 @@ struct ColTile {
 // ---------------------------------------------------------------------------
 // TZ = G_z W
 // ---------------------------------------------------------------------------
-template <int ZG_NT>
+template <int ZG_NT, int C = CC>
 __device__ __forceinline__ void zgrow_tile(const Batch& B, const TileTable& tt, int tile,
                                            unsigned char* smem) {
+  constexpr int NL = 4 * C, SUB = CC / C;
   double* lds = (double*)smem;
   const int lb = find_box(tt, tile);
   const BoxDesc bd = B.box[table_box(tt, lb)];
   const int N3 = bd.N[2], L3 = bd.L[2], per = bd.per;
-  const ColTile ct(bd, tile - box_first_tile(tt, lb));
-  load_columns<ZG_NT>(lds, bd, B.psi, ct.q0, ct.nq);
+  const ColTile<C> ct(bd, tile - box_first_tile(tt, lb));
+  load_columns<ZG_NT, 2, C>(lds, bd, B.psi, ct.q0, ct.nq);
   __syncthreads();
-  const double* c = lds + (threadIdx.x & 63);
+  const ZLane<C> zl;
+  const double* c = lds + zl.line;
   const double* d = c + N3 * NL;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t ps = 4 * (size_t)(bd.N[0] * bd.N[1]);
   double* out = (double*)B.TZ + bd.tz_off + ct.at;
-  for (int p0 = 8 * w; p0 < L3; p0 += 8 * (ZG_NT / 64)) {
+  for (int pw = 8 * SUB * w; pw < L3; pw += 8 * SUB * (ZG_NT / 64)) {
+    const int p0 = pw + 8 * zl.sub;
     double o[8];
 #pragma unroll
     for (int r = 0; r < 8; ++r) o[r] = 0.0;
-    line_taps<19>(grow_k0(p0, per), N3, per,
-                  [&](int kk, int k) { grow_tap(kk, c[k * NL], d[k * NL], o); });
+    line_taps<19, SUB>(grow_k0(p0, per), N3, per,
+                       [&](int kk, int k) { grow_tap(kk, c[k * NL], d[k * NL], o); });
     if (ct.on) {
       double* q = out + ps * p0;
 #pragma unroll
@@ -229,10 +254,10 @@ __device__ __forceinline__ void zgrow_tile(const Batch& B, const TileTable& tt, 
     }
   }
 }
-template <int ZG_NT>
+template <int ZG_NT, int C = CC>
 __global__ __launch_bounds__(ZG_NT) void k_zgrow(Batch B, TileTable tt) {
   extern __shared__ __align__(16) unsigned char smem[];
-  zgrow_tile<ZG_NT>(B, tt, tile_of(tt), smem);
+  zgrow_tile<ZG_NT, C>(B, tt, tile_of(tt), smem);
 }
 
 // ---------------------------------------------------------------------------
@@ -241,10 +266,10 @@ __global__ __launch_bounds__(ZG_NT) void k_zgrow(Batch B, TileTable tt) {
 // from W to TZ to the records of hpsi.  The
 // first loads of K and TZ are issued before the passes ahead of them.
 // ---------------------------------------------------------------------------
-template <int ZB_NT, int MI, int WPE>
+template <int ZB_NT, int MI, int WPE, int C = CC>
 __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, TileTable ft,
                                                  double* part) {
-  constexpr int NW = ZB_NT / 64;
+  constexpr int NW = ZB_NT / 64, NL = 4 * C, SUB = CC / C;
   extern __shared__ __align__(16) unsigned char smem[];
   double* lds = (double*)smem;
   __shared__ double red[NW];
@@ -254,10 +279,13 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
   const BoxDesc bd = B.box[b];
   const int lt = tile - box_first_tile(tt, lb);
   const int N3 = bd.N[2], L3 = bd.L[2], per = bd.per;
-  const ColTile ct(bd, lt);
-  const int lane = threadIdx.x & 63;
+  const ColTile<C> ct(bd, lt);
+  const ZLane<C> zl;
+  const int lane = zl.line;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t ps = 4 * (size_t)(bd.N[0] * bd.N[1]);
+  // chunk (row) j of this wave's
+  auto mine = [&](int j) { return SUB == 1 ? j : SUB * j + zl.sub; };
   // K of a chunk; the lines of TZ, TR rows of this wave at a time
   const double* K = (const double*)B.K + bd.w_off + ct.at;
   auto load_k = [&](int i0, double k[8]) {
@@ -272,11 +300,11 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
   const double* tz = (const double*)B.TZ + bd.tz_off + ct.at;
   auto load_tz = [&](int pb, double v[TR]) {
 #pragma unroll
-    for (int u = 0; u < TR; ++u) v[u] = tz[ps * min(pb + u * NW, L3 - 1)];
+    for (int u = 0; u < TR; ++u) v[u] = tz[ps * min(mine(pb + u * NW), L3 - 1)];
   };
   double k0[8], tv[TR];
-  load_k(4 * w, k0);
-  load_columns<ZB_NT>(lds, bd, B.psi, ct.q0, ct.nq);
+  load_k(4 * mine(w), k0);
+  load_columns<ZB_NT, 2, C>(lds, bd, B.psi, ct.q0, ct.nq);
   __syncthreads();
   load_tz(w, tv);
   double o[MI][8];   // c, then d
@@ -287,13 +315,13 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
     const double ks = bd.kscale[2];
 #pragma unroll
     for (int m = 0; m < MI; ++m) {
-      const int i0 = 4 * (w + m * NW);
+      const int i0 = 4 * mine(w + m * NW);
       if (i0 < N3) {
         double k[8];
         if (m > 0) load_k(i0, k);
 #pragma unroll
         for (int r = 0; r < 8; ++r) o[m][r] = 0.0;
-        kin_taps(i0 - 14, N3, per, [&](int kk, int z) {
+        kin_taps<SUB>(i0 - 14, N3, per, [&](int kk, int z) {
           kin_tap(kk, c[z * NL], d[z * NL], o[m], o[m] + 4);
         });
 #pragma unroll
@@ -309,21 +337,21 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
     }
   }
   __syncthreads();
-  for (int pb = w; pb < L3; pb += NW * TR) {
+  for (int pb = w; SUB * pb < L3; pb += NW * TR) {
     if (pb > w) load_tz(pb, tv);
 #pragma unroll
     for (int u = 0; u < TR; ++u)
-      if (pb + u * NW < L3) lds[(pb + u * NW) * NL + lane] = tv[u];
+      if (mine(pb + u * NW) < L3) lds[mine(pb + u * NW) * NL + lane] = tv[u];
   }
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < MI; ++m) {
-    const int i0 = 4 * (w + m * NW);
+    const int i0 = 4 * mine(w + m * NW);
     if (i0 < N3) {
       // summed by itself: on top of the larger kinetic term every tap would
       // round at its size
       double g[8] = {};
-      line_taps<37>(per ? 2 * i0 - 14 : 2 * i0, L3, per, [&](int qq, int p) {
+      line_taps<37, SUB>(per ? 2 * i0 - 14 : 2 * i0, L3, per, [&](int qq, int p) {
         shrink_tap<double, 4>(qq, lds[p * NL + lane], g, g + 4);
       });
 #pragma unroll
@@ -335,11 +363,11 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
   // the sums as records: row i3, element e of RecElem (lane's component
   // s + 4 s3, s = lane / CC; component 0 is the scaling coefficient)
   {
-    const int col = lane & (CC - 1), s = lane / CC;
-    const int ec = s == 0 ? col : CC + 7 * col + s - 1, ed = CC + 7 * col + s + 3;
+    const int col = lane & (C - 1), s = lane / C;
+    const int ec = s == 0 ? col : C + 7 * col + s - 1, ed = C + 7 * col + s + 3;
 #pragma unroll
     for (int m = 0; m < MI; ++m) {
-      const int i0 = 4 * (w + m * NW);
+      const int i0 = 4 * mine(w + m * NW);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (i0 + r < N3) {
@@ -350,16 +378,16 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
   }
   __syncthreads();
   {
-    constexpr int ZS = ZB_NT / 128, UR = 8;
-    const int e = threadIdx.x & 127, npl = bd.N[0] * bd.N[1];
-    const RecElem re(e);
+    constexpr int EL = 8 * C, ZS = ZB_NT / EL, UR = 8;
+    const int e = threadIdx.x & (EL - 1), npl = bd.N[0] * bd.N[1];
+    const RecElem<C> re(e);
     if (re.col < ct.nq) {
       char* dst = (char*)(B.hpsi + bd.psi_off);
       const unsigned off = re.t == 0 ? 0u : 8u * (unsigned)(bd.nvctr_c + re.t - 1);
       const unsigned mul = re.t == 0 ? 8u : 56u;
       const int lin0 = ct.q0 + re.col;
       const int* inv = re.t == 0 ? bd.cinv : bd.finv;
-      for (int zb = threadIdx.x >> 7; zb < N3; zb += ZS * UR) {
+      for (int zb = threadIdx.x / EL; zb < N3; zb += ZS * UR) {
         int rec[UR];
         double v[UR];
 #pragma unroll
@@ -392,19 +420,20 @@ __global__ __launch_bounds__(ZB_NT, WPE) void k_zback(Batch B, TileTable tt, Til
 // per coefficient, 5.2 TB/s: bound by memory), k_xykin 0.53, the update of r
 // 0.23.
 // ---------------------------------------------------------------------------
-constexpr int PZ_NT = 512;
-template <int MODE>
-__global__ __launch_bounds__(PZ_NT, 6) void k_pcz(Batch B, TileTable tt, PcArgs P) {
-  constexpr int NW = PZ_NT / 64, ZS = PZ_NT / 128, UR = MODE == 2 ? 4 : 8;
+template <int MODE, int PZ_NT, int WPE, int C = CC>
+__global__ __launch_bounds__(PZ_NT, WPE) void k_pcz(Batch B, TileTable tt, PcArgs P) {
+  constexpr int NW = PZ_NT / 64, NL = 4 * C, SUB = CC / C, EL = 8 * C, ZS = PZ_NT / EL,
+                UR = MODE == 2 ? 4 : 8;
   extern __shared__ __align__(16) unsigned char smem[];
   double* lds = (double*)smem;
   const int tile = tile_of(tt);
-  const int b = find_box(tt, tile);
+  const int lb = find_box(tt, tile);
+  const int b = table_box(tt, lb);
   const BoxDesc bd = B.box[b];
   const int N3 = bd.N[2], per = bd.per, npl = bd.N[0] * bd.N[1];
-  const ColTile ct(bd, tile - box_first_tile(tt, b));
+  const ColTile<C> ct(bd, tile - box_first_tile(tt, lb));
   {
-    const RecElem re(threadIdx.x & 127);
+    const RecElem<C> re(threadIdx.x & (EL - 1));
     const bool on = re.col < ct.nq;
     const int lin0 = ct.q0 + (on ? re.col : 0);
     const int* inv = re.t == 0 ? bd.cinv : bd.finv;
@@ -415,8 +444,8 @@ __global__ __launch_bounds__(PZ_NT, 6) void k_pcz(Batch B, TileTable tt, PcArgs 
     const double sc = P.pc[9 * b + 1 + re.t];
     const double alpha = MODE == 2 ? P.sc[4 * b + 1] : 0.0;
     const double beta = MODE == 2 ? P.sc[4 * b + 2] : 0.0;
-    double* dst = lds + (re.t >> 2) * N3 * NL + re.col + CC * (re.t & 3);
-    for (int zb = threadIdx.x >> 7; zb < N3; zb += ZS * UR) {
+    double* dst = lds + (re.t >> 2) * N3 * NL + re.col + C * (re.t & 3);
+    for (int zb = threadIdx.x / EL; zb < N3; zb += ZS * UR) {
       int e[UR];
       double v[UR], rv[UR], xv[UR];
 #pragma unroll
@@ -447,17 +476,19 @@ __global__ __launch_bounds__(PZ_NT, 6) void k_pcz(Batch B, TileTable tt, PcArgs 
     }
   }
   __syncthreads();
-  const double* c = lds + (threadIdx.x & 63);
+  const ZLane<C> zl;
+  const double* c = lds + zl.line;
   const double* d = c + N3 * NL;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t ps = 4 * (size_t)npl;
   const double ks = bd.kscale[2], cp = P.pc[9 * b];
   double* K = (double*)B.K + bd.w_off + ct.at;
-  for (int i0 = 4 * w; i0 < N3; i0 += 4 * NW) {
+  for (int iw = 4 * SUB * w; iw < N3; iw += 4 * SUB * NW) {
+    const int i0 = iw + 4 * zl.sub;
     double o[8];
 #pragma unroll
     for (int h = 0; h < 8; ++h) o[h] = 0.0;
-    kin_taps(i0 - 14, N3, per,
+    kin_taps<SUB>(i0 - 14, N3, per,
                   [&](int kk, int z) { kin_tap(kk, c[z * NL], d[z * NL], o, o + 4); });
     if (ct.on) {
 #pragma unroll
@@ -1315,7 +1346,7 @@ __global__ __launch_bounds__(NTM, WPE) void k_xlines_kin(Batch B, TileTable tt) 
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // 128 threads per 16 records of a row, as load_columns
-  const RecElem re(threadIdx.x & 127);
+  const RecElem<> re(threadIdx.x & 127);
   const int z0 = threadIdx.x >> 7, nit = CC * ((N1 + CC - 1) / CC);
   const char* src = (const char*)(B.psi + bd.psi_off);
   const unsigned off = re.t == 0 ? 0u : 8u * (unsigned)(bd.nvctr_c + re.t - 1);
@@ -1484,11 +1515,15 @@ __global__ __launch_bounds__(256) void k_xyden_sum(DenArgs D) {
 // ---------------------------------------------------------------------------
 // LDS bytes of the kernels for a box
 constexpr size_t LDS_STATIC = 128;   // the kernels' static LDS (reductions)
-static size_t lds_w(int N3) { return (size_t)NL * 2 * N3 * 8; }   // rows of W
-static size_t lds_z(int N3, int L3) { return (size_t)NL * (L3 > 2 * N3 ? L3 : 2 * N3) * 8; }
-size_t fp64_fit_z(const BoxDesc& b, size_t plane_lds) {
-  const size_t v = lds_z(b.N[2], b.L[2]);
-  return v + LDS_STATIC <= plane_lds ? v : 0;
+// rows of W; of W or of TZ
+static size_t lds_w(int N3, int cols = CC) { return (size_t)4 * cols * 2 * N3 * 8; }
+size_t fp64_lds_z(const BoxDesc& b, int cols) {
+  return (size_t)4 * cols * std::max(b.L[2], 2 * b.N[2]) * 8;
+}
+int fp64_zcols(const BoxDesc& b, size_t plane_lds) {
+  for (int cols : {CC, CC / 2})
+    if (fp64_lds_z(b, cols) + LDS_STATIC <= plane_lds) return cols;
+  return 0;
 }
 static size_t fp64_lds_kin(int N1, int N2) {
   return 8 * ((size_t)(2 * N2 + 1) * pair_stride(N1) + map_len(N2)) + 4 * map_len(N1);
@@ -1552,27 +1587,45 @@ PlaneFit fp64_fit_pot(const BoxDesc& b, size_t plane_lds) {
                    plane_lds);
 }
 
+// the z kernels over the boxes of each tile width (shape 2: 16 columns, 1: 8):
+// f(table, tiles, shape, longest line, LDS of the back pass)
+template <typename F>
+static hipError_t z_pass(const PassTables& PT, F f) {
+  if (PT.n_zg == 0)
+    return PT.ntiles[P_CZ] <= 0 ? hipSuccess
+                                : f(PT.t[P_CZ], PT.ntiles[P_CZ], PT.shape_zg[0], PT.len_zg[0],
+                                    PT.lds_zg[0]);
+  hipError_t e = hipSuccess;
+  for (int k = 0; k < PT.n_zg && e == hipSuccess; ++k)
+    e = f(PT.zg[k], PT.nt_zg[k], PT.shape_zg[k], PT.len_zg[k], PT.lds_zg[k]);
+  return e;
+}
 // 256 threads; more where long lines leave LDS for few work-groups per CU
-static hipError_t launch_zgrow(const Batch& B, const TileTable& t, int ntiles, int maxN3,
-                               hipStream_t s) {
-  const size_t lds = lds_w(maxN3);
-  if (ntiles <= 0) return hipSuccess;
-  if (maxN3 <= 64) k_zgrow<256><<<ntiles, 256, lds, s>>>(B, t);
-  else if (maxN3 <= 80) k_zgrow<512><<<ntiles, 512, lds, s>>>(B, t);
-  else k_zgrow<1024><<<ntiles, 1024, lds, s>>>(B, t);
-  return hipGetLastError();
+static hipError_t launch_zgrow(const Batch& B, const PassTables& PT, hipStream_t s) {
+  return z_pass(PT, [&](const TileTable& t, int n, int shape, int n3, size_t) {
+    const size_t lds = lds_w(n3);
+    if (shape == 1) k_zgrow<1024, CC / 2><<<n, 1024, lds_w(n3, CC / 2), s>>>(B, t);
+    else if (n3 <= 64) k_zgrow<256><<<n, 256, lds, s>>>(B, t);
+    else if (n3 <= 80) k_zgrow<512><<<n, 512, lds, s>>>(B, t);
+    else k_zgrow<1024><<<n, 1024, lds, s>>>(B, t);
+    return hipGetLastError();
+  });
 }
 // The launch shape says which chunks of a line a wave adds to its ekin sum, so
-// it follows the longest line n3 of the whole batch: a part of a chunked batch
-// that chose by its own lines summed 33 to 64 points in another order.
-static hipError_t launch_zback(const Batch& B, const TileTable& t, const TileTable& ft,
-                               int ntiles, size_t lds, int n3, double* part, hipStream_t s) {
-  if (ntiles <= 0) return hipSuccess;
-  if (n3 <= 32) k_zback<512, 1, 4><<<ntiles, 512, lds, s>>>(B, t, ft, part);
-  else if (n3 <= 48) k_zback<768, 1, 6><<<ntiles, 768, lds, s>>>(B, t, ft, part);
-  else if (n3 <= 64) k_zback<512, 2, 4><<<ntiles, 512, lds, s>>>(B, t, ft, part);
-  else k_zback<1024, 3, 4><<<ntiles, 1024, lds, s>>>(B, t, ft, part);
-  return hipGetLastError();
+// it follows the longest line of the whole batch (zb_n3, of the boxes in tiles
+// of 16 columns): a part of a chunked batch that chose by its own lines summed
+// 33 to 64 points in another order.
+static hipError_t launch_zback(const Batch& B, const PassTables& PT, hipStream_t s) {
+  const TileTable& ft = PT.t[P_CZ];
+  double* part = PT.part[0];
+  return z_pass(PT, [&](const TileTable& t, int n, int shape, int, size_t lds) {
+    if (shape == 1) k_zback<1024, 2, 4, CC / 2><<<n, 1024, lds, s>>>(B, t, ft, part);
+    else if (PT.zb_n3 <= 32) k_zback<512, 1, 4><<<n, 512, lds, s>>>(B, t, ft, part);
+    else if (PT.zb_n3 <= 48) k_zback<768, 1, 6><<<n, 768, lds, s>>>(B, t, ft, part);
+    else if (PT.zb_n3 <= 64) k_zback<512, 2, 4><<<n, 512, lds, s>>>(B, t, ft, part);
+    else k_zback<1024, 3, 4><<<n, 1024, lds, s>>>(B, t, ft, part);
+    return hipGetLastError();
+  });
 }
 template <int PC>
 static hipError_t launch_xykin(const Batch& B, const TileTable& t, const TileTable& ft,
@@ -1644,8 +1697,9 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
   // work-group on a CU (32^3 x 300: 1.955 of 1.960 ms, 40^3 x 128: 1.760 of
   // 1.745).
   const int nz = PT.ntiles[P_CZ], nx = PT.ntiles[P_PF];
-  if (!ev && !PT.kin_lines && PT.n_pfg == 0 && PT.shape_pfg[0] >= 2 && nz + nx <= FP64_JOIN) {
-    const size_t lds = std::max(lds_w(PT.maxN3), PT.lds_pfg[0]);
+  if (!ev && !PT.kin_lines && PT.n_pfg == 0 && PT.shape_pfg[0] >= 2 && nz + nx <= FP64_JOIN &&
+      PT.n_zg == 0 && PT.shape_zg[0] == 2) {
+    const size_t lds = std::max(lds_w(PT.len_zg[0]), PT.lds_pfg[0]);
     const TileTable &tz = PT.t[P_CZ], &tx = PT.t[P_PF];
     if (nz + nx <= 0) return hipSuccess;
     if (PT.nthr_pfg[0] <= 256) k_zgrow_xykin<256><<<nz + nx, 256, lds, s>>>(B, tz, tx, nx);
@@ -1654,7 +1708,7 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
     e = hipGetLastError();
   } else {
     mark(S_ZG, 0);
-    e = launch_zgrow(B, PT.t[P_CZ], nz, PT.maxN3, s);
+    e = launch_zgrow(B, PT, s);
     mark(S_ZG, 1);
     // one launch per group of boxes, or one over all of them
     mark(S_KXY, 0);
@@ -1673,8 +1727,7 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
   mark(S_XYP, 1);
   mark(S_ZB, 0);
   if (e == hipSuccess)
-    e = launch_zback(B, PT.t[P_CZ], PT.t[P_CZ], PT.ntiles[P_CZ], PT.lds_cz, PT.zb_n3,
-                     PT.part[0], s);
+    e = launch_zback(B, PT, s);
   mark(S_ZB, 1);
   if (e != hipSuccess) return e;
   EnergyTables et;
@@ -1697,7 +1750,7 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
 
 hipError_t launch_fp64_density(const Batch& B, const PassTables& PT, const DenArgs& D, int L3,
                                hipStream_t s) {
-  hipError_t e = launch_zgrow(B, PT.t[P_CZ], PT.ntiles[P_CZ], PT.maxN3, s);
+  hipError_t e = launch_zgrow(B, PT, s);
   if (e != hipSuccess) return e;
   const int n = D.ngroups * L3;
   const size_t lds = PT.lds_pbg[0];
@@ -1709,17 +1762,25 @@ hipError_t launch_fp64_density(const Batch& B, const PassTables& PT, const DenAr
   return hipGetLastError();
 }
 
+template <int MODE>
+static hipError_t launch_pcz(const Batch& B, const PassTables& PT, const PcArgs& P,
+                             hipStream_t s) {
+  return z_pass(PT, [&](const TileTable& t, int n, int shape, int n3, size_t) {
+    if (shape == 1)
+      k_pcz<MODE, 1024, 4, CC / 2><<<n, 1024, lds_w(n3, CC / 2), s>>>(B, t, P);
+    else
+      k_pcz<MODE, 512, 6><<<n, 512, lds_w(n3), s>>>(B, t, P);
+    return hipGetLastError();
+  });
+}
+
 // c W + K_z W + K_x W + K_y W of W = S v and the compressed sums that follow
 // (mode 0: v = x, r = d = b - A x; 1: v = d; 2: x and d of the step first)
 hipError_t launch_fp64_pc_apply(const Batch& B, const PassTables& PT, const PcArgs& P, int mode,
                                 hipStream_t s) {
-  const int n = PT.ntiles[P_CZ];
-  const TileTable& t = PT.t[P_CZ];
-  const size_t lds = lds_w(PT.maxN3);
-  if (mode == 0) k_pcz<0><<<n, PZ_NT, lds, s>>>(B, t, P);
-  else if (mode == 1) k_pcz<1><<<n, PZ_NT, lds, s>>>(B, t, P);
-  else k_pcz<2><<<n, PZ_NT, lds, s>>>(B, t, P);
-  const hipError_t e = hipGetLastError();
+  const hipError_t e = mode == 0   ? launch_pcz<0>(B, PT, P, s)
+                       : mode == 1 ? launch_pcz<1>(B, PT, P, s)
+                                   : launch_pcz<2>(B, PT, P, s);
   if (e != hipSuccess) return e;
   return mode == 0 ? xykin_pass<1>(B, PT, P, s) : xykin_pass<2>(B, PT, P, s);
 }
@@ -1741,7 +1802,11 @@ void fp64_attributes(size_t lds) {
                      (const void*)k_xykin<S2_NT, 6, 0>, (const void*)k_xypot<S2_NT, 2, 6>,
                      (const void*)k_xykin<S2_NT, 6, 1>, (const void*)k_xykin<S2_NT, 6, 2>,
                      (const void*)k_xykin<S1_NT, 4, 1>, (const void*)k_xykin<S1_NT, 4, 2>,
-                     (const void*)k_pcz<0>, (const void*)k_pcz<1>, (const void*)k_pcz<2>,
+                     (const void*)k_pcz<0, 512, 6>, (const void*)k_pcz<1, 512, 6>,
+                     (const void*)k_pcz<2, 512, 6>, (const void*)k_pcz<0, 1024, 4, CC / 2>,
+                     (const void*)k_pcz<1, 1024, 4, CC / 2>,
+                     (const void*)k_pcz<2, 1024, 4, CC / 2>,
+                     (const void*)k_zgrow<1024, CC / 2>, (const void*)k_zback<1024, 2, 4, CC / 2>,
                      (const void*)k_xykin<S1_NT, 4, 0>, (const void*)k_xypot<S1_NT, 3, 4>};
   for (const void* f : k)
     if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=

@@ -42,7 +42,8 @@ struct BoxDesc {
   int nvctr_c, nvctr_f;
   int potdim[3];        // potential box extents (n1ip, n2ip, n3ip)
   int ishift[3];        // potential box offset in wavefunction box coordinates
-  int pad_;
+  int zcol;             // FP64 sequence: coarse columns per z-line tile (CCOL,
+                        // or CCOL / 2 for long lines; 0: the lines do not fit)
   double kscale[3];     // -1/2/h_d^2, coarse grid spacing
   long long w_off;      // offset of the wavelet volume (8 N1 N2 N3)
   long long t1_off;     // offset of (L1, 2N2, 2N3)
@@ -401,13 +402,13 @@ __device__ __forceinline__ float t2_line_unscale(const Batch& B, const BoxDesc& 
 // P_ZP: z lines by rows of x (32 lines of one y per tile); P_ZPF: the same
 // lines as one run x + L1 y, 32 consecutive lines per tile (a tile may span
 // two rows), so that only a box's last tile is partly empty (k_zpot).
-// P_CZ: runs of CCOL coarse columns (z lines of the FP64 sequence); P_RP:
+// P_CZ: runs of BoxDesc::zcol coarse columns (z lines of the FP64 sequence); P_RP:
 // real-z planes of its potential pass; where planes do not fit in LDS, P_XK:
 // runs of CCOL rows of coarse points (x lines), P_YK: CCOL coarse x of one
 // coarse z (y lines), P_XR: 64 x lines of TZ, P_YL: 64 y lines of (L1, L3).
 enum Pass { P_UNC = 0, P_XF, P_YF, P_KY, P_KZ, P_ZP, P_YB, P_XB, P_PF, P_PB, P_KZG, P_ZPG,
             P_ZPF, P_CZ, P_RP, P_XK, P_YK, P_XR, P_YL, P_COUNT };
-constexpr int CCOL = 16;    // coarse columns (64 z lines) per P_CZ tile
+constexpr int CCOL = 16;    // coarse columns (64 z lines) per P_CZ tile (long lines: half)
 constexpr int ZGROUP = 3;   // bundles per z-line tile unless LDS asks for 2
 
 struct PassTables {
@@ -443,11 +444,17 @@ struct PassTables {
   size_t lds_pbg[4];
   int shape_pbg[4], nthr_pbg[4];
   int n_pbg;
-  // z-line kernels of the FP64 sequence: LDS and longest line of the batch
-  size_t lds_cz;
-  int maxN1, maxN2, maxN3, maxL1, maxL2;
+  // z-line kernels of the FP64 sequence: the boxes in groups by the columns of
+  // their tiles (shape 2: CCOL, 1: half), one launch per group; a group's
+  // longest line and the LDS of its back pass
+  TileTable zg[4];
+  int nt_zg[4];
+  size_t lds_zg[4];
+  int shape_zg[4], len_zg[4];
+  int n_zg;
   int zb_n3;    // longest z line that k_zback's launch shape is chosen for (of
                 // the whole batch where it runs in parts)
+  int maxN1, maxN2, maxL1, maxL2;
   // FP64 sequence: x-y kinetic, potential pass on lines (some plane does not
   // fit in LDS)
   int kin_lines, pot_lines;
@@ -621,8 +628,10 @@ hipError_t launch_mfma(const Batch& B, const PassTables& PT, const MfmaLds& L,
                        long long wtotal, bool need_zero, int precision, hipStream_t s,
                        hipEvent_t* ev, const Fork* fk = nullptr);
 // FP64 sequence (bdft_fp64.hip)
-// LDS bytes of the z-line kernels for a box, 0: they do not fit
-size_t fp64_fit_z(const BoxDesc& b, size_t plane_lds);
+// columns of a box's z-line tiles (CCOL or half; 0: they do not fit), and LDS
+// bytes of the back pass on them
+int fp64_zcols(const BoxDesc& b, size_t plane_lds);
+size_t fp64_lds_z(const BoxDesc& b, int cols);
 // launch shape of an in-plane kernel for a box: shape (1-4, of the boxes that
 // share a launch; 0: the plane does not fit), threads and LDS bytes
 struct PlaneFit {

@@ -320,3 +320,76 @@ def test_parts_of_a_batch_sum_ekin_as_the_whole(ctx, how):
             assert torch.equal(a, b)
     for l in lr.values():
         l.close()
+
+
+# z lines beyond the 64-line tiles (159 periodic, 145 free points), in tiles of
+# 32: the first lengths, a partly empty last tile of eight columns, lines whose
+# last pair of chunks is half empty, the longest lines of the library
+LONG = [("P", n) for n in [(1, 0, 159), (4, 3, 160), (2, 2, 163), (6, 5, 199), (3, 4, 255)]] + \
+       [("F", n) for n in [(0, 1, 145), (4, 3, 146), (5, 2, 180), (3, 4, 255)]]
+LONG_IDS = [f"{g}{n[0]}x{n[1]}x{n[2]}" for g, n in LONG]
+
+
+@pytest.mark.parametrize("geo,n", LONG, ids=LONG_IDS)
+@pytest.mark.parametrize("keys", ["dense", "sparse"])
+def test_long_z_lines_match_the_oracle(ctx, geo, n, keys):
+    test_launch_edges_match_the_oracle(ctx, geo, n, keys)
+    if keys == "dense":
+        test_density_launch_edges_match_the_oracle(ctx, geo, n, [0, 1, 1])
+    test_precond_launch_edges_match_the_oracle(ctx, geo, n, keys)
+
+
+def test_long_z_lines_keep_the_plane_kernels(ctx):
+    """a batch with z lines of 20, 60, 200 and 256 points: boxes in z-line tiles of
+    both widths, no line pass runs; against the oracle, and the same bits in
+    chunks and in the fixed device array.  Then the preconditioner on it."""
+    ns = [("P", (23, 23, 199)), ("F", (7, 5, 19)), ("F", (4, 5, 255)), ("P", (5, 3, 59)),
+          ("F", (9, 7, 150))]
+    regs = [dense_region(g, n, (0.45, 0.4, 0.5)) for g, n in ns]
+    psi = [random_psi(r, 1, 121 + i)[0] for i, r in enumerate(regs)]
+    pots = [random_pot(r, 131 + i) for i, r in enumerate(regs)]
+    lrs = [ctx.region(r) for r in regs]
+    po = np.cumsum([0] + [p.size for p in pots])
+    so = np.cumsum([0] + [p.size for p in psi])
+    x, pot = dev(np.concatenate(psi)), dev(np.concatenate(pots))
+
+    def run(fn):
+        h = torch.zeros_like(x)
+        ek = torch.zeros(len(lrs), dtype=torch.float64, device="cuda")
+        ep = torch.zeros_like(ek)
+        fn(lrs, pot, x, h, ek, ep, pot_off=po[:-1], psi_off=so[:-1])
+        ctx.sync()
+        return h.cpu().numpy(), ek.cpu().numpy(), ep.cpu().numpy()
+    got = run(ctx.locham_batch)
+    ctx.set_option("chunk_mb", 4)
+    try:
+        cut = run(ctx.locham_batch)
+    finally:
+        ctx.set_option("chunk_mb", 0)
+    for other in (cut, run(ctx.locham_batch_fixed)):
+        for a, b in zip(got, other):
+            assert np.array_equal(a, b)
+    ctx.profile(True)
+    try:
+        run(ctx.locham_batch)
+        stages = ctx.profile_read()[0]
+    finally:
+        ctx.profile(False)
+    busy = sorted(stages, key=stages.get)[-4:]
+    assert set(busy) == {"z_grow", "xy_kin", "xy_pot", "z_back"}, stages
+    h = np.split(got[0], so[1:-1])
+    cpr, b = [0.3, 0.5, 0.7, 0.9, 1.1], [random_psi(r, 1, 141 + i)[0] for i, r in enumerate(regs)]
+    x0 = 0.05 * x
+    ctx.precond_cg(lrs, cpr, 3, x0, dev(np.concatenate(b)), psi_off=so[:-1])
+    x0 = np.split(x0.cpu().numpy(), so[1:-1])
+    for i, r in enumerate(regs):
+        print(f"box {i}", flush=True)
+        ho, eo, vo = oracle.locham(r.geocode, r.n, r.nfl, r.nfu, r.hgrid, okeys(r), pots[i],
+                                   psi[i][None])
+        assert np.abs(h[i] - ho[0]).max() < TOL * np.abs(ho).max()
+        assert rel_err(got[1][i:i + 1], eo) < TOL
+        assert rel_err(got[2][i:i + 1], vo) < TOL
+        want = oracle.precond_cg(r.geocode, r.n, r.hgrid, cpr[i], 3, okeys(r), 0.05 * psi[i], b[i])
+        assert np.abs(x0[i] - want).max() < 1e-10 * np.abs(want).max()
+    for lr in lrs:
+        lr.close()
