@@ -1614,12 +1614,21 @@ static hipError_t launch_zgrow(const Batch& B, const PassTables& PT, hipStream_t
 // The launch shape says which chunks of a line a wave adds to its ekin sum, so
 // it follows the longest line of the whole batch (zb_n3, of the boxes in tiles
 // of 16 columns): a part of a chunked batch that chose by its own lines summed
-// 33 to 64 points in another order.
+// 33 to 64 points in another order.  (Up to 32 points every shape has one chunk
+// per wave.)
+//
+// Lines of at most 16 points keep one to four waves busy; the idle ones of a
+// work-group of eight hold its CU's wave slots.  Two or four waves from two
+// work-groups per CU on: free boxes of 44 x 44 x 2, 128 of them 217 -> 106 us,
+// 20 x 20 x 1 x 256 90 -> 35 us, periodic 44 x 44 x 16 x 64 185 -> 140 us; a
+// single box loads faster with eight (16^3: 10.5 against 11.7 us).
 static hipError_t launch_zback(const Batch& B, const PassTables& PT, hipStream_t s) {
   const TileTable& ft = PT.t[P_CZ];
   double* part = PT.part[0];
   return z_pass(PT, [&](const TileTable& t, int n, int shape, int, size_t lds) {
     if (shape == 1) k_zback<1024, 2, 4, CC / 2><<<n, 1024, lds, s>>>(B, t, ft, part);
+    else if (PT.zb_n3 <= 8 && n > 512) k_zback<128, 1, 4><<<n, 128, lds, s>>>(B, t, ft, part);
+    else if (PT.zb_n3 <= 16 && n > 512) k_zback<256, 1, 4><<<n, 256, lds, s>>>(B, t, ft, part);
     else if (PT.zb_n3 <= 32) k_zback<512, 1, 4><<<n, 512, lds, s>>>(B, t, ft, part);
     else if (PT.zb_n3 <= 48) k_zback<768, 1, 6><<<n, 768, lds, s>>>(B, t, ft, part);
     else if (PT.zb_n3 <= 64) k_zback<512, 2, 4><<<n, 512, lds, s>>>(B, t, ft, part);
@@ -1796,6 +1805,7 @@ void fp64_attributes(size_t lds) {
                      (const void*)k_xlines_shrink<1024, 3, 4>,
                      (const void*)k_xlines_kin<768, 2, 6>, (const void*)k_xlines_kin<1024, 3, 4>,
                      (const void*)k_ylines_kin<768, 6>, (const void*)k_ylines_kin<1024, 4>, (const void*)k_zback<512, 1, 4>,
+                     (const void*)k_zback<128, 1, 4>,   (const void*)k_zback<256, 1, 4>,
                      (const void*)k_zback<768, 1, 6>,   (const void*)k_zback<512, 2, 4>,
                      (const void*)k_zback<1024, 3, 4>,
                      (const void*)k_xyden<512, 3, 4>, (const void*)k_xyden<S1_NT, 3, 4>,

@@ -393,3 +393,38 @@ def test_long_z_lines_keep_the_plane_kernels(ctx):
         assert np.abs(x0[i] - want).max() < 1e-10 * np.abs(want).max()
     for lr in lrs:
         lr.close()
+
+
+@pytest.mark.parametrize("geo", ["P", "F"])
+@pytest.mark.parametrize("n3", [1, 2, 7, 8, 9, 15, 16, 17])
+def test_flat_batches_match_the_oracle(ctx, geo, n3):
+    """more than 512 z-line tiles of short lines: the back pass runs two or four
+    waves per work-group (up to 8 or 16 points), in the chunks of a cut batch
+    (one box of 27 tiles or so each) eight; the same bits"""
+    reg = dense_region(geo, (19, 20, n3 - 1), (0.45, 0.4, 0.5))
+    norb = 20
+    print(f"case {geo} n3={n3}", flush=True)
+    psi, h0, pot = random_psi(reg, norb, 151), random_psi(reg, norb, 152), random_pot(reg, 153)
+    lr = ctx.region(reg)
+    d_pot, d_psi = dev(pot), dev(psi)
+
+    def run():
+        h = dev(h0)
+        ek = torch.zeros(norb, dtype=torch.float64, device="cuda")
+        ep = torch.zeros_like(ek)
+        ctx.locham(lr, d_pot, d_psi, h, ek, ep)
+        ctx.sync()
+        return h.cpu().numpy(), ek.cpu().numpy(), ep.cpu().numpy()
+    got = run()
+    ctx.set_option("chunk_mb", 1)
+    try:
+        cut = run()
+    finally:
+        ctx.set_option("chunk_mb", 0)
+    for a, b in zip(got, cut):
+        assert np.array_equal(a, b)
+    ho, eo, po = oracle.locham(geo, reg.n, reg.nfl, reg.nfu, reg.hgrid, okeys(reg), pot, psi, h0)
+    assert np.abs(got[0] - ho).max() < TOL * np.abs(ho - h0).max()
+    assert rel_err(got[1], eo) < TOL
+    assert rel_err(got[2], po) < TOL
+    lr.close()
