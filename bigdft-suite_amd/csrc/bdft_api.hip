@@ -1932,16 +1932,28 @@ extern "C" int bdft_density_d(bdft_ctx* ctx, const bdft_lr* lr, int norb, const 
   size_t nparts;
   const bool planes = plan->T.plane && precision == BDFT_PREC_FP64;
   if (planes) {
-    // the orbitals by spin, in groups of one spin: 1536 planes or so of
-    // work-groups (six per CU; more groups would only write more partials)
+    // the orbitals by spin, in groups of one spin
     meta.clear();
     for (int s = 0; s < nspin; ++s)
       for (int i = 0; i < norb; ++i)
         if (sp[i] == s) meta.push_back(i);
     for (int k = 0; k < norb; ++k) hf[k] = hfac[meta[k]];
     const int n0 = (int)std::count(sp.begin(), sp.end(), 0);
-    const int want = std::max(1, std::min(norb, cdiv(1536, lr->L[2])));
-    D.gsize = cdiv(norb, want);
+    // group size: the fewest trips of the resident work-groups, each over its
+    // group's orbitals and, a quarter as long as one of them, its partial density;
+    // and the groups that a thread of the sum adds up, eight in an orbital's time
+    // (44 x 44 x 1 free, 128 orbitals: 0.45 ms in 43 groups, 0.36 in 8 of one
+    // trip; periodic 64^3 x 16: 0.46 in 8, 0.40 in 2; 8^3 x 256: 0.16 in 128)
+    const long long res = fp64_den_resident(plan->T, ctx->plane_lds);
+    long long best = 0;
+    for (int g = norb; g >= 1; --g) {
+      const long long groups = cdiv(n0, g) + cdiv(norb - n0, g);
+      const long long cost = (groups * lr->L[2] + res - 1) / res * (8 * g + 2) + groups;
+      if (g == norb || cost < best) {
+        best = cost;
+        D.gsize = g;
+      }
+    }
     std::vector<int32_t> start;
     for (int k = 0; k < n0; k += D.gsize) start.push_back(k);
     D.gspin = (int)start.size();

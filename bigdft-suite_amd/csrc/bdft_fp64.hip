@@ -1757,16 +1757,23 @@ hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
   return hipGetLastError();
 }
 
+static int den_threads(const PassTables& PT) {
+  return PT.shape_pbg[0] >= 2 ? std::min(512, PT.nthr_pbg[0]) : PT.nthr_pbg[0];
+}
+// work-groups of k_xyden that 256 CUs hold at a time: 16 waves of 128 VGPRs and
+// plane_lds bytes of LDS each
+int fp64_den_resident(const PassTables& PT, size_t plane_lds) {
+  const size_t lds = std::max(PT.lds_pbg[0], (size_t)1);
+  return 256 * std::max(1, std::min(1024 / den_threads(PT), (int)(plane_lds / lds)));
+}
 hipError_t launch_fp64_density(const Batch& B, const PassTables& PT, const DenArgs& D, int L3,
                                hipStream_t s) {
   hipError_t e = launch_zgrow(B, PT, s);
   if (e != hipSuccess) return e;
-  const int n = D.ngroups * L3;
+  const int n = D.ngroups * L3, nt = den_threads(PT);
   const size_t lds = PT.lds_pbg[0];
-  if (PT.shape_pbg[0] >= 2)
-    k_xyden<512, 3, 4><<<n, std::min(512, PT.nthr_pbg[0]), lds, s>>>(B, D);
-  else
-    k_xyden<S1_NT, 3, 4><<<n, PT.nthr_pbg[0], lds, s>>>(B, D);
+  if (PT.shape_pbg[0] >= 2) k_xyden<512, 3, 4><<<n, nt, lds, s>>>(B, D);
+  else k_xyden<S1_NT, 3, 4><<<n, nt, lds, s>>>(B, D);
   k_xyden_sum<<<dim3((unsigned)((D.nisf + 255) / 256), D.nspin), 256, 0, s>>>(D);
   return hipGetLastError();
 }

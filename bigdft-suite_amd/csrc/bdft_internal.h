@@ -647,6 +647,7 @@ bool fp64_pot_lines_ok(const BoxDesc& b, size_t plane_lds);
 void fp64_attributes(size_t lds);
 hipError_t launch_fp64_pc_apply(const Batch& B, const PassTables& PT, const PcArgs& P, int mode,
                                 hipStream_t s);
+int fp64_den_resident(const PassTables& PT, size_t plane_lds);
 hipError_t launch_fp64_density(const Batch& B, const PassTables& PT, const DenArgs& D, int L3,
                                hipStream_t s);
 hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,

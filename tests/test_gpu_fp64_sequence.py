@@ -428,3 +428,17 @@ def test_flat_batches_match_the_oracle(ctx, geo, n3):
     assert rel_err(got[1], eo) < TOL
     assert rel_err(got[2], po) < TOL
     lr.close()
+
+
+# group sizes of every kind: all orbitals in one group, several trips of groups,
+# a last group partly full in both spins, one orbital of a spin, one spin empty
+GROUPS = [("F", (43, 43, 0), [0] * 40 + [1]), ("F", (39, 39, 1), [1] * 33),
+          ("F", (53, 53, 53), [0, 1]), ("P", (49, 49, 5), [k % 2 for k in range(25)]),
+          ("P", (3, 3, 3), [int(k % 3 == 0) for k in range(257)]),
+          ("P", (11, 9, 149), [k % 2 for k in range(9)])]
+
+
+@pytest.mark.parametrize("geo,n,spin", GROUPS,
+                         ids=[f"{g}{n[0]}x{n[1]}x{n[2]}-{len(s)}" for g, n, s in GROUPS])
+def test_density_groups_match_the_oracle(ctx, geo, n, spin):
+    test_density_launch_edges_match_the_oracle(ctx, geo, n, spin)
