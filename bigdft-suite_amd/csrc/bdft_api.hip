@@ -1109,6 +1109,25 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
       }
     }
     if (d64) fits = fits && (density ? pp : (kp || kl) && (pp || pl));
+    // Flat free boxes: z first makes 2 N3 + 29 planes for the x and y passes
+    // where x and y first make 2 N3.  From more than two planes per CU on the
+    // line passes win at one coarse z point if a plane fills a CU's LDS (256
+    // boxes of 43 x 43 x 1: 1.20 against 1.02 ms; x 2: 1.33 against 1.32, 50 x 50
+    // x 2 1.72 against 1.88), up to three if x and y go on lines (64 boxes of 60
+    // x 60 x 2: 0.77 against 0.67, x 3 0.84 against 0.78, x 4 0.89 against 0.91),
+    // while three of their work-groups fit a CU (68 x 68 x 1 x 128: 1.61 against
+    // 1.31, 70 x 70 x 1: 1.75 against 1.91)
+    if (d64 && !density && plane && fits) {
+      long long planes = 0;
+      bool flat = true;
+      for (const BoxDesc& b : box) {
+        planes += b.L[2];
+        flat = flat && !b.per && b.N[2] <= (pp ? 1 : 3) &&
+               fp64_fit_pot(b, ctx->plane_lds).shape < 2 &&
+               3 * (lds_bytes(std::max(b.N[0], b.N[1]), (int)esz) + 1024) <= ctx->plane_lds;
+      }
+      if (flat && planes > 512) plane = false;
+    }
     if (!fits || std::max(lpf, lpb) > ctx->plane_lds) plane = false;
     T.plane = plane ? 1 : 0;
     T.kin_lines = plane && d64 && !kp;

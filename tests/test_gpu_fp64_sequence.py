@@ -442,3 +442,37 @@ GROUPS = [("F", (43, 43, 0), [0] * 40 + [1]), ("F", (39, 39, 1), [1] * 33),
                          ids=[f"{g}{n[0]}x{n[1]}x{n[2]}-{len(s)}" for g, n, s in GROUPS])
 def test_density_groups_match_the_oracle(ctx, geo, n, spin):
     test_density_launch_edges_match_the_oracle(ctx, geo, n, spin)
+
+
+@pytest.mark.parametrize("n", [(42, 40, 0), (57, 59, 0), (57, 60, 1), (66, 60, 2)],
+                         ids=lambda n: "x".join(map(str, n)))
+def test_flat_free_batches_on_line_passes_match_the_oracle(ctx, n):
+    """flat free boxes with large planes: z first up to 512 planes, then the line
+    passes, of the whole batch also where it is cut into parts of fewer planes"""
+    reg = dense_region("F", n, (0.45, 0.4, 0.5))
+    psi, pot, lr = random_psi(reg, 20, 161), random_pot(reg, 162), ctx.region(reg)
+    for norb in (14, 20):   # 434 to 490 planes; 620 to 700
+        print(f"case {n} norb={norb}", flush=True)
+        x, v = dev(psi[:norb]), dev(pot)
+
+        def run():
+            h = torch.zeros_like(x)
+            ek = torch.zeros(norb, dtype=torch.float64, device="cuda")
+            ep = torch.zeros_like(ek)
+            ctx.locham(lr, v, x, h, ek, ep)
+            ctx.sync()
+            return h.cpu().numpy(), ek.cpu().numpy(), ep.cpu().numpy()
+        got = run()
+        ctx.set_option("chunk_mb", 4)
+        try:
+            cut = run()
+        finally:
+            ctx.set_option("chunk_mb", 0)
+        for a, b in zip(got, cut):
+            assert np.array_equal(a, b)
+        ho, eo, po = oracle.locham("F", reg.n, reg.nfl, reg.nfu, reg.hgrid, okeys(reg), pot,
+                                   psi[:norb], np.zeros_like(psi[:norb]))
+        assert np.abs(got[0] - ho).max() < TOL * np.abs(ho).max()
+        assert rel_err(got[1], eo) < TOL
+        assert rel_err(got[2], po) < TOL
+    lr.close()
