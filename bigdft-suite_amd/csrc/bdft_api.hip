@@ -2074,7 +2074,11 @@ static int xfer(bdft_ctx* ctx, const bdft_lr* glr, int norb, const bdft_lr* cons
                    "region transfers are defined between free-BC regions "
                    "(shift_locreg_indexes, locreg_operations.f90:2338-2343)");
   const long long gnc = (long long)glr->nvctr_c + 7LL * glr->nvctr_f;
-  std::vector<XferDesc> d((size_t)norb);
+  // descriptors and the counter of missing points, as they are uploaded
+  auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+  const size_t nb_d = sizeof(XferDesc) * norb, nb_up = al(nb_d) + sizeof(int);
+  std::vector<unsigned char> up(nb_up);
+  XferDesc* d = (XferDesc*)up.data();
   long long lacc = 0;
   long long tiles = 0;
   for (int i = 0; i < norb; ++i) {
@@ -2109,14 +2113,12 @@ static int xfer(bdft_ctx* ctx, const bdft_lr* glr, int norb, const bdft_lr* cons
   }
   if (tiles > 0x7fffffffLL) return set_err(ctx, BDFT_ERR_UNSUPPORTED, "batch too large");
   HIPCHK(ctx, hipSetDevice(ctx->device));
-  auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-  const size_t nb_d = sizeof(XferDesc) * norb;
   DevBuf& buf = ctx->xfer_buf;
-  const unsigned char* dh = (const unsigned char*)d.data();
+  const unsigned char* dh = up.data();
   const bool same = buf.p && ctx->xfer_last.size() == nb_d &&
                     std::memcmp(ctx->xfer_last.data(), dh, nb_d) == 0;
   hipError_t e = hipSuccess;
-  if (!ctx->xfer_flag) {
+  if (!to_local && !ctx->xfer_flag) {
     e = hipHostMalloc((void**)&ctx->xfer_flag, sizeof(int), hipHostMallocDefault);
     if (e != hipSuccess) {
       ctx->xfer_flag = nullptr;
@@ -2128,19 +2130,17 @@ static int xfer(bdft_ctx* ctx, const bdft_lr* glr, int norb, const bdft_lr* cons
     // the previous call's kernel may still read the descriptors
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     ctx->xfer_last.clear();
-    int rc = dev_alloc(ctx, buf, al(nb_d) + al(sizeof(int)));
+    int rc = dev_alloc(ctx, buf, nb_up);
     if (rc) return rc;
-    e = hipMemcpy(buf.p, dh, nb_d, hipMemcpyHostToDevice);
-    const int zero = 0;
-    if (e == hipSuccess)
-      e = hipMemcpy((char*)buf.p + al(nb_d), &zero, sizeof zero, hipMemcpyHostToDevice);
+    e = hipMemcpy(buf.p, dh, nb_up, hipMemcpyHostToDevice);
     if (e == hipSuccess) ctx->xfer_last.assign(dh, dh + nb_d);
   }
   char* q = (char*)buf.p;
-  // only scatters into the global orbital count missing points.  The counter
-  // is zero between calls and read only where a kernel has raised the host
-  // flag: clearing and copying it on every call took 40 of 175 us of a batch
-  // of 128 spheres in both directions
+  // only scatters into the global orbital count missing points (a gather needs
+  // no flag, whose allocation took 40 of 175 us of a context's first).  The
+  // counter is zero between calls and read only where a kernel has raised the
+  // host flag: clearing and copying it on every call took 40 of 175 us of a
+  // batch of 128 spheres in both directions
   int* miss = (int*)(q + al(nb_d));
   int nmiss = 0;
   if (e == hipSuccess) {
@@ -2161,7 +2161,7 @@ static int xfer(bdft_ctx* ctx, const bdft_lr* glr, int norb, const bdft_lr* cons
     e = launch_xfer(A, (int)tiles, ctx->stream);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  if (e == hipSuccess && *(volatile int*)ctx->xfer_flag) {
+  if (e == hipSuccess && !to_local && *(volatile int*)ctx->xfer_flag) {
     e = hipMemcpy(&nmiss, miss, sizeof(int), hipMemcpyDeviceToHost);
     *ctx->xfer_flag = 0;
     ctx->xfer_last.clear();   // the next call's upload clears the counter

@@ -186,3 +186,55 @@ def test_missing_points_are_counted_on_every_call(ctx):
     assert torch.equal(out, torch.ones_like(out))
     lr.close()
     g.close()
+
+
+def test_alternating_sets_of_regions(ctx):
+    """calls that alternate between sets of regions (new descriptors each time,
+    of more and of fewer regions), gathers before the context's first scatter,
+    and a set with missing points among them: bit-exact, every count its own"""
+    import bigdft_hip
+    from bigdft_hip.descriptors import region_from_grids
+    h = (0.4, 0.4, 0.4)
+    ng = (12, 11, 10)
+    cm = np.ones(tuple(x + 1 for x in ng), dtype=bool)
+    cm[10:, 9:, 8:] = False
+    glob = region_from_grids("F", ng, h, cm, np.zeros_like(cm))
+    own = bigdft_hip.Context(0)
+    g = own.region(glob)
+    # regions of coarse points only, as the global one
+    full = {n: np.ones(tuple(x + 1 for x in n), dtype=bool) for n in ((3, 2, 4), (6, 5, 3))}
+    small, big = (region_from_grids("F", n, h, m, np.zeros_like(m)) for n, m in full.items())
+    hl = {id(r): own.region(r) for r in (small, big)}
+    # 24 regions of one kind, 5 of both, 1 that reaches into the hole
+    sets = [([small] * 24, [(i % 5, i % 4, i % 3) for i in range(24)], 0),
+            ([big, small, big, small, small], [(0, 1, 2), (5, 4, 2), (3, 3, 3), (1, 0, 0), (6, 6, 3)], 0),
+            ([big], [(6, 6, 7)], 27)]
+    rng = np.random.default_rng(17)
+    psi = rng.standard_normal(glob.ncoef)
+    want = []
+    for regs, ns, miss in sets:
+        want.append(np.concatenate([oracle.psi_to_locreg2(r.n, ng, list(o), okeys(r), okeys(glob), psi)
+                                    for r, o in zip(regs, ns)]))
+    d_psi = dev(psi)
+    goff = {k: np.zeros(len(s[0]), dtype=np.int64) for k, s in enumerate(sets)}
+    for scatter in (False, True, True):
+        for _ in range(2):
+            for k, (regs, ns, miss) in enumerate(sets):
+                lrs = [hl[id(r)] for r in regs]
+                o = np.array(ns, dtype=np.int32)
+                lp = torch.full((want[k].size,), np.nan, dtype=torch.float64, device="cuda")
+                own.psi_to_locreg(g, lrs, o, d_psi, lp, goff=goff[k])
+                assert np.array_equal(lp.cpu().numpy(), want[k])
+                if not scatter:
+                    continue
+                back = d_psi.clone()
+                if miss:
+                    with pytest.raises(bigdft_hip.BigDFTError, match=f"^.*{miss} local points"):
+                        own.locreg_to_psi(g, lrs, o, lp, back, goff=goff[k])
+                else:
+                    own.locreg_to_psi(g, lrs, o, lp, back, goff=goff[k])
+                assert torch.equal(back, d_psi)
+    for l in hl.values():
+        l.close()
+    g.close()
+    own.close()
