@@ -1519,8 +1519,21 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   return BDFT_OK;
 }
 
+// Working grids of an orbital in bytes: K, TZ (on lines TX too) of the FP64
+// sequence, else W, K, T2, T1 (line passes) and T3 (long z lines)
+static size_t orbital_grids(const bdft_lr* lr, size_t esz, bool fp64_seq, bool pot_lines) {
+  const size_t n12 = (size_t)lr->N[0] * lr->N[1], W = 8 * n12 * lr->N[2];
+  if (fp64_seq)
+    return esz * (W + 4 * n12 * lr->L[2] +
+                  (pot_lines ? (size_t)2 * lr->N[1] * lr->L[0] * lr->L[2] : 0));
+  const size_t T2 = (size_t)lr->L[0] * lr->L[1] * 2 * lr->N[2];
+  const size_t T1 = (size_t)lr->L[0] * 4 * lr->N[1] * lr->N[2];
+  const size_t T3 = lr->L[2] > REG_L ? (size_t)lr->L[0] * lr->L[1] * lr->L[2] : 0;
+  return esz * (2 * W + T2 + T1 + T3);
+}
+
 // Chunked plan: orbitals split into consecutive ranges whose working grids
-// (W, K, T2, and T1 for line passes) take at most opt_chunk_mb MiB, each
+// (those of the sequence that the batch runs) take at most opt_chunk_mb MiB, each
 // range a plan of its own on one shared workspace, run in order.  A chunk's
 // grids are written and read again while they are still in the device's
 // last-level cache (256 MiB on MI355X) instead of making an HBM round trip
@@ -1535,25 +1548,20 @@ static int make_plan_chunked(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
                              bdft_plan** out, const bdft_confpot* conf = nullptr) {
   if (!ctx || !out) return BDFT_ERR_ARG;
   const size_t budget = (size_t)ctx->opt_chunk_mb << 20;
-  std::vector<size_t> need;
-  size_t total = 0;
-  if (budget && norb > 1 && lrs && psi) {
-    const size_t esz = precision == BDFT_PREC_FP64 ? 8 : 4;
-    need.resize((size_t)norb);
+  const size_t esz = precision == BDFT_PREC_FP64 ? 8 : 4;
+  // at most (whichever sequence it is)
+  size_t most = 0;
+  if (budget && norb > 1 && lrs && psi)
     for (int i = 0; i < norb; ++i) {
-      const bdft_lr* lr = lrs[i];
-      if (!lr) return set_err(ctx, BDFT_ERR_ARG, "orbital %d: region missing", i);
-      const size_t W = 8ull * lr->N[0] * lr->N[1] * lr->N[2];
-      const size_t T2 = (size_t)lr->L[0] * lr->L[1] * 2 * lr->N[2];
-      const size_t T1 = (size_t)lr->L[0] * 4 * lr->N[1] * lr->N[2];
-      const size_t T3 = lr->L[2] > REG_L ? (size_t)lr->L[0] * lr->L[1] * lr->L[2] : 0;
-      need[i] = esz * (2 * W + T2 + T1 + T3);
-      total += need[i];
+      if (!lrs[i]) return set_err(ctx, BDFT_ERR_ARG, "orbital %d: region missing", i);
+      most += std::max(orbital_grids(lrs[i], esz, false, false),
+                       esz == 8 ? orbital_grids(lrs[i], esz, true, true) : 0);
     }
-  }
-  if (!budget || total <= budget)
+  auto whole = [&] {
     return make_plan(ctx, norb, lrs, pot, pot_off, potdim, ishift, psi, psi_off, hpsi, ekin,
                      epot, precision, own_ws, out, false, conf);
+  };
+  if (!budget || most <= budget) return whole();
   *out = nullptr;
   // the whole batch's launch choices, imposed on every part
   PlanChoice choice{};
@@ -1562,6 +1570,13 @@ static int make_plan_chunked(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
                       epot, precision, own_ws, &none, false, conf, false, nullptr, true,
                       nullptr, &choice);
   if (rc0) return rc0;
+  std::vector<size_t> need((size_t)norb);
+  size_t total = 0;
+  for (int i = 0; i < norb; ++i) {
+    need[i] = orbital_grids(lrs[i], esz, esz == 8 && choice.plane, choice.pot_lines);
+    total += need[i];
+  }
+  if (total <= budget) return whole();
   std::vector<int64_t> so((size_t)norb), po((size_t)norb);
   long long run = 0;
   for (int i = 0; i < norb; ++i) {
@@ -1818,8 +1833,9 @@ extern "C" int bdft_locham_batch_fixed_d(bdft_ctx* ctx, int norb, const bdft_lr*
     return set_err(ctx, BDFT_ERR_UNSUPPORTED, "precision %d not available", precision);
   HIPCHK(ctx, hipSetDevice(ctx->device));
   const size_t cap = BDFT_FIXED_BYTES;
-  // working grids per orbital (W, K, T2, and T1 for line passes, T3 for
-  // long z lines), the bound a chunk is first cut to
+  // working grids per orbital as the line passes have them: what the entry
+  // admits, and the bound a chunk is first cut to (the tables lie beside the
+  // grids, so a chunk that does not fit after all is halved)
   const size_t esz = precision == BDFT_PREC_FP64 ? 8 : 4;
   std::vector<size_t> need((size_t)norb);
   std::vector<int64_t> so((size_t)norb), po((size_t)norb);
@@ -1828,11 +1844,7 @@ extern "C" int bdft_locham_batch_fixed_d(bdft_ctx* ctx, int norb, const bdft_lr*
     const bdft_lr* lr = lrs[i];
     if (!lr || lr->ctx != ctx)
       return set_err(ctx, BDFT_ERR_ARG, "orbital %d: region missing or from another context", i);
-    const size_t W = 8ull * lr->N[0] * lr->N[1] * lr->N[2];
-    const size_t T2 = (size_t)lr->L[0] * lr->L[1] * 2 * lr->N[2];
-    const size_t T1 = (size_t)lr->L[0] * 4 * lr->N[1] * lr->N[2];
-    const size_t T3 = lr->L[2] > REG_L ? (size_t)lr->L[0] * lr->L[1] * lr->L[2] : 0;
-    need[i] = esz * (2 * W + T2 + T1 + T3);
+    need[i] = orbital_grids(lr, esz, false, false);
     if (need[i] > cap)
       return set_err(ctx, BDFT_ERR_UNSUPPORTED,
                      "orbital %d needs %zu bytes of working grids, the fixed device array "

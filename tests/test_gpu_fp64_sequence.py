@@ -476,3 +476,41 @@ def test_flat_free_batches_on_line_passes_match_the_oracle(ctx, n):
         assert rel_err(got[1], eo) < TOL
         assert rel_err(got[2], po) < TOL
     lr.close()
+
+
+@pytest.mark.parametrize("geo,n,norb,mb", [("F", (49, 49, 1), 64, 64), ("P", (23, 23, 23), 48, 32),
+                                           ("P", (71, 72, 5), 24, 48)],
+                         ids=["flat_free", "periodic", "lines"])
+def test_chunks_keep_to_their_size(ctx, geo, n, norb, mb):
+    """a plan cut into chunks of mb MiB holds at most that much in working grids
+    (FP64: K and TZ, 2.9 MB a flat free box, and TX on lines) and not less than
+    half of it; with the bits of one chunk"""
+    reg = dense_region(geo, n, (0.45, 0.4, 0.5))
+    lr = ctx.region(reg)
+    psi, pot = dev(random_psi(reg, norb, 171)).ravel(), dev(random_pot(reg, 172))
+
+    def run():
+        h = torch.zeros_like(psi)
+        ek = torch.zeros(norb, dtype=torch.float64, device="cuda")
+        ep = torch.zeros_like(ek)
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        plan = ctx.plan([lr] * norb, pot, psi, h, ek, ep)
+        used = before - torch.cuda.mem_get_info()[0]
+        plan.execute()
+        ctx.sync()
+        plan.close()
+        return used, (h, ek, ep)
+    run()   # (the first plan also sets up what the runtime keeps)
+    whole, one = run()
+    ctx.set_option("chunk_mb", mb)
+    try:
+        used, cut = run()
+    finally:
+        ctx.set_option("chunk_mb", 0)
+    print(f"case {geo} {n}: {whole >> 20} MiB in one chunk, {used >> 20} of {mb}", flush=True)
+    assert whole > 1.3 * mb * 2 ** 20
+    assert mb * 2 ** 19 < used < (mb + 8) * 2 ** 20   # tables and allocation units beside
+    for a, b in zip(one, cut):
+        assert torch.equal(a, b)
+    lr.close()
