@@ -235,7 +235,16 @@ def tune(ctx, lrs, pot, psi, precision, cache=None, timer=time_plan, check=check
     # then the tile order of the plane and (un)compress passes, then the
     # persistent z potential pass
     trial(dict(best[1], tile_order=1))
-    trial(dict(best[1], persist=1))
+    late = dict(best[1], persist=1)
+    if PREC_NAMES.get(precision) == "fp64" and not late["line_passes"]:
+        # the FP64 sequence has no such pass; where the automatic choice is the
+        # line passes they are timed alike, and the pass is theirs
+        auto, lines = (times.get(cand_name(c)) for c in candidates(precision))
+        late["line_passes"] = 1
+        if auto is None or lines is None or abs(lines - auto) > REFINE * auto:
+            late = None
+    if late is not None:
+        trial(late)
     # one timing carries a few per cent of noise: the candidates within
     # REFINE of the fastest are timed REFINE_ROUNDS more times, in turn, and
     # the mean of all their timings decides

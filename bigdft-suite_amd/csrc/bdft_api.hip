@@ -1341,10 +1341,11 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     for (int k = 0; k < T.n_zg; ++k)
       tb_z[k] = T.nt_zg[k] <= TB_MAX ? tiles_of(zg_off[k][0], T.zg[k].nbox) : -1;
   }
-  // work queue of the persistent z potential pass: the boxes in order of
-  // decreasing work (fine points), each box's tiles together
+  const bool fp64_seq = T.plane && esz == 8;
+  // work queue of the persistent z potential pass (the FP64 sequence has none):
+  // the boxes in order of decreasing work (fine points), each box's tiles together
   int zq_off = -1;
-  if (ctx->opt_persist == 1 && T.ntiles[P_ZPF] > 0) {
+  if (ctx->opt_persist == 1 && T.ntiles[P_ZPF] > 0 && !fp64_seq) {
     std::vector<int> order((size_t)norb);
     for (int i = 0; i < norb; ++i) order[i] = i;
     auto work = [&](int i) { return (long long)box[i].L[0] * box[i].L[1] * box[i].L[2]; };
@@ -1359,7 +1360,6 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   }
   const size_t nb_st = sizeof(int) * starts.size();
   int epass[4] = {P_XF, P_KY, P_KZ, P_ZP};
-  const bool fp64_seq = T.plane && esz == 8;
   if (fp64_seq) {
     epass[0] = P_CZ;
     epass[3] = T.pot_lines ? P_YL : P_RP;

@@ -166,3 +166,24 @@ def test_close_candidates_are_timed_again(tmp_path):
     assert calls[lucky] == 1 + autotune.REFINE_ROUNDS
     assert times[lucky] == pytest.approx((3.5 + autotune.REFINE_ROUNDS * 4.2) /
                                          (1 + autotune.REFINE_ROUNDS))
+
+
+@pytest.mark.parametrize("lines,tried", [(9.0, False), (5.1, True), (3.0, True)])
+def test_fp64_has_the_persistent_pass_on_line_passes_only(tmp_path, lines, tried):
+    """the FP64 plane sequence has no z potential pass: the persistent launch is
+    timed only as an option of the line passes, where they are chosen or are
+    what the automatic choice runs (they take its time)"""
+    lrs = [FakeLr(dense_region("P", (23, 23, 23), (0.45,) * 3))] * 3
+    seen = []
+
+    def timer(ctx, lrs_, pot, psi, prec, kw):
+        o = dict(ctx.opts)
+        seen.append(o)
+        # what an option that changes nothing can show: a lucky timing
+        return (lines if o["line_passes"] else 5.0) - 2.0 * o["persist"]
+    ctx = FakeCtx()
+    _, opts, _ = autotune.tune(ctx, lrs, None, None, bigdft_hip.PREC_FP64,
+                               cache=autotune.TuneCache(str(tmp_path / "t.json")), timer=timer)
+    assert all(o["line_passes"] for o in seen if o["persist"])
+    assert any(o["persist"] for o in seen) == tried
+    assert opts["persist"] == int(tried) and opts["line_passes"] == int(tried)
