@@ -1261,7 +1261,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   for (int p = 0; p < P_COUNT; ++p) T.t[p].xcd = 1;
   {
     const int po = ctx->opt_order == 1 ? 1 : 0;
-    T.t[P_PF].xcd = T.t[P_PB].xcd = T.t[P_UNC].xcd = po;
+    T.t[P_PF].xcd = T.t[P_PB].xcd = T.t[P_RP].xcd = T.t[P_UNC].xcd = po;
     T.pf2.xcd = T.pb2.xcd = po;
     for (int k = 0; k < 4; ++k) T.vbg[k].xcd = T.pfg[k].xcd = T.pbg[k].xcd = po;
     for (int k = 0; k < 4; ++k) T.zg[k].xcd = 1;

@@ -514,3 +514,35 @@ def test_chunks_keep_to_their_size(ctx, geo, n, norb, mb):
     for a, b in zip(one, cut):
         assert torch.equal(a, b)
     lr.close()
+
+
+@pytest.mark.parametrize("ns", [[(23, 22, 24)], [(9, 8, 20), (27, 30, 24), (38, 41, 27)]],
+                         ids=["one_group", "several"])
+def test_potential_planes_in_either_order(ctx, ns):
+    """more than 512 planes, in one launch and in one per box shape: both tile
+    orders give the same bits"""
+    regs = [dense_region("P", n, (0.4, 0.4, 0.4)) for n in ns] * 12
+    psi = [random_psi(r, 1, 181 + i)[0] for i, r in enumerate(regs[:len(ns)])] * 12
+    pots = [random_pot(r, 185 + i) for i, r in enumerate(regs[:len(ns)])]
+    lr = [ctx.region(r) for r in regs[:len(ns)]]
+    lrs = lr * 12
+    po = np.tile(np.cumsum([0] + [p.size for p in pots[:-1]]), 12)
+    so = np.cumsum([0] + [p.size for p in psi])[:-1]
+    x, v = dev(np.concatenate(psi)), dev(np.concatenate(pots))
+    outs = []
+    for order in (0, 1):
+        print(f"case {ns} order {order}", flush=True)
+        ctx.set_option("tile_order", order)
+        try:
+            h = torch.zeros_like(x)
+            ek = torch.zeros(len(lrs), dtype=torch.float64, device="cuda")
+            ep = torch.zeros_like(ek)
+            ctx.locham_batch(lrs, v, x, h, ek, ep, pot_off=po, psi_off=so)
+            ctx.sync()
+        finally:
+            ctx.set_option("tile_order", 0)
+        outs.append((h, ek, ep))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+    for l in lr:
+        l.close()
