@@ -950,8 +950,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
     size_t vb_max = 0;
     for (int i = 0; i < norb; ++i) {
       const BoxDesc& b = box[i];
-      vb_max = std::max(vb_max, plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1],
-                                              (int)sizeof(float)));
+      vb_max = std::max(vb_max, plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1]));
     }
     valu_bwd_ok = valu_bwd_ok && vb_max <= ctx->plane_lds;
     mfma_bwd_ok = ml.bwd <= ctx->plane_lds;
@@ -1018,7 +1017,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
       const BoxDesc& b = box[i];
       const size_t f = mfma_lds_fwd(2 * b.N[0], 2 * b.N[1], b.L[0], b.mfp);
       const size_t w = mfma_lds_bwd(2 * b.N[0], b.L[0], b.L[1]);
-      const size_t v = plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1], (int)sizeof(float));
+      const size_t v = plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1]);
       if ((bv ? f : std::max(f, w)) <= half) {
         sm.push_back(i);
         fs = std::max(fs, f);
@@ -1057,7 +1056,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
       size_t gl[4] = {0, 0, 0, 0};
       for (int i = 0; i < norb; ++i) {
         const BoxDesc& b = box[i];
-        const size_t v = plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1], (int)sizeof(float));
+        const size_t v = plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1]);
         const size_t fit = ctx->plane_lds / std::max(v, (size_t)1);
         const int c = (int)std::min((size_t)4, std::max((size_t)1, fit));
         grp[c - 1].push_back(i);
@@ -1089,7 +1088,7 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
   {
     // density plans (grow_plane) use the first half of the sequence (FP32:
     // the forward plane kernel without its kinetic part); the
-    // preconditioner's plans keep the line passes
+    // preconditioner's plans have a rule of their own (pc_plane, below)
     bool plane = !ctx->force_lines && !mfma && (!density || grow_plane);
     const bool d64 = esz == 8;   // the FP64 sequence (bdft_fp64.hip)
     size_t lpf = 0, lpb = 0;
@@ -1104,8 +1103,8 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
         pl = pl && fp64_pot_lines_ok(b, ctx->plane_lds);
         fits = fits && b.zcol;
       } else {
-        lpf = std::max(lpf, plane_lds_fwd(b.N[0], b.N[1], b.L[0], (int)esz));
-        lpb = std::max(lpb, plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1], (int)esz));
+        lpf = std::max(lpf, plane_lds_fwd(b.N[0], b.N[1], b.L[0]));
+        lpb = std::max(lpb, plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1]));
       }
     }
     if (d64) fits = fits && (density ? pp : (kp || kl) && (pp || pl));
@@ -1236,12 +1235,12 @@ static int make_plan(bdft_ctx* ctx, int norb, const bdft_lr* const* lrs,
       };
       group(P_PF,
             [&](const BoxDesc& b) {
-              return fit(plane_lds_fwd(b.N[0], b.N[1], b.L[0], (int)esz));
+              return fit(plane_lds_fwd(b.N[0], b.N[1], b.L[0]));
             },
             T.pfg, T.nt_pfg, T.lds_pfg, T.shape_pfg, T.nthr_pfg, T.n_pfg, pf_off);
       group(P_PB,
             [&](const BoxDesc& b) {
-              return fit(plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1], (int)esz));
+              return fit(plane_lds_bwd(b.N[0], b.N[1], b.L[0], b.L[1]));
             },
             T.pbg, T.nt_pbg, T.lds_pbg, T.shape_pbg, T.nthr_pbg, T.n_pbg, pb_off);
     }

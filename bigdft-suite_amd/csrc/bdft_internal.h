@@ -652,15 +652,13 @@ hipError_t launch_fp64_density(const Batch& B, const PassTables& PT, const DenAr
                                hipStream_t s);
 hipError_t launch_fp64_seq(const Batch& B, const PassTables& PT, hipStream_t s,
                            hipEvent_t* ev);
-size_t plane_lds_fwd(int N1, int N2, int L1, int elem);
-size_t plane_lds_bwd(int N1, int N2, int L1, int L2, int elem);
+size_t plane_lds_fwd(int N1, int N2, int L1);
+size_t plane_lds_bwd(int N1, int N2, int L1, int L2);
 size_t plane_attributes();
-template <typename T>
 hipError_t launch_plane_fwd(const Batch& B, const TileTable& t, const TileTable& ft,
                             int ntiles, size_t lds, double* part, hipStream_t s);
 hipError_t launch_plane_grow(const Batch& B, const TileTable& t, int ntiles, size_t lds,
                              hipStream_t s);
-template <typename T>
 hipError_t launch_plane_bwd(const Batch& B, const TileTable& t, int ntiles, size_t lds,
                             hipStream_t s);
 hipError_t launch_transfer(const Batch& B, const TileTable& t, int ntiles,

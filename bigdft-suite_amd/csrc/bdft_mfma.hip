@@ -1484,7 +1484,7 @@ static hipError_t launch_mfma_t(const Batch& B, const PassTables& PT, const Mfma
       hipError_t e = hipSuccess;
       for (int k = 0; k < PT.n_vbg && e == hipSuccess; ++k)
         if (PT.nt_vbg[k] > 0)
-          e = launch_plane_bwd<float>(B, PT.vbg[k], PT.nt_vbg[k], L.lds_vbg[k], s);
+          e = launch_plane_bwd(B, PT.vbg[k], PT.nt_vbg[k], L.lds_vbg[k], s);
       if (e != hipSuccess) return e;
     } else {
       if (PT.ntiles[P_PB] > 0)

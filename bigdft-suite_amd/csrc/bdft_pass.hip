@@ -1312,10 +1312,10 @@ static hipError_t launch_seq(const Batch& B, const PassTables& PT, int maxN,
     if (PT.n_pfg > 0) {
       for (int k = 0; k < PT.n_pfg; ++k)
         if (PT.nt_pfg[k] > 0)
-          launch_plane_fwd<T>(B, PT.pfg[k], PT.t[P_PF], PT.nt_pfg[k], PT.lds_pfg[k],
+          launch_plane_fwd(B, PT.pfg[k], PT.t[P_PF], PT.nt_pfg[k], PT.lds_pfg[k],
                               PT.part[0], s);
     } else if (PT.ntiles[P_PF] > 0) {
-      launch_plane_fwd<T>(B, PT.t[P_PF], PT.t[P_PF], PT.ntiles[P_PF], PT.lds_pf, PT.part[0],
+      launch_plane_fwd(B, PT.t[P_PF], PT.t[P_PF], PT.ntiles[P_PF], PT.lds_pf, PT.part[0],
                           s);
     }
     mark(S_PF, 1);
@@ -1327,9 +1327,9 @@ static hipError_t launch_seq(const Batch& B, const PassTables& PT, int maxN,
     if (PT.n_pbg > 0) {
       for (int k = 0; k < PT.n_pbg; ++k)
         if (PT.nt_pbg[k] > 0)
-          launch_plane_bwd<T>(B, PT.pbg[k], PT.nt_pbg[k], PT.lds_pbg[k], s);
+          launch_plane_bwd(B, PT.pbg[k], PT.nt_pbg[k], PT.lds_pbg[k], s);
     } else if (PT.ntiles[P_PB] > 0) {
-      launch_plane_bwd<T>(B, PT.t[P_PB], PT.ntiles[P_PB], PT.lds_pb, s);
+      launch_plane_bwd(B, PT.t[P_PB], PT.ntiles[P_PB], PT.lds_pb, s);
     }
     mark(S_PB, 1);
     et.t[0] = PT.t[P_PF];

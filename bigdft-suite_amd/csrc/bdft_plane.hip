@@ -1,5 +1,6 @@
-// Plane-fused kernels: one work-group holds a whole x-y plane of one box in
-// LDS and applies both in-plane axes there.
+// Plane-fused kernels of the FP32 sequence (and of the matrix-core ones'
+// backward pass on the vector units): one work-group holds a whole x-y plane of
+// one box in LDS and applies both in-plane axes there.
 //
 //   k_plane_fwd  plane j3 of W (wavelet x,y at wavelet z index j3):
 //                K  = K_x W + K_y W              (kinetic, + ekin partial)
@@ -20,32 +21,26 @@
 
 namespace bdft {
 
-// threads per plane work-group: a large FP64 plane fills most of a CU's
-// LDS, so one work-group runs per CU and it takes 12 waves (smaller boxes'
-// forward planes, launched in their own group, two per CU); FP32 planes run
-// two to four work-groups of 8 waves per CU
-template <typename T>
-struct PlaneNT {
-  static constexpr int v = sizeof(T) == 8 ? 768 : 512;
-};
+// threads per plane work-group: two to four work-groups of 8 waves run per CU
+constexpr int NTP = 512;
 
 // A contiguous n1 x n2 plane (x fastest) from memory into LDS rows of
 // stride rs > n1: element i = tid + k NTP of the plane, its row carried from
 // step to step (no division per element), UR loads in flight per thread.
 // TRANS: stored transposed, x = j of row ch at j rs + ch (rs >= n2, odd).
-template <typename T, int NTP, bool TRANS = false>
-__device__ __forceinline__ void plane_load(T* dst, int rs, const T* __restrict__ src, int n1,
-                                           int n2) {
+template <bool TRANS = false>
+__device__ __forceinline__ void plane_load(float* dst, int rs, const float* __restrict__ src,
+                                           int n1, int n2) {
   constexpr int UR = 8;
   const int tot = n1 * n2;
   ItDiv d(threadIdx.x, n1, NTP);
   for (int base = threadIdx.x; base < tot; base += NTP * UR) {
-    T v[UR];
+    float v[UR];
     int a[UR];
 #pragma unroll
     for (int u = 0; u < UR; ++u) {
       const int i = base + u * NTP;
-      v[u] = i < tot ? src[i] : (T)0;
+      v[u] = i < tot ? src[i] : 0.0f;
       // row r, column i - r n1 at r rs + i - r n1 (transposed: (i - r n1) rs + r)
       a[u] = TRANS ? d.j * rs + d.ch : i + d.ch * (rs - n1);
       d.next(n1);
@@ -57,9 +52,8 @@ __device__ __forceinline__ void plane_load(T* dst, int rs, const T* __restrict__
 }
 
 // the reverse: LDS rows of stride rs into a contiguous n1 x n2 plane
-template <typename T, int NTP>
-__device__ __forceinline__ void plane_store(T* __restrict__ dst, const T* src, int rs, int n1,
-                                            int n2) {
+__device__ __forceinline__ void plane_store(float* __restrict__ dst, const float* src, int rs,
+                                            int n1, int n2) {
   const int tot = n1 * n2;
   ItDiv d(threadIdx.x, n1, NTP);
   for (int i = threadIdx.x; i < tot; i += NTP) {
@@ -68,7 +62,6 @@ __device__ __forceinline__ void plane_store(T* __restrict__ dst, const T* src, i
   }
 }
 
-template <int NW>
 __device__ __forceinline__ double block_sum_p(double v, double* red) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -78,26 +71,26 @@ __device__ __forceinline__ double block_sum_p(double v, double* red) {
   __syncthreads();
   double s = 0.0;
   if (threadIdx.x == 0)
-    for (int i = 0; i < NW; ++i) s += red[i];
+    for (int i = 0; i < NTP / 64; ++i) s += red[i];
   return s;
 }
 
-// LDS layout of the forward and preconditioner plane kernels: the W plane A
+// LDS layout of the forward plane kernel: the W plane A
 // (W2 rows of stride RA = W1 + 1, then a zero row; column W1 of every row is
 // zero: the free lines' zero slots), the second plane C (W2 + 1 rows of
 // stride RC), then the line maps (x on the rows of A, y on the columns of A,
 // y on the columns of C).  Byte offset of the maps:
-__host__ __device__ inline size_t plane_maps_off(int N1, int N2, int RC, int elem) {
+__host__ __device__ inline size_t plane_maps_off(int N1, int N2, int RC) {
   const size_t rows = 2 * N2 + 1, RA = 2 * N1 + 1;
-  return ((rows * RA + rows * RC) * elem + 7) & ~(size_t)7;
+  return ((rows * RA + rows * RC) * sizeof(float) + 7) & ~(size_t)7;
 }
 
 // zero slots: column W1 and row W2 of A, row W2 of C (stride RC)
-template <typename T, int NTP>
-__device__ __forceinline__ void plane_zero_slots(T* A, int RA, int W1, int W2, T* C, int RC) {
-  for (int i = threadIdx.x; i < W2; i += NTP) A[i * RA + W1] = (T)0;
-  for (int i = threadIdx.x; i < RA; i += NTP) A[W2 * RA + i] = (T)0;
-  for (int i = threadIdx.x; i < RC; i += NTP) C[W2 * RC + i] = (T)0;
+__device__ __forceinline__ void plane_zero_slots(float* A, int RA, int W1, int W2, float* C,
+                                                 int RC) {
+  for (int i = threadIdx.x; i < W2; i += NTP) A[i * RA + W1] = 0.0f;
+  for (int i = threadIdx.x; i < RA; i += NTP) A[W2 * RA + i] = 0.0f;
+  for (int i = threadIdx.x; i < RC; i += NTP) C[W2 * RC + i] = 0.0f;
 }
 
 // ---------------------------------------------------------------------------
@@ -106,10 +99,9 @@ __device__ __forceinline__ void plane_zero_slots(T* A, int RA, int W1, int W2, T
 // launch's tiles (all boxes, or one group of them); ft: the table over all
 // boxes whose tile numbers index the kinetic partials
 // ---------------------------------------------------------------------------
-template <typename T, bool KIN = true>
-__global__ __launch_bounds__(PlaneNT<T>::v) void k_plane_fwd(Batch B, TileTable tt,
-                                                             TileTable ft, double* part) {
-  constexpr int NTP = PlaneNT<T>::v;
+template <bool KIN = true>
+__global__ __launch_bounds__(NTP) void k_plane_fwd(Batch B, TileTable tt, TileTable ft,
+                                                   double* part) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double red[NTP / 64];
   const int tile = tile_of(tt);
@@ -122,29 +114,29 @@ __global__ __launch_bounds__(PlaneNT<T>::v) void k_plane_fwd(Batch B, TileTable 
   const int RA = W1 + 1;            // row stride of the wavelet plane
   const int RB = odd_stride(L1);    // row stride of the G_x output
   const int RC = max(RA, RB);
-  T* A = (T*)smem;                  // W plane: A[j2*RA + j1]
-  T* C = A + (W2 + 1) * RA;         // kinetic accumulator, later G_x output
-  int2* mx = (int2*)(smem + plane_maps_off(N1, N2, RC, sizeof(T)));
+  float* A = (float*)smem;              // W plane: A[j2*RA + j1]
+  float* C = A + (W2 + 1) * RA;         // kinetic accumulator, later G_x output
+  int2* mx = (int2*)(smem + plane_maps_off(N1, N2, RC));
   int2* mya = mx + map_len(N1);
   int2* myc = mya + map_len(N2);
-  const T* src = (const T*)B.W + bd.w_off + (long long)W1 * W2 * j3;
+  const float* src = (const float*)B.W + bd.w_off + (long long)W1 * W2 * j3;
   const int tid = threadIdx.x;
   // load the plane (contiguous), UNR loads in flight per thread
-  plane_load<T, NTP>(A, RA, src, W1, W2);
-  build_map(mx, N1, per, sizeof(T), W1, tid, NTP);
-  build_map(mya, N2, per, RA * sizeof(T), W2, tid, NTP);
-  build_map(myc, N2, per, RB * sizeof(T), W2, tid, NTP);
-  plane_zero_slots<T, NTP>(A, RA, W1, W2, C, RB);
+  plane_load(A, RA, src, W1, W2);
+  build_map(mx, N1, per, sizeof(float), W1, tid, NTP);
+  build_map(mya, N2, per, RA * sizeof(float), W2, tid, NTP);
+  build_map(myc, N2, per, RB * sizeof(float), W2, tid, NTP);
+  plane_zero_slots(A, RA, W1, W2, C, RB);
   __syncthreads();
   if constexpr (KIN) {
   // K_x: rows j2, chunks of 4 coarse x positions -> C
-  const T kx = (T)bd.kscale[0], ky = (T)bd.kscale[1];
+  const float kx = (float)bd.kscale[0], ky = (float)bd.kscale[1];
   const int cx = (N1 + 3) >> 2;
   for (ItDiv d(tid, W2, NTP); d.ch < cx; d.next(W2)) {
     const int ch = d.ch, j2 = d.j;
     const int i0 = 4 * ch;
-    T oc[4], od[4];
-    kin4_any(PLine<T>{A + j2 * RA, 1}, mx, N1, i0, oc, od);
+    float oc[4], od[4];
+    kin4_any(PLine<float>{A + j2 * RA, 1}, mx, N1, i0, oc, od);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       if (i0 + r < N1) {
@@ -159,25 +151,25 @@ __global__ __launch_bounds__(PlaneNT<T>::v) void k_plane_fwd(Batch B, TileTable 
   for (ItDiv d(tid, W1, NTP); d.ch < cy; d.next(W1)) {
     const int ch = d.ch, j1 = d.j;
     const int i0 = 4 * ch;
-    T oc[4], od[4];
-    kin4_any(PLine<T>{A + j1, RA}, mya, N2, i0, oc, od);
+    float oc[4], od[4];
+    kin4_any(PLine<float>{A + j1, RA}, mya, N2, i0, oc, od);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       if (i0 + r < N2) {
         const int a = (i0 + r) * RA + j1, d = (N2 + i0 + r) * RA + j1;
-        const T vc = C[a] + oc[r] * ky, vd = C[d] + od[r] * ky;
+        const float vc = C[a] + oc[r] * ky, vd = C[d] + od[r] * ky;
         C[a] = vc;
         C[d] = vd;
         ek += (double)vc * (double)A[a] + (double)vd * (double)A[d];
       }
   }
-  const double eks = block_sum_p<NTP / 64>(ek, red);
+  const double eks = block_sum_p(ek, red);
   if (tid == 0) part[box_first_tile(ft, b) + j3] = eks;
   __syncthreads();
   // K plane -> memory (contiguous)
   {
-    T* kd = (T*)B.K + bd.w_off + (long long)W1 * W2 * j3;
-    plane_store<T, NTP>(kd, C, RA, W1, W2);
+    float* kd = (float*)B.K + bd.w_off + (long long)W1 * W2 * j3;
+    plane_store(kd, C, RA, W1, W2);
   }
   __syncthreads();
   }
@@ -186,21 +178,21 @@ __global__ __launch_bounds__(PlaneNT<T>::v) void k_plane_fwd(Batch B, TileTable 
   for (ItDiv d(tid, W2, NTP); d.ch < gx; d.next(W2)) {
     const int ch = d.ch, j2 = d.j;
     const int p0 = 8 * ch;
-    T o[8];
-    grow8_any(PLine<T>{A + j2 * RA, 1}, mx, N1, grow_k0(p0, per), o);
+    float o[8];
+    grow8_any(PLine<float>{A + j2 * RA, 1}, mx, N1, grow_k0(p0, per), o);
 #pragma unroll
     for (int r = 0; r < 8; ++r)
       if (p0 + r < L1) C[j2 * RB + p0 + r] = o[r];
   }
   __syncthreads();
   // G_y: columns p1 of C -> T2 plane (real x,y at wavelet z j3)
-  T* dst = (T*)B.T2 + bd.t2_off + (long long)L1 * L2 * j3;
+  float* dst = (float*)B.T2 + bd.t2_off + (long long)L1 * L2 * j3;
   const int gy = (L2 + 7) >> 3;
   for (ItDiv d(tid, L1, NTP); d.ch < gy; d.next(L1)) {
     const int ch = d.ch, p1 = d.j;
     const int p0 = 8 * ch;
-    T o[8];
-    grow8_any(PLine<T>{C + p1, RB}, myc, N2, grow_k0(p0, per), o);
+    float o[8];
+    grow8_any(PLine<float>{C + p1, RB}, myc, N2, grow_k0(p0, per), o);
 #pragma unroll
     for (int r = 0; r < 8; ++r)
       if (p0 + r < L2) dst[p1 + (long long)L1 * (p0 + r)] = o[r];
@@ -210,9 +202,7 @@ __global__ __launch_bounds__(PlaneNT<T>::v) void k_plane_fwd(Batch B, TileTable 
 // ---------------------------------------------------------------------------
 // backward plane kernel with compress-accumulate
 // ---------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(PlaneNT<T>::v) void k_plane_bwd(Batch B, TileTable tt) {
-  constexpr int NTP = PlaneNT<T>::v;
+__global__ __launch_bounds__(NTP) void k_plane_bwd(Batch B, TileTable tt) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int tile = tile_of(tt);
   const int lb = find_box(tt, tile);   // tables over a subset carry a box map
@@ -227,38 +217,37 @@ __global__ __launch_bounds__(PlaneNT<T>::v) void k_plane_bwd(Batch B, TileTable 
   const int RU = L2 | 1;            // T2 plane, transposed: y lines as rows
   const int RQ = L1 | 1;            // G_y^T output rows (read by rows)
   const int RO = W1 + 1;
-  T* U = (T*)smem;                // T2 plane: U[p1*RU + p2], later output O
-  T* Bq = U + max(L1 * RU, W2 * RO);  // G_y^T output: Bq[j2*RQ + p1]
+  float* U = (float*)smem;            // T2 plane: U[p1*RU + p2], later output O
+  float* Bq = U + max(L1 * RU, W2 * RO);  // G_y^T output: Bq[j2*RQ + p1]
   int* fmx = (int*)(Bq + W2 * RQ);     // periodic fine-line maps (x: rows of Bq,
   int* fmy = fmx + fmap_len(N1);       // y: rows of U)
   const int tid = threadIdx.x;
-  const T* src = (const T*)B.T2 + bd.t2_off + (long long)L1 * L2 * j3;
+  const float* src = (const float*)B.T2 + bd.t2_off + (long long)L1 * L2 * j3;
   // the compress's first point per thread (indices, K, old hpsi) is loaded
   // before the plane, so that its latency overlaps the plane load and the
   // two passes (one point: more registers held through the passes cost
   // occupancy); later steps take UC points each
-  constexpr int UC = NTP >= 768 ? 3 : 2, UP = 1;
-  const T* Kp = (const T*)B.K + bd.w_off + (long long)W1 * W2 * j3;
-  CompressStep<T, UP> st0;
+  constexpr int UC = 2, UP = 1;
+  const float* Kp = (const float*)B.K + bd.w_off + (long long)W1 * W2 * j3;
+  CompressStep<float, UP> st0;
   compress_load<UP, NTP>(bd, j3, Kp, B.hpsi, tid, st0);
-  plane_load<T, NTP, true>(U, RU, src, L1, L2);
+  plane_load<true>(U, RU, src, L1, L2);
   if (per) {
-    build_fmap(fmx, N1, L1, sizeof(T), tid, NTP);
-    build_fmap(fmy, N2, L2, sizeof(T), tid, NTP);
+    build_fmap(fmx, N1, L1, sizeof(float), tid, NTP);
+    build_fmap(fmy, N2, L2, sizeof(float), tid, NTP);
   }
   __syncthreads();
   // G_y^T: y lines p1 (rows of U) -> Bq rows (c: i2, d: N2+i2), NOY coarse outputs
-  // per work item (NOX for G_x^T): two in FP32, so that the last round of
-  // items leaves fewer lanes idle between the barriers (C4 FP32 backward
-  // pass 3.41 -> 3.22 ms); four in FP64 (two was slower on the periodic
-  // 48^3 planes, 2.27 -> 2.47 ms)
-  constexpr int NOY = sizeof(T) == 4 ? 2 : 4, NOX = NOY;
+  // per work item (NOX for G_x^T): two, so that the last round of items leaves
+  // fewer lanes idle between the barriers than with four (1024 spheres, 3.41 ->
+  // 3.22 ms)
+  constexpr int NOY = 2, NOX = NOY;
   const int cy = (N2 + NOY - 1) / NOY;
   for (ItDiv d(tid, L1, NTP); d.ch < cy; d.next(L1)) {
     const int ch = d.ch, p1 = d.j;
     const int i0 = NOY * ch;
-    T oc[NOY], od[NOY];
-    shrink4_any<T, NOY>(U + p1 * RU, fmy, L2, i0, per, oc, od);
+    float oc[NOY], od[NOY];
+    shrink4_any<float, NOY>(U + p1 * RU, fmy, L2, i0, per, oc, od);
 #pragma unroll
     for (int r = 0; r < NOY; ++r)
       if (i0 + r < N2) {
@@ -268,13 +257,13 @@ __global__ __launch_bounds__(PlaneNT<T>::v) void k_plane_bwd(Batch B, TileTable 
   }
   __syncthreads();
   // G_x^T: rows j2 of Bq -> output plane O (reuses U), row stride RO
-  T* O = U;
+  float* O = U;
   const int cx = (N1 + NOX - 1) / NOX;
   for (ItDiv d(tid, W2, NTP); d.ch < cx; d.next(W2)) {
     const int ch = d.ch, j2 = d.j;
     const int i0 = NOX * ch;
-    T oc[NOX], od[NOX];
-    shrink4_any<T, NOX>(Bq + j2 * RQ, fmx, L1, i0, per, oc, od);
+    float oc[NOX], od[NOX];
+    shrink4_any<float, NOX>(Bq + j2 * RQ, fmx, L1, i0, per, oc, od);
 #pragma unroll
     for (int r = 0; r < NOX; ++r)
       if (i0 + r < N1) {
@@ -286,30 +275,31 @@ __global__ __launch_bounds__(PlaneNT<T>::v) void k_plane_bwd(Batch B, TileTable 
   // out = O + K, accumulated into hpsi at the compressed positions of the
   // plane's four components (s3 fixed by j3), compress_and_accumulate_mixed
   // (un-compress.f90:2174-2238)
-  compress_store<T, UP, NTP>(bd, j3, O, RO, B.hpsi, tid, st0);
+  compress_store<float, UP, NTP>(bd, j3, O, RO, B.hpsi, tid, st0);
   for (int i0 = tid + NTP * UP; i0 < N1 * N2; i0 += NTP * UC) {
-    CompressStep<T, UC> st;
+    CompressStep<float, UC> st;
     compress_load<UC, NTP>(bd, j3, Kp, B.hpsi, i0, st);
-    compress_store<T, UC, NTP>(bd, j3, O, RO, B.hpsi, i0, st);
+    compress_store<float, UC, NTP>(bd, j3, O, RO, B.hpsi, i0, st);
   }
 }
 
 // LDS bytes of the two plane kernels for the largest box extents
-size_t plane_lds_fwd(int N1, int N2, int L1, int elem) {
+size_t plane_lds_fwd(int N1, int N2, int L1) {
   const int RA = 2 * N1 + 1, RB = odd_stride(L1);
-  return plane_maps_off(N1, N2, RA > RB ? RA : RB, elem) +
+  return plane_maps_off(N1, N2, RA > RB ? RA : RB) +
          8 * (size_t)(map_len(N1) + 2 * map_len(N2));
 }
-size_t plane_lds_bwd(int N1, int N2, int L1, int L2, int elem) {
+size_t plane_lds_bwd(int N1, int N2, int L1, int L2) {
   const size_t RU = L2 | 1, RQ = L1 | 1, RO = 2 * N1 + 1;
   const size_t u = (size_t)L1 * RU > 2 * N2 * RO ? (size_t)L1 * RU : 2 * N2 * RO;
   const bool per = L1 == 2 * N1;
-  return (u + 2 * N2 * RQ) * elem + (per ? 4 * (size_t)(fmap_len(N1) + fmap_len(N2)) : 0);
+  return (u + 2 * N2 * RQ) * sizeof(float) +
+         (per ? 4 * (size_t)(fmap_len(N1) + fmap_len(N2)) : 0);
 }
 
 static hipError_t plane_setup(int bytes) {
-  const void* k[] = {(const void*)k_plane_fwd<float>, (const void*)k_plane_fwd<float, false>,
-                     (const void*)k_plane_bwd<float>};
+  const void* k[] = {(const void*)k_plane_fwd<true>, (const void*)k_plane_fwd<false>,
+                     (const void*)k_plane_bwd};
   for (const void* f : k) {
     const hipError_t e =
         hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
@@ -333,26 +323,20 @@ size_t plane_attributes() {
   return (size_t)v;
 }
 
-template <typename T>
 hipError_t launch_plane_fwd(const Batch& B, const TileTable& t, const TileTable& ft,
                             int ntiles, size_t lds, double* part, hipStream_t s) {
-  k_plane_fwd<T><<<ntiles, PlaneNT<T>::v, lds, s>>>(B, t, ft, part);
+  k_plane_fwd<true><<<ntiles, NTP, lds, s>>>(B, t, ft, part);
   return hipGetLastError();
 }
 hipError_t launch_plane_grow(const Batch& B, const TileTable& t, int ntiles, size_t lds,
                              hipStream_t s) {
-  k_plane_fwd<float, false><<<ntiles, PlaneNT<float>::v, lds, s>>>(B, t, t, nullptr);
+  k_plane_fwd<false><<<ntiles, NTP, lds, s>>>(B, t, t, nullptr);
   return hipGetLastError();
 }
-template <typename T>
 hipError_t launch_plane_bwd(const Batch& B, const TileTable& t, int ntiles, size_t lds,
                             hipStream_t s) {
-  k_plane_bwd<T><<<ntiles, PlaneNT<T>::v, lds, s>>>(B, t);
+  k_plane_bwd<<<ntiles, NTP, lds, s>>>(B, t);
   return hipGetLastError();
 }
-template hipError_t launch_plane_fwd<float>(const Batch&, const TileTable&, const TileTable&,
-                                            int, size_t, double*, hipStream_t);
-template hipError_t launch_plane_bwd<float>(const Batch&, const TileTable&, int, size_t,
-                                            hipStream_t);
 
 }  // namespace bdft
