@@ -18,14 +18,15 @@
 //
 // Measured on 128 orbitals of a periodic 40^3 box (6.6e7 fine points), the
 // x-y-z order's kernels before: uncompress 183 us, forward planes 1085, z
-// kinetic 553, z potential 413, backward planes 689, an apply 2.65 ms; now
-// k_zgrow 0.24 ms (16 B per point: 4.4 TB/s, a large copy runs at 4.9),
-// k_xykin 0.47 and k_xypot 0.49 (three times the time of their FMAs at the
-// FP64 peak; a quarter of their vector instructions are addresses, the rest
-// waits at barriers and LDS loads), k_zback 0.60 (40 B per point: 4.4 TB/s),
-// an apply 1.71 ms.  48 orbitals of a 64^3 box, whose pairs of planes did not
-// fit in LDS (line passes): 4.61 -> 2.84 ms; 256 free boxes of 16 to 40 points
-// an axis 2.66 -> 2.03 ms.
+// kinetic 553, z potential 413, backward planes 689, an apply 2.65 ms; now,
+// each the fastest of five launches under the tracer, k_zgrow 0.24 ms (16 B per
+// point: 4.5 TB/s, a large copy runs at 4.9), k_xykin 0.46 and k_xypot 0.47
+// (three times the time of their FMAs at the FP64 peak; a quarter of their
+// vector instructions are addresses, the rest waits at barriers and LDS
+// loads), k_zback 0.57 (40 B per point: 4.6 TB/s); an apply without the tracer
+// 1.68 ms.  48 orbitals of a 64^3 box, whose pairs of planes did not fit in LDS
+// (line passes): 4.54 -> 2.80 ms; 256 free boxes of 16 to 40 points an axis
+// 2.66 -> 2.02 ms.
 //
 // Grid TZ of a box (tz_off): plane p3 = 0 .. L3 - 1, in it the wavelet plane
 // [j1 + 2 N1 j2]; K (w_off): the wavelet volume.
@@ -512,7 +513,7 @@ __global__ __launch_bounds__(PZ_NT, WPE) void k_pcz(Batch B, TileTable tt, PcArg
 // whose load, passes and store run one after the other).  Two chunks of a
 // line per item (half the LDS reads, half the coefficients) and coefficients
 // from scalar loads (half the scalar instructions) were both slower: 0.60 and
-// 0.65 ms against 0.59 for k_xypot on the batch above.
+// 0.65 ms for k_xypot on the batch above when it took 0.59.
 //
 // Line ends: a wave whose chunks all lie inside their lines reads them
 // directly.  Otherwise, periodic: through a line map in LDS (any N); free:

@@ -321,7 +321,9 @@ int bdft_ctx_info(const bdft_ctx *ctx, int64_t *lds_per_block,
 /* Launch options of the context.  No counterpart in the reference (its
  * OpenCL kernels have fixed work-group shapes); these are the choices the
  * autotuner (bigdft_hip/autotune.py) times per box shape and caches.
- *   BDFT_OPT_LINE_PASSES  0: plane-fused sequences where they fit (default),
+ *   BDFT_OPT_LINE_PASSES  0: plane-fused sequences where they fit (default;
+ *                            large FP64 batches of flat free boxes, up to three
+ *                            coarse points on z, may run the line passes),
  *                         1: line passes (FP64/FP32) and per-pass
  *                            matrix-core kernels for every batch
  *   BDFT_OPT_ZGROUP       matrix-core z-line bundles of 32 lines per
